@@ -1,0 +1,284 @@
+"""The work that programs have this engine do, as cases to be timed and compared.
+
+A case is one of eight kinds, each built from the workloads of
+``mcell_amd.workloads`` and run through ``DiffuseReactEngine``:
+
+* ``free``        volume molecules without reactions in a reflective cube, one
+                  instance or many, positions read at the end of the pass
+* ``member``      a whole small simulation, as one member of an ensemble or a
+                  parameter sweep: engine, A + B -> C, counts, end state, close
+* ``reversible``  E <-> A + B in a cube at its equilibrium (products,
+                  unimolecular lifetimes, ids that grow)
+* ``timesteps``   the same with species time steps other than one iteration
+* ``receptors``   ligands on a sphere with receptors, a third species crossing
+                  the sphere as a counted volume
+* ``surface``     the same with receptors that diffuse on the sphere in half
+                  time steps
+* ``sweep``       a batch of replicas over one mesh with a diffusion constant of
+                  their own, counts per replica and the log of reactions
+* ``crowded``     perturbed finely meshed spheres, every kind of reaction
+
+Apart from ``member`` a pass goes on from where the last one ended, as a
+running simulation does: step to the next count, take the counts, read what
+the pass is for.  Molecules come back in the engine's order, which is not
+fixed, so a program that follows them sorts them by (replica, id); their number
+changes with the reactions, so it keeps them in tables of a fixed size.
+"""
+import math
+
+import numpy as np
+
+from mcell_amd import workloads as W
+from mcell_amd.engine import DiffuseReactEngine
+
+COUNT_EVERY = 10  # iterations between counts, as in the workloads' barriers
+
+
+def listed():
+    return [
+        # the smallest: one free-diffusion instance, a few launches per iteration, positions at the end
+        dict(name="free_box_10k", kind="free", replicas=1, n=10000, precision="fp64", iterations=100),
+        # a batch of free-diffusion instances in the FP32 form: the light pass at its largest
+        dict(name="free_batch_2m", kind="free", replicas=256, n=2000000, precision="fp32", iterations=500),
+        # one seed of the 32-seed A + B -> C ensemble: thousands of molecules, every launch counts
+        dict(name="member_4k", kind="member", n_a=2000, n_b=2000, precision="fp64", iterations=1000),
+        # the A + B -> C benchmark box, its first 200 iterations, set-up and end state included
+        dict(name="member_100k", kind="member", n_a=50000, n_b=50000, precision="fp32", iterations=200),
+        # binding and unbinding at equilibrium, an odd size
+        dict(name="reversible_50k", kind="reversible", n=50001, precision="fp64", iterations=50),
+        # species with time steps of 1/2, 1 and 3 iterations
+        dict(name="timesteps_30k", kind="timesteps", n=30000, precision="fp64", iterations=20),
+        # the volume-surface case: 100,000 ligands, 20,000 receptors, 10,000 crossing molecules
+        dict(name="receptors_110k", kind="receptors", n_l=100000, n_r=20000, n_t=10000, precision="fp32",
+             iterations=50),
+        # the same with receptors that diffuse in half steps
+        dict(name="surface_110k", kind="surface", n_l=100000, n_r=20000, n_t=10000, precision="fp64", iterations=20),
+        # a sweep of small replicas in the FP64 form
+        dict(name="sweep_24_small", kind="sweep", replicas=24, n_max=20000, precision="fp64", iterations=10),
+        # the replica batch of the benchmark at a quarter of its replicas (about 1e7 molecules)
+        dict(name="sweep_64", kind="sweep", replicas=64, n_max=200000, precision="fp32", iterations=10),
+        # crowded geometry at the density and mesh of the benchmark, an eighth of its spheres
+        dict(name="crowded_1m", kind="crowded", spheres=8, n=1250000, n_s=25000, precision="fp32", iterations=10),
+    ]
+
+
+def draw(rng):
+    def log(lo, hi):
+        return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+    kind = rng.choice(["free", "member", "reversible", "timesteps", "receptors", "surface", "sweep", "crowded"])
+    c = dict(kind=kind, precision=rng.choice(["fp64", "fp32"]))
+    if kind == "free":
+        r = log(1, 256)
+        c.update(replicas=r, n=max(r, log(1000, 2000000)))
+        c.update(iterations=max(10, min(1000, int(2e8 / c["n"]))))
+    elif kind == "member":
+        c.update(n_a=log(500, 50000), n_b=log(500, 50000))
+        c.update(iterations=max(100, min(1000, int(1e7 / (c["n_a"] + c["n_b"])))) // 10 * 10)
+    elif kind in ("reversible", "timesteps"):
+        c.update(n=log(2000, 50000 if kind == "timesteps" else 200000), iterations=20)
+    elif kind in ("receptors", "surface"):
+        c.update(n_l=log(5000, 150000), n_r=log(1000, 20000), n_t=log(1000, 50000), iterations=20)
+    elif kind == "sweep":
+        c.update(replicas=log(2, 64), n_max=log(2000, 200000), iterations=10)
+    else:
+        c.update(spheres=rng.randint(1, 8), n=log(100000, 1250000), n_s=log(2000, 25000), iterations=10)
+    return c
+
+
+def workload(case, seed):
+    kind = case["kind"]
+    if kind == "free":
+        return W.free_diffusion_replicas(case["replicas"], case["n"] // case["replicas"], seed=seed)
+    if kind == "member":
+        return W.bimol_box(n_a=case["n_a"], n_b=case["n_b"], seed=seed, barrier_interval=COUNT_EVERY)
+    if kind in ("reversible", "timesteps"):
+        wl = W.decay_box(n_e=case["n"], seed=seed, rate=1e3, back_rate=1e8)
+        return wl if kind == "reversible" else W.with_time_steps(wl, [0.5, 1, 3])
+    if kind in ("receptors", "surface"):
+        wl = W.receptor_sphere(n_l=case["n_l"], n_r=case["n_r"], n_t=case["n_t"], seed=seed, down_fraction=0.0,
+                               counted=kind == "receptors")
+        if kind == "surface":
+            wl = W.with_time_steps(W.with_diffusing_surface(wl, {1: 1e-8, 2: 1e-8}), [1, 0.5, 0.5, 1])
+        wl.barrier_interval = COUNT_EVERY
+        return wl
+    if kind == "sweep":
+        return W.replicas_sphere_in_cube(num_replicas=case["replicas"], seed=seed, n_max=case["n_max"])
+    return W.crowded_spheres(n_molecules=case["n"], n_surface=case["n_s"], seed=seed, num_spheres=case["spheres"],
+                             cube_um=2.0)
+
+
+class State:
+    """A running simulation: its workload, engine and next iteration."""
+
+    def __init__(self, case, seed):
+        self.case = case
+        self.wl = workload(case, seed)
+        self.it = 0
+        self.engine = None
+        # reactions of one stretch: far below these shares of the molecules
+        self.log_rows = {"sweep": lambda: case["replicas"] * case["n_max"] // 20 + 1000,
+                         "crowded": lambda: case["n"] // 2}.get(case["kind"], lambda: 0)()
+        if case["kind"] != "member":
+            self.engine = self.create()
+
+    def create(self):
+        return DiffuseReactEngine.from_workload(self.wl, precision=self.case["precision"],
+                                                log_capacity=self.log_rows)
+
+
+def prepare(case, seed):
+    return State(case, seed)
+
+
+def molecules(s, engine):
+    m = engine.molecules()
+    order = np.argsort(m["replica"].astype(np.uint64) << np.uint64(32) | m["id"])
+    out = {}
+    for k, v in m.items():
+        out[k] = np.zeros((2 * s.wl.num_molecules,) + v.shape[1:], v.dtype)
+        np.take(v, order, axis=0, out=out[k][:len(v)])
+    return out
+
+
+def events(s, engine):
+    log, out = engine.rxn_log(), {}
+    for k in log.dtype.names:
+        out[k] = np.zeros((s.log_rows,) + log[k].shape[1:], log[k].dtype)
+        out[k][:len(log)] = log[k][:s.log_rows]
+    return out
+
+
+def counted_steps(s, engine, first):
+    """The pass's iterations with the species counts of every stretch."""
+    wl, end, counts = s.wl, first + s.case["iterations"], []
+    for it in range(first, end, COUNT_EVERY):
+        engine.step(it, min(COUNT_EVERY, end - it))
+        counts.append(engine.count_species(wl.num_replicas, len(wl.species_steps)))
+        if wl.counted_volumes is not None:
+            counts.append(engine.count_species_by_volume(wl.num_replicas, wl.counted_volumes["num"],
+                                                         len(wl.species_steps)).reshape(-1))
+    return np.concatenate([c.reshape(-1) for c in counts])
+
+
+def run(s):
+    kind, n = s.case["kind"], s.case["iterations"]
+    if kind == "member":
+        engine = s.create()
+        out = {"counts": counted_steps(s, engine, 0), "reactions": engine.rxn_counts(),
+               "molecules": molecules(s, engine)}
+        engine.close()
+        return out
+    first, s.it = s.it, s.it + n
+    if kind == "free":
+        s.engine.step(first, n)
+        return {"molecules": s.engine.molecules()}  # nothing reacts: the order stays
+    out = {"counts": counted_steps(s, s.engine, first), "reactions": s.engine.rxn_counts()}
+    if kind in ("sweep", "crowded"):
+        out["log"] = events(s, s.engine)
+    else:
+        out["molecules"] = molecules(s, s.engine)
+    if kind in ("receptors", "surface"):
+        out["surface"] = s.engine.surface_molecules()
+    return out
+
+
+def work(case):
+    """Every molecule's position, id and tag read and written once per
+    iteration (64 bytes in FP64, 40 in FP32), three Gaussians, the move and
+    one wall test."""
+    n = {"free": lambda: case["n"], "member": lambda: case["n_a"] + case["n_b"],
+         "reversible": lambda: case["n"], "timesteps": lambda: case["n"],
+         "receptors": lambda: case["n_l"] + case["n_t"] + case["n_r"],
+         "surface": lambda: case["n_l"] + case["n_t"] + case["n_r"],
+         "sweep": lambda: case["replicas"] * (1000 + case["n_max"]) // 2 * 3 // 2,
+         "crowded": lambda: case["n"]}[case["kind"]]()
+    steps = n * case["iterations"]
+    return {"bytes": steps * (64 if case["precision"] == "fp64" else 40), "flops": steps * 60}
+
+
+# ------------------------------------------------------------- exact values --
+def ziggurat_tables():
+    """The 128-strip Ziggurat of Marsaglia and Tsang (2000) for the normal
+    density (r = 3.44428647676, an exponential tail above it): densities y,
+    32-bit widths w, bounds k."""
+    r = 3.44428647676
+    v = math.exp(-0.5 * r * r) * (r + 1 / r)
+    x = np.zeros(129)
+    x[128], x[127] = v / math.exp(-0.5 * r * r), r
+    for i in range(126, 0, -1):
+        x[i] = math.sqrt(-2 * math.log(v / x[i + 1] + math.exp(-0.5 * x[i + 1] ** 2)))
+    edge = np.concatenate([[x[128]], x[1:128]])   # outer edge per strip, the base strip first
+    inner = np.concatenate([[x[127]], x[0:127]])  # inner edge
+    y = np.exp(-0.5 * np.concatenate([[0.0], x[1:128]]) ** 2)
+    w = edge / 2 ** 32
+    k = np.floor(inner / edge * 2 ** 24).astype(np.uint64) << np.uint64(8)
+    return y, w, k
+
+
+def philox(seed, block, ids, iteration, replica):
+    """Philox4x32-10 (Salmon et al., SC'11): four uint32 per molecule."""
+    m32 = np.uint64(0xFFFFFFFF)
+    x0, x1 = np.broadcast_to(np.uint64(block), ids.shape), ids.astype(np.uint64)
+    x2, x3 = np.full(ids.shape, iteration, np.uint64), replica.astype(np.uint64) << np.uint64(8)
+    ka, kb = seed & 0xFFFFFFFF, seed >> 32
+    for _ in range(10):
+        p0, p1 = np.uint64(0xD2511F53) * x0, np.uint64(0xCD9E8D57) * x2
+        x0, x1, x2, x3 = ((p1 >> np.uint64(32)) ^ x1 ^ np.uint64(ka), p1 & m32,
+                          (p0 >> np.uint64(32)) ^ x3 ^ np.uint64(kb), p0 & m32)
+        ka, kb = (ka + 0x9E3779B9) & 0xFFFFFFFF, (kb + 0xBB67AE85) & 0xFFFFFFFF
+    return np.stack([x0, x1, x2, x3], axis=1)
+
+
+def gaussians(seed, ids, iteration, replica, tables):
+    """Three normals per molecule from its own stream, one uint32 each unless
+    the draw falls outside its strip."""
+    y, w, k = tables
+    b = philox(seed, 0, ids, iteration, replica)[:, :3]
+    strip = (b & np.uint64(0x7F)).astype(np.int64)
+    pos = b & np.uint64(0xFFFFFF00)
+    g = np.where(b & np.uint64(0x80), -1.0, 1.0) * pos.astype(np.float64) * w[strip]
+    slow = np.flatnonzero((pos >= k[strip]).any(axis=1))
+    streams = np.concatenate([philox(seed, q, ids[slow], iteration, replica[slow]) for q in range(12)], axis=1)
+    for j, stream in zip(slow, streams.tolist()):
+        at, got = 0, []
+        while len(got) < 3:
+            u, i = stream[at], stream[at] & 0x7F
+            z, at = (u & 0xFFFFFF00) * w[i], at + 1
+            if (u & 0xFFFFFF00) >= int(k[i]):
+                if i:
+                    h = y[i] + (y[i - 1] - y[i]) * stream[at] / 2 ** 32
+                    at += 1
+                else:
+                    r = 3.442619855899  # the reference's tail starts here (src/rng.c:173-218)
+                    z = r - math.log1p(-stream[at] / 2 ** 32) / r
+                    h = math.exp(-r * (z - 0.5 * r)) * stream[at + 1] / 2 ** 32
+                    at += 2
+                if h >= math.exp(-0.5 * z * z):
+                    continue
+            got.append(-z if u & 0x80 else z)
+        g[j] = got
+    return g
+
+
+def exact(case, seed):
+    """Free diffusion in a cube in closed form: the molecules' own normals and
+    positions folded back at the faces, in 64 bits.  With reactions a run is
+    one history of random events, which has no value outside the engine's
+    rules for their order: the outputs are compared with each other alone."""
+    if case["kind"] != "free" or case["n"] * case["iterations"] > 2e6:
+        return None
+    wl = workload(case, seed)
+    tables = ziggurat_tables()
+    half = wl.vertices.max()
+    single = case["precision"] == "fp32"
+    pos = wl.positions.astype(np.float32).astype(np.float64) if single else wl.positions.copy()
+    scale = wl.species_steps[0][0] * math.sqrt(0.5)
+    for it in range(case["iterations"]):
+        pos += scale * gaussians(seed, wl.ids, it, wl.replica, tables)
+        pos = np.where(pos > half, 2 * half - pos, np.where(pos < -half, -2 * half - pos, pos))
+        if single:
+            pos = pos.astype(np.float32).astype(np.float64)
+    return {"molecules": {"id": None, "species": None, "replica": None, "pos": pos, "subpart": None,
+                          "diffusion_time": None, "unimol_time": None, "flags": None, "counted_volume": None,
+                          "birthday": None}}
