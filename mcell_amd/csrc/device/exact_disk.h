@@ -333,12 +333,13 @@ __host__ __device__ double area_multiple(Pool& P, int head, double R2) {
 
 }  // namespace exd
 
-// exact_disk_utils.inl:840-1145; `full` set when the pool ran out.
-template <int N = exd::kPool>
+// exact_disk_utils.inl:840-1145; `full` set when the pool ran out.  A team's
+// lanes call it together (each with a pool of its own).
+template <int N = exd::kPool, class TeamT = Solo>
 __host__ __device__ __noinline__ double exact_disk_dev(const PartitionParams& PP, const WallRec64* __restrict__ walls,
                                               const uint32_t* __restrict__ off, const uint32_t* __restrict__ idx,
                                               const uint32_t* __restrict__ box, D3 loc, D3 mv, double R, D3 target,
-                                              bool* full) {
+                                              bool* full, TeamT T = TeamT{}) {
   using namespace exd;
   const double PI = 3.14159265358979323846;
   PoolT<N> P;
@@ -367,7 +368,7 @@ __host__ __device__ __noinline__ double exact_disk_dev(const PartitionParams& PP
   // bounding-box test below), so the cube loc +- R bounds their entry boxes
   const uint32_t db = region_box(PP, csp, loc.x - R, loc.y - R, loc.z - R, loc.x + R, loc.y + R, loc.z + R);
   const uint32_t e1 = off[csp + 1];
-  for (uint32_t k = next_overlap(box, off[csp], e1, db); k < e1; k = next_overlap(box, k + 1, e1, db)) {
+  for (uint32_t k = next_overlap(T, box, off[csp], e1, db); k < e1; k = next_overlap(T, box, k + 1, e1, db)) {
     const WallRec64& w = walls[idx[k]];
     D3 wv[3] = {{w.p0x, w.p0y, w.p0z}, {w.p1x, w.p1y, w.p1z}, {w.p2x, w.p2y, w.p2z}};
     D3 n = {w.nx, w.ny, w.nz};

@@ -13,6 +13,7 @@
 #pragma once
 #include "filter32.h"
 #include "path64.h"
+#include "team.h"
 
 namespace mcg {
 
@@ -24,7 +25,7 @@ namespace mcg {
 constexpr uint32_t kQueueShards = 2048;
 
 // The drains read the shards as one list: every workgroup prefix-sums the
-// shard counts in LDS (pre[0..kQueueShards], part[256] scratch; all 256
+// shard counts in LDS (pre[0..kQueueShards], part[4] scratch; all 256
 // threads call this) and deals list positions out grid-stride, so that
 // movers crowded into a few shards (hard movers cluster near surfaces and the
 // light pass is cell-ordered) still spread over the whole GPU.  Returns the
@@ -34,28 +35,39 @@ __device__ __forceinline__ uint32_t queue_prefix(const uint32_t* __restrict__ co
   static_assert(kQueueShards % 256 == 0, "shards per thread");
   constexpr uint32_t kPer = kQueueShards / 256;
   uint32_t local[kPer];
-  uint32_t sum = 0;
+#pragma unroll
   for (uint32_t k = 0; k < kPer; ++k) {
     const uint32_t sh = threadIdx.x * kPer + k;
     local[k] = sh < nshards ? count[sh] : 0u;
-    sum += local[k];
   }
-  part[threadIdx.x] = sum;
+  uint32_t sum = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < kPer; ++k) sum += local[k];
+  // scan within the wave, then over the workgroup's four waves
+  const uint32_t lane = __lane_id(), wave = threadIdx.x / 64u;
+  uint32_t incl = sum;
+#pragma unroll
+  for (uint32_t o = 1; o < 64; o <<= 1) {
+    const uint32_t v = __shfl_up(incl, o);
+    if (lane >= o) incl += v;
+  }
+  if (lane == 63) part[wave] = incl;
   __syncthreads();
-  for (uint32_t off = 1; off < 256; off <<= 1) {
-    const uint32_t v = threadIdx.x >= off ? part[threadIdx.x - off] : 0u;
-    __syncthreads();
-    part[threadIdx.x] += v;
-    __syncthreads();
+  uint32_t run = incl - sum, total = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < 4; ++w) {
+    const uint32_t v = part[w];
+    if (w < wave) run += v;
+    total += v;
   }
-  uint32_t run = part[threadIdx.x] - sum;
+#pragma unroll
   for (uint32_t k = 0; k < kPer; ++k) {
     pre[threadIdx.x * kPer + k] = run;
     run += local[k];
   }
-  if (threadIdx.x == 255) pre[kQueueShards] = part[255];
+  if (threadIdx.x == 255) pre[kQueueShards] = total;
   __syncthreads();
-  return pre[kQueueShards];
+  return total;
 }
 
 // The queued value at list position q < total: the last shard k with
@@ -70,6 +82,44 @@ __device__ __forceinline__ uint32_t queue_at(const uint32_t* __restrict__ slots,
   }
   return slots[(size_t)lo * shard_cap + (q - pre[lo])];
 }
+
+// How a list of full steps is dealt to the waves of a grid.  The full step is
+// one serial chain per mover, and a wave waits for the union of its lanes'
+// paths: 64 movers in one wave take several times as long as one, while the
+// lists are often far shorter than the lanes of the chip.  So a wave takes
+// only as many movers at a time as it must for the grid to hold the list --
+// one per lane, or with teams one per team, the teams as large as the grid's
+// lanes allow.  Measured (drain of one iteration, 64 movers a wave / spread):
+// 4,000 molecules in a box 115 / 73 us, 50,000 124 / 71 us, 110,000 around a
+// sphere of 5,120 triangles 137 / 76 us.
+template <class TeamT>
+struct Spread {
+  TeamT team;
+  uint32_t block_first, wave_first;  // list position of the workgroup's and the wave's first mover
+  uint32_t mine;                     // this lane's mover among the wave's; none: kInvalid
+  uint32_t stride;                   // positions between two turns of a wave
+  __device__ __forceinline__ explicit Spread(uint32_t total) {
+    const uint32_t per_block = blockDim.x / 64u, waves = gridDim.x * per_block;
+    uint32_t movers;  // a wave takes this many at a time
+    if constexpr (TeamT::kShared) {
+      uint32_t size = 64u;
+      while (size > 1u && (uint64_t)total * size > (uint64_t)waves * 64u) size >>= 1;
+      team.size = size;
+      team.rank = __lane_id() & (size - 1u);
+      movers = 64u / size;
+      mine = __lane_id() / size;
+    } else {
+      movers = total / waves + (total % waves != 0);
+      movers = movers > 64u ? 64u : (movers ? movers : 1u);
+      mine = __lane_id() < movers ? __lane_id() : kInvalid;
+    }
+    block_first = blockIdx.x * per_block * movers;
+    wave_first = block_first + (threadIdx.x / 64u) * movers;
+    stride = waves * movers;
+  }
+  // the list position of this lane's mover in the turn that starts at base (>= total: none)
+  __device__ __forceinline__ uint32_t at(uint32_t base) const { return mine == kInvalid ? kInvalid : base + mine; }
+};
 
 // Wave-aggregated append of the `want` lanes' value to a shard: one atomic
 // per wave, slot order by lane.

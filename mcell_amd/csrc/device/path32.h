@@ -34,7 +34,8 @@ struct Walls32View {
 // plane, so passes repeat until one moves nothing.  Returns false when
 // kRoundPasses passes did not settle (the caller reports ERR_ROUND32).
 constexpr int kRoundPasses = 8;
-__device__ __forceinline__ bool round_to_fp32_same_side(const PartitionParams& P, const WallRec64* __restrict__ walls,
+template <class TeamT>
+__device__ __forceinline__ bool round_to_fp32_same_side(const TeamT& T, const PartitionParams& P, const WallRec64* __restrict__ walls,
                                                      const uint32_t* __restrict__ off,
                                                      const uint32_t* __restrict__ idx,
                                                      const uint32_t* __restrict__ box, double px, double py,
@@ -50,7 +51,7 @@ __device__ __forceinline__ bool round_to_fp32_same_side(const PartitionParams& P
     for (int pass = 0; pass < kRoundPasses && !settled; ++pass) {
       bool moved = false;
       const uint32_t e1 = off[s + 1];
-      for (uint32_t k = next_overlap(box, off[s], e1, pb); k < e1; k = next_overlap(box, k + 1, e1, pb)) {
+      for (uint32_t k = next_overlap(T, box, off[s], e1, pb); k < e1; k = next_overlap(T, box, k + 1, e1, pb)) {
         const WallRec64& w = walls[idx[k]];
         double sd = dot3(D3{w.nx, w.ny, w.nz}, D3{px, py, pz}) - w.d;
         double sf = dot3(D3{w.nx, w.ny, w.nz}, D3{(double)fx, (double)fy, (double)fz}) - w.d;

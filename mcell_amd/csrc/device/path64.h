@@ -5,6 +5,7 @@
 // FP64 CPU evaluation of the same formulas.
 #pragma once
 #include "rng.h"
+#include "team.h"
 #include "types.h"
 #include "wallbox.h"
 
@@ -161,7 +162,9 @@ __device__ __forceinline__ void jump_away_line(D3 p, double k, D3 A, D3 B, D3 n,
   v.z -= tiny * f.z;
 }
 
-// collision_utils.inl:629-812 (FP64, update_move = true)
+// collision_utils.inl:629-812 (FP64, update_move = true).  kDraw false: the
+// outcome alone; a re-draw is reported and move and stream stay as they are.
+template <bool kDraw>
 __device__ __forceinline__ int collide_wall64(const WallRec64& w, D3 pos, D3& move, double& t, D3& hit,
                                               PhiloxStream& rng) {
   D3 n = {w.nx, w.ny, w.nz};
@@ -181,6 +184,7 @@ __device__ __forceinline__ int collide_wall64(const WallRec64& w, D3 pos, D3& mo
   double a;
   if (dd == 0) {
     if (dv != 0) return WALL_MISS;
+    if (!kDraw) return WALL_REDO;
     a = (abs_max_2vec(pos, move) + 1.0) * POS_EPS;
     if ((rng.u32() & 1u) == 0) a = -a;
     move = {move.x - a * n.x, move.y - a * n.y, move.z - a * n.z};
@@ -206,19 +210,19 @@ __device__ __forceinline__ int collide_wall64(const WallRec64& w, D3 pos, D3& mo
     if (g > h) {
       if (c * w.uv1u + g < h + w.uv1u * w.uv2v) return dv > 0 ? WALL_BACK : WALL_FRONT;
       if (!distinguishable(c * w.uv1u + g, h + w.uv1u * w.uv2v, POS_EPS)) {
-        jump_away_line(pos, a, d3(w.p1x, w.p1y, w.p1z), d3(w.p2x, w.p2y, w.p2z), n, rng, move);
+        if (kDraw) jump_away_line(pos, a, d3(w.p1x, w.p1y, w.p1z), d3(w.p2x, w.p2y, w.p2z), n, rng, move);
         return WALL_REDO;
       }
       return WALL_MISS;
     }
     if (!distinguishable(g, h, POS_EPS)) {
-      jump_away_line(pos, a, d3(w.p2x, w.p2y, w.p2z), d3(w.p0x, w.p0y, w.p0z), n, rng, move);
+      if (kDraw) jump_away_line(pos, a, d3(w.p2x, w.p2y, w.p2z), d3(w.p0x, w.p0y, w.p0z), n, rng, move);
       return WALL_REDO;
     }
     return WALL_MISS;
   }
   if (!distinguishable(c, 0.0, POS_EPS)) {
-    jump_away_line(pos, a, d3(w.p0x, w.p0y, w.p0z), d3(w.p1x, w.p1y, w.p1z), n, rng, move);
+    if (kDraw) jump_away_line(pos, a, d3(w.p0x, w.p0y, w.p0z), d3(w.p1x, w.p1y, w.p1z), n, rng, move);
     return WALL_REDO;
   }
   return WALL_MISS;
@@ -276,9 +280,10 @@ struct WallHit {
 };
 
 // get_closest_wall_collision (collision_utils.inl:819-914, FP64): nearest hit
-// inside `subpart`; a REDO restarts the scan of this subpartition with the
-// re-drawn displacement.
-__device__ __forceinline__ bool closest_wall_in_subpart64(const PartitionParams& P, const WallRec64* __restrict__ walls,
+// inside `subpart` (the first in list order among equal ones); a REDO
+// restarts the scan of this subpartition with the re-drawn displacement.
+__device__ __forceinline__ bool closest_wall_in_subpart64(const Solo&, const PartitionParams& P,
+                                                          const WallRec64* __restrict__ walls,
                                                           const uint32_t* __restrict__ off,
                                                           const uint32_t* __restrict__ idx,
                                                           const uint32_t* __restrict__ box, uint32_t subpart,
@@ -298,7 +303,7 @@ __device__ __forceinline__ bool closest_wall_in_subpart64(const PartitionParams&
       if (wi == last_hit) continue;
       double t;
       D3 hit;
-      int ct = collide_wall64(walls[wi], pos, move, t, hit, rng);
+      int ct = collide_wall64<true>(walls[wi], pos, move, t, hit, rng);
       if (ct == WALL_REDO) {
         restarted = true;
         break;
@@ -322,6 +327,81 @@ __device__ __forceinline__ bool closest_wall_in_subpart64(const PartitionParams&
     }
   }
   return found;
+}
+
+// The same by a team: its lanes take the list's entries in turn (entry k0 +
+// rank, k0 + rank + size, ...) and test them without drawing; the first entry
+// in list order that asks for a re-draw then draws, whatever came before it:
+// the hits found up to there are dropped, as the restart drops them.
+__device__ __forceinline__ bool closest_wall_in_subpart64(const Team& T, const PartitionParams& P,
+                                                          const WallRec64* __restrict__ walls,
+                                                          const uint32_t* __restrict__ off,
+                                                          const uint32_t* __restrict__ idx,
+                                                          const uint32_t* __restrict__ box, uint32_t subpart,
+                                                          uint32_t last_hit, D3 pos, D3& move, PhiloxStream& rng,
+                                                          WallHit& best, uint32_t& err) {
+  const uint32_t k0 = off[subpart], k1 = off[subpart + 1];
+  if (k0 == k1) return false;
+  int redo = 0;
+  for (;;) {
+    bool found = false;
+    double closest = 1e20;  // TIME_FOREVER
+    uint32_t k_best = 0, k_redo = k1;
+    const uint32_t sb = segment_box(P, subpart, pos.x, pos.y, pos.z, move.x, move.y, move.z);
+    const uint32_t step = kOverlapGroup * T.size;
+    for (uint32_t k = k0 + T.rank; k < k1 && k_redo == k1; k += step) {
+      uint32_t bx[kOverlapGroup], near = 0;
+#pragma unroll
+      for (uint32_t u = 0; u < kOverlapGroup; ++u) {
+        const uint32_t e = k + u * T.size;
+        bx[u] = box[e < k1 ? e : k1 - 1];
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < kOverlapGroup; ++u)
+        near |= (k + u * T.size < k1 && boxes_overlap(bx[u], sb)) ? 1u << u : 0u;
+      for (; near; near &= near - 1) {
+        const uint32_t e = k + (uint32_t)(__ffs((int)near) - 1) * T.size;
+        const uint32_t wi = idx[e];
+        if (wi == last_hit) continue;
+        double t;
+        D3 hit;
+        const int ct = collide_wall64<false>(walls[wi], pos, move, t, hit, rng);
+        if (ct == WALL_REDO) {
+          k_redo = e;
+          break;
+        }
+        if (ct != WALL_MISS) {
+          if (subpart_index(P, hit) != subpart) continue;
+          if (t < closest) {
+            found = true;
+            closest = t;
+            k_best = e;
+            best.wall = wi;
+            best.type = ct;
+            best.t = t;
+            best.pos = hit;
+          }
+        }
+      }
+    }
+    k_redo = team_min_u32(T, k_redo);
+    if (k_redo == k1) {
+      if (team_first(T, found) == 64u) return false;
+      const uint32_t r = team_min(T, found, closest, k_best);
+      best.wall = team_get(T, best.wall, r);
+      best.type = team_get(T, best.type, r);
+      best.t = team_get(T, best.t, r);
+      best.pos = {team_get(T, best.pos.x, r), team_get(T, best.pos.y, r), team_get(T, best.pos.z, r)};
+      return true;
+    }
+    if (++redo > kMaxRedo) {
+      err |= ERR_REDO;
+      return false;
+    }
+    double t;
+    D3 hit;
+    (void)collide_wall64<true>(walls[idx[k_redo]], pos, move, t, hit, rng);
+  }
 }
 
 // One step of a volume molecule that cannot react: Brownian displacement and
@@ -350,7 +430,7 @@ __device__ __forceinline__ bool diffuse_reflect64(const PartitionParams& P, cons
     }
     uint32_t start = subpart_of(P, sx, sy, sz);
     WallHit hit;
-    bool found = closest_wall_in_subpart64(P, walls, off, idx, box, start, last_hit, pos, disp, rng, hit, err);
+    bool found = closest_wall_in_subpart64(Solo{}, P, walls, off, idx, box, start, last_hit, pos, disp, rng, hit, err);
     if (!found) {
       // the walk only runs when the move leaves the start subpartition
       D3 dst = {pos.x + part_disp.x, pos.y + part_disp.y, pos.z + part_disp.z};
@@ -360,7 +440,7 @@ __device__ __forceinline__ bool diffuse_reflect64(const PartitionParams& P, cons
         SubpartWalk64 walk;
         walk.init(P, pos, start, part_disp);
         while (walk.next(P, err)) {
-          if (closest_wall_in_subpart64(P, walls, off, idx, box, walk.cur, last_hit, pos, disp, rng, hit, err)) {
+          if (closest_wall_in_subpart64(Solo{}, P, walls, off, idx, box, walk.cur, last_hit, pos, disp, rng, hit, err)) {
             found = true;
             break;
           }

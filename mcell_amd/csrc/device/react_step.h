@@ -12,6 +12,7 @@
 #include "path32.h"
 #include "light.h"
 #include "react.h"
+#include "team.h"
 
 namespace mcg {
 
@@ -117,7 +118,7 @@ __device__ __forceinline__ bool segment_first_wall(const ReactParams& R, D3 pos,
     return false;
   }
   const uint32_t start = subpart_of(R.P, sx, sy, sz);
-  if (closest_wall_in_subpart64(R.P, R.walls, R.off, R.idx, R.ent_box, start, skip, pos, disp, rng, hit, err))
+  if (closest_wall_in_subpart64(Solo{}, R.P, R.walls, R.off, R.idx, R.ent_box, start, skip, pos, disp, rng, hit, err))
     return true;
   const D3 dst = {pos.x + part_disp.x, pos.y + part_disp.y, pos.z + part_disp.z};
   int dx, dy, dz;
@@ -126,7 +127,8 @@ __device__ __forceinline__ bool segment_first_wall(const ReactParams& R, D3 pos,
   SubpartWalk64 walk;
   walk.init(R.P, pos, start, part_disp);
   while (walk.next(R.P, err))
-    if (closest_wall_in_subpart64(R.P, R.walls, R.off, R.idx, R.ent_box, walk.cur, skip, pos, disp, rng, hit, err))
+    if (closest_wall_in_subpart64(Solo{}, R.P, R.walls, R.off, R.idx, R.ent_box, walk.cur, skip, pos, disp, rng, hit,
+                                  err))
       return true;
   return false;
 }
@@ -169,9 +171,10 @@ struct Proposal {
 constexpr uint32_t kPadMoverIsB = 1u << 31;  // the mover is the class's reactant b
 
 // Closest wall in one subpartition (FP64; the entry-box pre-test first).
-__device__ __forceinline__ bool closest_wall(const ReactParams& R, uint32_t s, uint32_t last_hit, D3 pos, D3& disp,
-                                             PhiloxStream& rng, WallHit& hit, uint32_t& err) {
-  return closest_wall_in_subpart64(R.P, R.walls, R.off, R.idx, R.ent_box, s, last_hit, pos, disp, rng, hit, err);
+template <class TeamT>
+__device__ __forceinline__ bool closest_wall(const TeamT& T, const ReactParams& R, uint32_t s, uint32_t last_hit,
+                                             D3 pos, D3& disp, PhiloxStream& rng, WallHit& hit, uint32_t& err) {
+  return closest_wall_in_subpart64(T, R.P, R.walls, R.off, R.idx, R.ent_box, s, last_hit, pos, disp, rng, hit, err);
 }
 
 // The snapshot range of species t's molecules in the k-th subpartition of the
@@ -192,13 +195,15 @@ __device__ __forceinline__ void set_range(const CellGrid& G, const SubpartSet& s
 
 // The next molecule collision after key (t_last, id_last) in time order
 // (ties: larger partner id first, diffuse_react_event.cpp:354-358), strictly
-// before t_limit.  Scans the partner lists of the collected subpartitions.
-template <typename PosT>
-__device__ __forceinline__ bool next_collision(const ReactParams& R, const Snapshot<PosT>& S, const SubpartSet& set,
-                                               uint32_t replica, uint32_t my_species, uint32_t my_id, D3 pos,
-                                               D3 disp, double t_limit, double t_last, uint32_t id_last,
-                                               bool first, double& t_best, uint32_t& slot_best, D3& pos_best,
-                                               int32_t& rxn_best, uint32_t& candidates) {
+// before t_limit.  Scans the partner lists of the collected subpartitions:
+// a team's lanes take up to four subpartitions at a time and share the
+// partners of each.
+template <typename PosT, class TeamT>
+__device__ __forceinline__ bool next_collision(const TeamT& T, const ReactParams& R, const Snapshot<PosT>& S,
+                                               const SubpartSet& set, uint32_t replica, uint32_t my_species,
+                                               uint32_t my_id, D3 pos, D3 disp, double t_limit, double t_last,
+                                               uint32_t id_last, bool first, double& t_best, uint32_t& slot_best,
+                                               D3& pos_best, int32_t& rxn_best, uint32_t& candidates) {
   const double sigma2 = R.P.rxn_radius * R.P.rxn_radius;
   bool found = false;
   uint32_t id_best = 0;
@@ -213,26 +218,30 @@ __device__ __forceinline__ bool next_collision(const ReactParams& R, const Snaps
   // current one's partners are tested, and partner positions two at a time
   // (the result does not depend on the order: the key is a total order)
   constexpr int kGroup = 2;
+  const int cells = T.size < 4u ? (int)T.size : 4;  // subpartitions the team reads at a time
+  const uint32_t per_cell = T.size / (uint32_t)cells;
+  const uint32_t lane = T.rank / (uint32_t)cells;   // this lane's place among those of its subpartition
+  const int k_first = (int)(T.rank % (uint32_t)cells);
   for (uint32_t t = 0; t < R.G.ns && set.n > 0; ++t) {
     const int32_t rx = R.pair_rxn[my_species * R.num_species + t];
     if (rx < 0) continue;
-    uint32_t n0, n1;
-    set_range(R.G, set, 0, replica, t, n0, n1);
-    for (int k = 0; k < set.n; ++k) {
-      const uint32_t j0 = n0, j1 = n1;
-      if (k + 1 < set.n) set_range(R.G, set, k + 1, replica, t, n0, n1);
-      for (uint32_t jb = j0; jb < j1; jb += kGroup) {
+    uint32_t n0 = 0, n1 = 0;
+    if (k_first < set.n) set_range(R.G, set, k_first, replica, t, n0, n1);
+    for (int k = k_first; k < set.n; k += cells) {
+      const uint32_t j0 = n0 + lane, j1 = n1;
+      if (k + cells < set.n) set_range(R.G, set, k + cells, replica, t, n0, n1);
+      for (uint32_t jb = j0; jb < j1; jb += kGroup * per_cell) {
         PosT gx[kGroup], gy[kGroup], gz[kGroup];
 #pragma unroll
         for (int u = 0; u < kGroup; ++u) {
-          const uint32_t j = jb + u < j1 ? jb + u : j1 - 1;
+          const uint32_t j = jb + u * per_cell < j1 ? jb + u * per_cell : j1 - 1;
           gx[u] = S.x[j];
           gy[u] = S.y[j];
           gz[u] = S.z[j];
         }
 #pragma unroll
         for (int u = 0; u < kGroup; ++u) {
-          const uint32_t j = jb + u;
+          const uint32_t j = jb + u * per_cell;
           if (j >= j1) break;
           if (box.outside(gx[u], gy[u], gz[u])) continue;
           double tt;
@@ -260,7 +269,18 @@ __device__ __forceinline__ bool next_collision(const ReactParams& R, const Snaps
       }
     }
   }
-  return found;
+  if constexpr (TeamT::kShared) {
+    if (team_first(T, found) == 64u) return false;
+    candidates = team_sum(T, candidates);
+    const uint32_t r = team_min(T, found, t_best, ~id_best);
+    t_best = team_get(T, t_best, r);
+    slot_best = team_get(T, slot_best, r);
+    pos_best = {team_get(T, pos_best.x, r), team_get(T, pos_best.y, r), team_get(T, pos_best.z, r)};
+    rxn_best = team_get(T, rxn_best, r);
+    return true;
+  } else {
+    return found;
+  }
 }
 
 __device__ __forceinline__ bool cmp_eq_d(double a, double b, double eps) { return fabs(a - b) < eps; }
@@ -284,12 +304,13 @@ struct MoverEnd {
 // exact_disk is exactly 1 unless an entry of the collision point's
 // subpartition has a box overlapping the point's +-R cube (the walls it
 // would process; exact_disk_dev returns 1 when it processes none).
-__device__ __forceinline__ bool disk_meets_walls(const ReactParams& R, D3 cp) {
+template <class TeamT>
+__device__ __forceinline__ bool disk_meets_walls(const TeamT& T, const ReactParams& R, D3 cp) {
   const double r = R.P.rxn_radius;
   const uint32_t csp = subpart_index(R.P, cp);
   const uint32_t db = region_box(R.P, csp, cp.x - r, cp.y - r, cp.z - r, cp.x + r, cp.y + r, cp.z + r);
   const uint32_t e1 = R.off[csp + 1];
-  return next_overlap(R.ent_box, R.off[csp], e1, db) < e1;
+  return next_overlap(T, R.ent_box, R.off[csp], e1, db) < e1;
 }
 
 // The molecule's unimolecular time at the start of its step
@@ -330,8 +351,11 @@ __device__ __forceinline__ double start_unimol_time(const UnimolRec* __restrict_
 // stayed); they are passed as the reference's ray trace goes on after them
 // (collide_and_react_with_vol_mol returns false for a kept mover,
 // diffuse_react_event.cpp:463-470, 823-827).
-template <typename PosT, int kPoolN>
-__device__ __forceinline__ bool react_mover(const ReactParams& R, const Snapshot<PosT>& S, const SpeciesRec& sp,
+//
+// The team's lanes call it together with the same mover and get the same
+// result (team.h).
+template <typename PosT, int kPoolN, class TeamT>
+__device__ __forceinline__ bool react_mover(const TeamT& L, const ReactParams& R, const Snapshot<PosT>& S, const SpeciesRec& sp,
                                             const ZigguratTables& T, D3 pos, uint32_t idv, uint32_t tag, double toff,
                                             double utime, double birth, double barrier, uint32_t pass_through,
                                             uint32_t born_tile, Proposal& prop, MoverEnd& out, uint32_t& err,
@@ -401,12 +425,12 @@ __device__ __forceinline__ bool react_mover(const ReactParams& R, const Snapshot
     const uint32_t dest = subpart_of(R.P, dx, dy, dz);
     WallHit hit;
     uint32_t hit_sp = start;
-    bool found = closest_wall(R, start, last_hit, pos, disp, rng, hit, err);
+    bool found = closest_wall(L, R, start, last_hit, pos, disp, rng, hit, err);
     if (!found && dest != start) {
       SubpartWalk64 walk;
       walk.init(R.P, pos, start, part_disp);
       while (walk.next(R.P, err)) {
-        if (closest_wall(R, walk.cur, last_hit, pos, disp, rng, hit, err)) {
+        if (closest_wall(L, R, walk.cur, last_hit, pos, disp, rng, hit, err)) {
           found = true;
           hit_sp = walk.cur;
           break;
@@ -434,7 +458,7 @@ __device__ __forceinline__ bool react_mover(const ReactParams& R, const Snapshot
         D3 cp;
         int32_t rx;
         uint32_t candidates;
-        if (!next_collision(R, S, set, rep, spc, idv, pos, disp, t_limit, t_last, id_last, first, tc, slot, cp, rx,
+        if (!next_collision(L, R, S, set, rep, spc, idv, pos, disp, t_limit, t_last, id_last, first, tc, slot, cp, rx,
                             candidates))
           break;
         first = false;
@@ -445,7 +469,7 @@ __device__ __forceinline__ bool react_mover(const ReactParams& R, const Snapshot
           continue;
         }
         double factor = 1.0;
-        if (disk_meets_walls(R, cp)) {
+        if (disk_meets_walls(L, R, cp)) {
           if constexpr (kPoolN == 0) {
             out.exd = true;
             return false;
@@ -453,7 +477,7 @@ __device__ __forceinline__ bool react_mover(const ReactParams& R, const Snapshot
             bool full = false;
             const D3 target = {(double)S.x[slot], (double)S.y[slot], (double)S.z[slot]};
             factor = exact_disk_dev<kPoolN>(R.P, R.walls, R.off, R.idx, R.ent_box, cp, disp, R.P.rxn_radius, target,
-                                            &full);
+                                            &full, L);
             if (full) {
               if constexpr (kPoolN >= exd::kPool) {
                 err |= ERR_EXD;

@@ -203,7 +203,8 @@ int mcg_set_geometry(mcg_ctx* c, const double* vertices, uint32_t nv, const uint
   }
   // sub-cell box of every entry: the wall's bounding box within the entry's subpartition
   std::vector<uint32_t> eb;
-  entry_boxes(P, c->walls_host, c->off_host, c->idx_host, eb);
+  const uint64_t scanned = entry_boxes(P, c->walls_host, c->off_host, c->idx_host, eb);
+  c->long_wall_lists = !c->idx_host.empty() && scanned >= 64 * (uint64_t)c->idx_host.size();
   if (c->ent64.alloc(e64.size()) || c->ent32.alloc(e32.size()) || c->ent_box.alloc(eb.size()))
     return fail(MCG_E_NOMEM, "wall entry buffers");
   HIP_TRY(hipMemcpy(c->ent64.p, e64.data(), e64.size() * sizeof(WallRec64), hipMemcpyHostToDevice));

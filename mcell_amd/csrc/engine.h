@@ -164,6 +164,13 @@ struct mcg_ctx {
   mcg::DevBuf<mcg::WallRec32> ent32;
   mcg::DevBuf<uint32_t> ent_box;  // sub-cell box of every list entry
   bool have_geometry = false;
+  // full steps run by teams of lanes (device/team.h): worth the exchanges
+  // only where a mover's wall lists are long.  The line is a mean list of 64
+  // entries, eight lanes with eight boxes each: 1.25M molecules among spheres
+  // of 20,480 triangles (mean list 233) take 2.4 ms an iteration with teams
+  // and 3.5 without; with the 12 walls of a box teams are 10-20 % slower, and
+  // at a mean of 19 (a sphere of 5,120 triangles) the two are equal.
+  bool long_wall_lists = false;
   // surface classes
   std::vector<uint32_t> wall_class_host;
   mcg::DevBuf<uint32_t> wall_class_d;

@@ -58,6 +58,7 @@ ReactPipeline<PosT> make_pipeline(mcg_ctx* c, PosT* x, PosT* y, PosT* z, PosT* s
   p.R.ent64 = c->ent64.p;
   p.R.ent_box = c->ent_box.p;
   p.queue = SlowQueue{c->queue.p, c->qcount.p, 0};
+  p.teams = c->long_wall_lists;
   p.R.G = r.grid;
   p.R.G.start = r.cell_start.p;
   p.R.rxns = r.rxns_d.p;

@@ -190,17 +190,21 @@ void bin_walls(const PartitionParams& P, const std::vector<WallRec64>& walls, st
   for (size_t i = 0; i < pairs.size(); ++i) idx[i] = pairs[i].second;
 }
 
-void entry_boxes(const PartitionParams& P, const std::vector<WallRec64>& walls, const std::vector<uint32_t>& off,
-                 const std::vector<uint32_t>& idx, std::vector<uint32_t>& box) {
+uint64_t entry_boxes(const PartitionParams& P, const std::vector<WallRec64>& walls, const std::vector<uint32_t>& off,
+                     const std::vector<uint32_t>& idx, std::vector<uint32_t>& box) {
   box.assign(std::max<size_t>(idx.size(), 1), kBoxAll);
   const size_t n3 = off.size() - 1;
-  for (size_t s = 0; s < n3; ++s)
+  uint64_t scanned = 0;
+  for (size_t s = 0; s < n3; ++s) {
+    scanned += (uint64_t)(off[s + 1] - off[s]) * (off[s + 1] - off[s]);
     for (uint32_t k = off[s]; k < off[s + 1]; ++k) {
       const WallRec64& w = walls[idx[k]];
       box[k] = region_box(P, (uint32_t)s, std::min({w.p0x, w.p1x, w.p2x}), std::min({w.p0y, w.p1y, w.p2y}),
                           std::min({w.p0z, w.p1z, w.p2z}), std::max({w.p0x, w.p1x, w.p2x}),
                           std::max({w.p0y, w.p1y, w.p2y}), std::max({w.p0z, w.p1z, w.p2z}));
     }
+  }
+  return scanned;
 }
 
 }  // namespace mcg

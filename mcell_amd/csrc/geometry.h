@@ -20,8 +20,9 @@ void bin_walls(const PartitionParams& P, const std::vector<WallRec64>& walls, st
                std::vector<uint32_t>& idx);
 
 // The sub-cell box (device/wallbox.h) of every list entry: the wall's
-// bounding box within the entry's subpartition.
-void entry_boxes(const PartitionParams& P, const std::vector<WallRec64>& walls, const std::vector<uint32_t>& off,
+// bounding box within the entry's subpartition.  Returns the sum of the
+// squared list lengths (over the entries: the mean list an entry sits in).
+uint64_t entry_boxes(const PartitionParams& P, const std::vector<WallRec64>& walls, const std::vector<uint32_t>& off,
                  const std::vector<uint32_t>& idx, std::vector<uint32_t>& box);
 
 }  // namespace mcg

@@ -133,7 +133,7 @@ __global__ __launch_bounds__(256) void k_mid64(MolView64 m, SpeciesTable species
                                                SlowQueue HQ, HitTrace trace) {
   __shared__ ZigguratTables T;
   __shared__ uint32_t pre[kQueueShards + 1];
-  __shared__ uint32_t part[256];
+  __shared__ uint32_t part[4];
   const uint32_t total = queue_prefix(MQ.count, MQ.nshards, pre, part);
   if ((uint64_t)blockIdx.x * blockDim.x >= total) return;
   stage_ziggurat(T);
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(256) void k_hard64(MolView64 m, SpeciesTable specie
                                                 unsigned long long* __restrict__ ctr) {
   __shared__ ZigguratTables T;
   __shared__ uint32_t pre[kQueueShards + 1];
-  __shared__ uint32_t part[256];
+  __shared__ uint32_t part[4];
   // the shards read as one list, grid-stride
   const uint32_t total = queue_prefix(Q.count, Q.nshards, pre, part);
   if ((uint64_t)blockIdx.x * blockDim.x >= total) return;
@@ -249,7 +249,7 @@ __global__ __launch_bounds__(256) void k_mid32(MolView32 m, SpeciesTable species
                                                uint32_t iteration, SlowQueue MQ, SlowQueue HQ, HitTrace trace) {
   __shared__ ZigguratTables T;
   __shared__ uint32_t pre[kQueueShards + 1];
-  __shared__ uint32_t part[256];
+  __shared__ uint32_t part[4];
   const uint32_t total = queue_prefix(MQ.count, MQ.nshards, pre, part);
   if ((uint64_t)blockIdx.x * blockDim.x >= total) return;
   stage_ziggurat(T);
@@ -285,7 +285,7 @@ __global__ __launch_bounds__(256) void k_hard32(MolView32 m, SpeciesTable specie
                                                 unsigned long long* __restrict__ ctr) {
   __shared__ ZigguratTables T;
   __shared__ uint32_t pre[kQueueShards + 1];
-  __shared__ uint32_t part[256];
+  __shared__ uint32_t part[4];
   // the shards read as one list, grid-stride
   const uint32_t total = queue_prefix(Q.count, Q.nshards, pre, part);
   if ((uint64_t)blockIdx.x * blockDim.x >= total) return;
@@ -311,7 +311,7 @@ __global__ __launch_bounds__(256) void k_hard32(MolView32 m, SpeciesTable specie
                                          tw, tn, n_reflect, n_cross);
     if (!alive) m.tag[i] = tag | (MF_DEFUNCT << 8);
     float fx, fy, fz;
-    if (!round_to_fp32_same_side(P, W.w64, W.off, W.idx, W.box, pos.x, pos.y, pos.z, &fx, &fy, &fz))
+    if (!round_to_fp32_same_side(Solo{}, P, W.w64, W.off, W.idx, W.box, pos.x, pos.y, pos.z, &fx, &fy, &fz))
       err |= ERR_ROUND32;
     m.x[i] = fx;
     m.y[i] = fy;

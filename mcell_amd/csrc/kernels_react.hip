@@ -122,25 +122,30 @@ __global__ __launch_bounds__(256) void k_scatter(RMolView<PosT> m, uint32_t n, c
 // ----------------------------------------------------------------- moves --
 // FP32 form: the end point in FP32, kept on the FP64 point's side of nearby
 // wall planes.  Returns the error bit of a rounding that did not settle.
-__device__ __forceinline__ uint32_t store_pos(const ReactParams& R, double* x, double* y, double* z, uint32_t j, D3 p,
-                                              bool) {
+// A team's lanes call it together; the leader stores.
+template <class TeamT>
+__device__ __forceinline__ uint32_t store_pos(const TeamT& T, const ReactParams& R, double* x, double* y, double* z,
+                                              uint32_t j, D3 p, bool) {
+  if (!T.leader()) return 0;
   x[j] = p.x;
   y[j] = p.y;
   z[j] = p.z;
   return 0;
 }
-__device__ __forceinline__ uint32_t store_pos(const ReactParams& R, float* x, float* y, float* z, uint32_t j, D3 p,
-                                              bool near_plane) {
+template <class TeamT>
+__device__ __forceinline__ uint32_t store_pos(const TeamT& T, const ReactParams& R, float* x, float* y, float* z,
+                                              uint32_t j, D3 p, bool near_plane) {
   float fx, fy, fz;
   uint32_t e = 0;
   if (near_plane) {
-    if (!round_to_fp32_same_side(R.P, R.walls, R.off, R.idx, R.ent_box, p.x, p.y, p.z, &fx, &fy, &fz))
+    if (!round_to_fp32_same_side(T, R.P, R.walls, R.off, R.idx, R.ent_box, p.x, p.y, p.z, &fx, &fy, &fz))
       e = ERR_ROUND32;
   } else {
     fx = (float)p.x;
     fy = (float)p.y;
     fz = (float)p.z;
   }
+  if (!T.leader()) return 0;
   x[j] = fx;
   y[j] = fy;
   z[j] = fz;
@@ -203,8 +208,10 @@ __device__ __forceinline__ void append_slot(bool want, uint32_t j, uint32_t* __r
 // A step that needs a larger exact_disk pool than kPoolN (react_mover)
 // writes nothing and sets `deferred` (the caller queues the mover for a pass
 // with a larger pool).
-template <typename PosT, int kPoolN>
-__device__ __forceinline__ bool move_one(const ReactParams& R, const Snapshot<PosT>& S, const RMolView<PosT>& src,
+// The team's lanes call it together; the leader writes and returns the
+// outcome, the others return false with nothing due or deferred.
+template <typename PosT, int kPoolN, class TeamT>
+__device__ __forceinline__ bool move_one(const TeamT& L, const ReactParams& R, const Snapshot<PosT>& S, const RMolView<PosT>& src,
                                          const RMolView<PosT>& out, uint32_t j, SpeciesTable species,
                                          const ZigguratTables& T, double barrier, uint32_t propose_only,
                                          Proposal* __restrict__ prop, uint32_t* __restrict__ owner,
@@ -238,14 +245,17 @@ __device__ __forceinline__ bool move_one(const ReactParams& R, const Snapshot<Po
   const uint32_t pass_through = R.kept ? R.kept[j] : 0u;
   const uint32_t born = R.born ? R.born[j] : 0u;
   if (moves)
-    proposed = react_mover<PosT, kPoolN>(R, S, sp, T, pos, idv, tag, toff, utime, birth, barrier, pass_through, born,
-                                         p, e, err, set_lds);
-  deferred = e.exd;
-  if (deferred) {
-    due = false;
-    if (err) atomicOr(err_out, err);
+    proposed = react_mover<PosT, kPoolN>(L, R, S, sp, T, pos, idv, tag, toff, utime, birth, barrier, pass_through,
+                                         born, p, e, err, set_lds);
+  deferred = e.exd && L.leader();
+  due = false;
+  if (e.exd) {
+    if (err && L.leader()) atomicOr(err_out, err);
     return false;
   }
+  const bool commits = !proposed || propose_only;
+  if (commits) err |= store_pos(L, R, out.x, out.y, out.z, j, e.pos, e.near_plane);
+  if (!L.leader()) return false;
   due = e.due != 0;
   if (due) {
     // the unimolecular event, settled after the phase's bimolecular claims
@@ -275,8 +285,7 @@ __device__ __forceinline__ bool move_one(const ReactParams& R, const Snapshot<Po
       else atomicMin(owner + p.partner_slot, idv);
     }
   }
-  if (!proposed || propose_only) {
-    err |= store_pos(R, out.x, out.y, out.z, j, e.pos, e.near_plane);
+  if (commits) {
     out.id[j] = idv;
     uint32_t t2 = (tag & ~(MF_STEP_FLAGS << 8)) | (e.mature ? (MF_MATURE << 8) : 0u);
     if (e.cont && !propose_only) {
@@ -316,7 +325,7 @@ __device__ __forceinline__ bool move_one(const ReactParams& R, const Snapshot<Po
 // workgroups share a CU (2 waves per SIMD); their registers are capped at
 // what two waves per SIMD allow (256), the rest spilling to scratch, which
 // measured ~10 % faster than the uncapped one-wave form.
-template <typename PosT, int kPoolN>
+template <typename PosT, int kPoolN, class TeamT>
 __global__ __launch_bounds__(256, 2) void k_move(ReactParams R, Snapshot<PosT> S, RMolView<PosT> src,
                                               RMolView<PosT> out, const uint32_t* __restrict__ list,
                                               const uint32_t* __restrict__ count,
@@ -330,18 +339,17 @@ __global__ __launch_bounds__(256, 2) void k_move(ReactParams R, Snapshot<PosT> S
   __shared__ ZigguratTables T;
   __shared__ uint32_t sets[SubpartSet::kCap * 256];
   const uint32_t n = *count;
-  if ((uint64_t)blockIdx.x * blockDim.x >= n) return;  // (uniform per block)
+  const Spread<TeamT> W(n);
+  if (W.block_first >= n) return;
   stage_zig(T);
   uint32_t n_reflect = 0, n_cross = 0;
-  // grid-stride: the launch is sized by a host bound on the count, so a
-  // small grid walks a list whose actual length is known only on the device
-  for (uint32_t b = blockIdx.x * blockDim.x; b < n; b += gridDim.x * blockDim.x) {
-    const uint32_t q = b + threadIdx.x;
+  for (uint32_t b = W.wave_first; b < n; b += W.stride) {
+    const uint32_t q = W.at(b);
     bool proposed = false, due = false, deferred = false;
     uint32_t j = 0;
     if (q < n) {
       j = list ? list[q] : q;
-      proposed = move_one<PosT, kPoolN>(R, S, src, out, j, species, T, barrier, propose_only, prop, owner,
+      proposed = move_one<PosT, kPoolN>(W.team, R, S, src, out, j, species, T, barrier, propose_only, prop, owner,
                                         tile_owner, err_out, due, deferred, sets + threadIdx.x, n_reflect, n_cross);
     }
     append_slot(proposed, j, plist, pcount);
@@ -355,7 +363,7 @@ __global__ __launch_bounds__(256, 2) void k_move(ReactParams R, Snapshot<PosT> S
 // The full step for every queued mover (the shards read as one list,
 // grid-stride; consecutive threads take consecutive slots of a shard, which
 // came from neighbouring cells).
-template <typename PosT, int kPoolN>
+template <typename PosT, int kPoolN, class TeamT>
 __global__ __launch_bounds__(256, 2) void k_move_drain(ReactParams R, Snapshot<PosT> S, RMolView<PosT> src,
                                                     RMolView<PosT> out, SlowQueue Q, SpeciesTable species, double barrier,
                                                     uint32_t propose_only, Proposal* __restrict__ prop,
@@ -367,18 +375,19 @@ __global__ __launch_bounds__(256, 2) void k_move_drain(ReactParams R, Snapshot<P
   __shared__ ZigguratTables T;
   __shared__ uint32_t sets[SubpartSet::kCap * 256];
   __shared__ uint32_t pre[kQueueShards + 1];
-  __shared__ uint32_t part[256];
+  __shared__ uint32_t part[4];
   const uint32_t total = queue_prefix(Q.count, Q.nshards, pre, part);
-  if ((uint64_t)blockIdx.x * blockDim.x >= total) return;
+  const Spread<TeamT> W(total);
+  if (W.block_first >= total) return;
   stage_zig(T);
   uint32_t n_reflect = 0, n_cross = 0;
-  for (uint32_t base = blockIdx.x * blockDim.x; base < total; base += gridDim.x * blockDim.x) {
-    const uint32_t q = base + threadIdx.x;
+  for (uint32_t base = W.wave_first; base < total; base += W.stride) {
+    const uint32_t q = W.at(base);
     bool proposed = false, due = false, deferred = false;
     uint32_t j = 0;
     if (q < total) {
       j = queue_at(Q.slots, Q.shard_cap, pre, q);
-      proposed = move_one<PosT, kPoolN>(R, S, src, out, j, species, T, barrier, propose_only, prop, owner,
+      proposed = move_one<PosT, kPoolN>(W.team, R, S, src, out, j, species, T, barrier, propose_only, prop, owner,
                                         tile_owner, err_out, due, deferred, sets + threadIdx.x, n_reflect, n_cross);
     }
     append_slot(proposed, j, plist, pcount);
@@ -432,7 +441,7 @@ __global__ __launch_bounds__(256, 4) void k_move_light(ReactParams R, Snapshot<P
     if (!ready_this_iteration(R.iteration, toff)) {
       // scheduled for a later iteration (Partition::get_molecules_ready_for_
       // diffusion, partition.h:232-246): stays where it is
-      store_pos(R, out.x, out.y, out.z, j, pos, false);
+      store_pos(Solo{}, R, out.x, out.y, out.z, j, pos, false);
       out.id[j] = idv;
       out.tag[j] = store_toff(out.toff, j, toff_past_iteration(R.iteration, toff), tag);
       if (out.utime) out.utime[j] = utime;
@@ -584,7 +593,7 @@ __global__ __launch_bounds__(256, 4) void k_move_light(ReactParams R, Snapshot<P
       }
       if (clear) {
         // an end point next to a wall plane keeps its side in FP32
-        err |= store_pos(R, out.x, out.y, out.z, j, end, near_plane);
+        err |= store_pos(Solo{}, R, out.x, out.y, out.z, j, end, near_plane);
         out.id[j] = idv;
         out.tag[j] = store_toff(out.toff, j, next_toff(R.iteration, toff, t_steps), tag & ~(MF_STEP_FLAGS << 8));
         if (out.utime) out.utime[j] = utime;
@@ -595,7 +604,7 @@ __global__ __launch_bounds__(256, 4) void k_move_light(ReactParams R, Snapshot<P
         partner_hard = walls_clear;
       }
     } else {
-      store_pos(R, out.x, out.y, out.z, j, pos, false);
+      store_pos(Solo{}, R, out.x, out.y, out.z, j, pos, false);
       out.id[j] = idv;
       out.tag[j] = store_toff(out.toff, j, immobile_toff(R.iteration, utime), tag & ~(MF_STEP_FLAGS << 8));
       if (out.utime) out.utime[j] = utime;
@@ -933,7 +942,7 @@ __global__ __launch_bounds__(256) void k_products(ReactParams R, const uint32_t*
       aux.init(R.seed, id, R.iteration, rep, kAuxPass);
       uint32_t e2 = 0;
       const D3 vp = volume_product_position(R, D3{p.x, p.y, p.z}, wall, o, aux, e2);
-      if (store_pos(R, out.x, out.y, out.z, slot, vp, true)) e2 |= ERR_ROUND32;
+      if (store_pos(Solo{}, R, out.x, out.y, out.z, slot, vp, true)) e2 |= ERR_ROUND32;
       if (e2) atomicOr(err, e2);
       out.id[slot] = id;
       out.tag[slot] = store_toff(out.toff, slot, p.time - (double)(R.iteration + (moves_now ? 0u : 1u)),
@@ -981,7 +990,7 @@ __global__ __launch_bounds__(256) void k_products(ReactParams R, const uint32_t*
       atomicOr(err, ERR_QUEUE);
       break;
     }
-    if (store_pos(R, out.x, out.y, out.z, slot, D3{p.x, p.y, p.z}, true)) atomicOr(err, ERR_ROUND32);
+    if (store_pos(Solo{}, R, out.x, out.y, out.z, slot, D3{p.x, p.y, p.z}, true)) atomicOr(err, ERR_ROUND32);
     out.id[slot] = first_id + i;
     out.tag[slot] = store_toff(out.toff, slot, p.time - (double)(R.iteration + (moves_now ? 0u : 1u)),
                                make_tag(prods[i], MF_SCHEDULE_UNIMOL, rep));
@@ -1121,11 +1130,15 @@ __global__ __launch_bounds__(256) void k_count_tiles(const uint32_t* __restrict_
 
 // --------------------------------------------------------------- launchers --
 static inline dim3 blocks_for(uint32_t n) { return dim3((n + 255) / 256 > 0 ? (n + 255) / 256 : 1); }
-// The full-step list kernel walks its list grid-stride: at most two
-// workgroups per CU fit (its LDS), and every workgroup launched beyond the
-// list's actual length (a device count under a host bound) still costs a
-// workgroup launch.
-static inline dim3 move_grid(uint32_t max_movers) { return dim3(std::min<uint32_t>(blocks_for(max_movers).x, 512u)); }
+// The full-step kernels walk their list grid-stride: at most two workgroups
+// per CU fit (their LDS), and every workgroup launched beyond the list's
+// actual length (a device count under a host bound) still costs a workgroup
+// launch.
+// A wave takes as few movers as the grid's waves allow (Spread), so the grid
+// is what the chip holds at once, two workgroups per CU: 1024 and 2048
+// workgroups, each with its share of set-up, measured 3-10 % slower on lists
+// of hundreds to thousands of movers.
+static inline dim3 move_grid(uint32_t max_movers) { return dim3(std::min<uint32_t>((max_movers + 3) / 4, 512u)); }
 
 template <typename PosT>
 hipError_t ReactPipeline<PosT>::sort(hipStream_t s, uint32_t n_in, uint32_t num_cells, uint32_t* err) {
@@ -1180,31 +1193,38 @@ hipError_t ReactPipeline<PosT>::move(hipStream_t s, bool snapshot_src, const uin
   // read next
   uint32_t* const xlist = (list == nullptr) ? mlist : (list == rlist0 ? rlist1 : rlist0);
   const RMolView<PosT> src = snapshot_src ? Sm : M;
+  SlowQueue Q = queue;
   if (list == nullptr && snapshot_src) {
     // every snapshot slot: light pass, then the queued movers in full
-    SlowQueue Q = queue;
     Q.shard_cap = shard_capacity(max_movers, kQueueShards / 2);
     hipLaunchKernelGGL(k_fill_u32, dim3(kQueueShards / 256), dim3(256), 0, s, Q.count, 0u, kQueueShards);
     hipLaunchKernelGGL(k_move_light<PosT>, blocks_for(max_movers), dim3(256), 0, s, R, S, M, count, species, barrier,
                        Q, err);
     Q.nshards = kQueueShards / 2 + std::min<uint32_t>(kQueueShards / 2, blocks_for(max_movers).x);
-    if (drain_inline)
-      hipLaunchKernelGGL((k_move_drain<PosT, kDrainPool>), dim3(Q.nshards), dim3(256), 0, s, R, S, Sm, M, Q, species,
-                         barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err, ulist,
+  } else {
+    Q.nshards = 0;
+  }
+  const auto full_steps = [&](auto team) {
+    using TeamT = decltype(team);
+    if (Q.nshards && drain_inline)
+      hipLaunchKernelGGL((k_move_drain<PosT, kDrainPool, TeamT>), move_grid(max_movers), dim3(256), 0, s, R, S, Sm, M,
+                         Q, species, barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err, ulist,
+                         hdr + kHdrUnimolDue, xlist, hdr + kHdrExd);
+    else if (Q.nshards)
+      hipLaunchKernelGGL((k_move_drain<PosT, 0, TeamT>), move_grid(max_movers), dim3(256), 0, s, R, S, Sm, M, Q,
+                         species, barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err, ulist,
                          hdr + kHdrUnimolDue, xlist, hdr + kHdrExd);
     else
-      hipLaunchKernelGGL((k_move_drain<PosT, 0>), dim3(Q.nshards), dim3(256), 0, s, R, S, Sm, M, Q, species, barrier,
-                         po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err, ulist, hdr + kHdrUnimolDue,
-                         xlist, hdr + kHdrExd);
-  } else {
-    hipLaunchKernelGGL((k_move<PosT, kListPool>), move_grid(max_movers), dim3(256), 0, s, R, S, src, M, list, count,
-                       species, barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err, ulist,
-                       hdr + kHdrUnimolDue, xlist, hdr + kHdrExd);
-  }
-  // the deferred steps, with the large pool
-  hipLaunchKernelGGL((k_move<PosT, exd::kPool>), move_grid(max_movers), dim3(256), 0, s, R, S, src, M, xlist,
-                     hdr + kHdrExd, species, barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err,
-                     ulist, hdr + kHdrUnimolDue, nullptr, nullptr);
+      hipLaunchKernelGGL((k_move<PosT, kListPool, TeamT>), move_grid(max_movers), dim3(256), 0, s, R, S, src, M, list,
+                         count, species, barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err, ulist,
+                         hdr + kHdrUnimolDue, xlist, hdr + kHdrExd);
+    // the deferred steps, with the large pool
+    hipLaunchKernelGGL((k_move<PosT, exd::kPool, TeamT>), move_grid(max_movers), dim3(256), 0, s, R, S, src, M, xlist,
+                       hdr + kHdrExd, species, barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err,
+                       ulist, hdr + kHdrUnimolDue, nullptr, nullptr);
+  };
+  if (teams) full_steps(Team{1, 0});
+  else full_steps(Solo{});
   return hipGetLastError();
 }
 
