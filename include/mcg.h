@@ -406,6 +406,14 @@ int mcg_set_next_molecule_ids(mcg_ctx* ctx, const uint32_t* next_ids);
 int mcg_step(mcg_ctx* ctx, uint32_t first_iteration, uint32_t num_iterations, double time_up_to_next_barrier,
              mcg_step_stats* stats);
 
+/* *matter: 0 while no step of the context depends on the time up to the next
+ * barrier (no reaction classes, every species moves with the global time
+ * step, every molecule due at the clock): a step then always spans one
+ * iteration, and one mcg_step call may cover a stretch with barriers in it
+ * at which the caller has nothing to do (its time_up_to_next_barrier the
+ * whole stretch), with the results of single calls.  1 otherwise. */
+int mcg_barriers_matter(mcg_ctx* ctx, uint32_t* matter);
+
 /* Waits for all queued work. */
 int mcg_sync(mcg_ctx* ctx);
 

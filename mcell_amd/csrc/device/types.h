@@ -130,7 +130,9 @@ enum : uint32_t {
 
 // per-call statistics counters (SimulationStats::mol_wall_reflections and
 // the transparent crossings), one wave-summed atomic per wave
-enum : uint32_t { CTR_REFLECTIONS = 0, CTR_CROSSINGS = 1, CTR_WORDS = 2 };
+// (CTR_LAST_TRACED: full ray traces of the last iteration of a run of
+// iterations, free diffusion only)
+enum : uint32_t { CTR_REFLECTIONS = 0, CTR_CROSSINGS = 1, CTR_LAST_TRACED = 2, CTR_WORDS = 3 };
 __device__ __forceinline__ void wave_count(unsigned long long* ctr, uint32_t v) {
   if (ctr == nullptr) return;
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);

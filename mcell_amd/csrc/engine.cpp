@@ -5,6 +5,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -398,25 +399,41 @@ int free_step(mcg_ctx* c, uint32_t first_iteration, uint32_t num_iterations, mcg
   HIP_TRY(hipEventRecord(c->ev0, c->stream));
   // every molecule has its diffusion time at the iteration start and the
   // species time step 1, so the barrier (>= 1 ahead) never clips a step
-  for (uint32_t k = 0; k < num_iterations; ++k) {
-    if (c->fp32())
+  const bool run = !tr.enabled && run_pays(n);
+  // launches of some 2.7e8 steps: about ten milliseconds each
+  const uint32_t per_launch = run ? (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(4096, (1ull << 28) / std::max(n, 1u))) : 1u;
+  uint32_t launches = 0;
+  for (uint32_t k = 0; k < num_iterations; k += per_launch, launches += run ? 1 : 3) {
+    const uint32_t first = first_iteration + k, num = std::min(per_launch, num_iterations - k);
+    if (run) {
+      if (k) HIP_TRY(launch_fill_u64(c->stream, c->counters.p + CTR_LAST_TRACED, 0ull, 1));
+      if (c->fp32())
+        HIP_TRY(launch_run32(c->stream, mf, n, c->species_table(), c->surface_classes(), c->P, W, c->walls32.p,
+                             c->max_abs_coord, c->cfg.seed, first, num, c->err.p, c->counters.p));
+      else
+        HIP_TRY(launch_run64(c->stream, m, n, c->species_table(), c->surface_classes(), c->P, W, c->cfg.seed, first,
+                             num, c->err.p, c->counters.p));
+    } else if (c->fp32()) {
       HIP_TRY(launch_diffuse_reflect32(c->stream, mf, n, c->species_table(), c->surface_classes(), c->P, W,
-                                       c->walls32.p, c->max_abs_coord, c->cfg.seed, first_iteration + k, MQ, Q,
-                                       c->err.p, tr, c->counters.p));
-    else
+                                       c->walls32.p, c->max_abs_coord, c->cfg.seed, first, MQ, Q, c->err.p, tr,
+                                       c->counters.p));
+    } else {
       HIP_TRY(launch_diffuse_reflect64(c->stream, m, n, c->species_table(), c->surface_classes(), c->P, W,
-                                       c->cfg.seed, first_iteration + k, MQ, Q, c->err.p, tr, c->counters.p));
+                                       c->cfg.seed, first, MQ, Q, c->err.p, tr, c->counters.p));
+    }
   }
   HIP_TRY(hipEventRecord(c->ev1, c->stream));
   uint32_t err = 0, slow = 0;
-  unsigned long long ctr[CTR_WORDS] = {0, 0};
-  std::vector<uint32_t> shard_counts(kNumQueueShards, 0);
+  unsigned long long ctr[CTR_WORDS] = {};
+  std::vector<uint32_t> shard_counts;
   HIP_TRY(hipMemcpyAsync(&err, c->err.p, 4, hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipMemcpyAsync(ctr, c->counters.p, sizeof(ctr), hipMemcpyDeviceToHost, c->stream));
-  if (num_iterations && n)
+  if (num_iterations && n && !run) {
+    shard_counts.resize(kNumQueueShards);
     HIP_TRY(hipMemcpyAsync(shard_counts.data(), c->qcount.p, kNumQueueShards * 4, hipMemcpyDeviceToHost, c->stream));
+  }
   HIP_TRY(hipStreamSynchronize(c->stream));
-  for (uint32_t v : shard_counts) slow += v;
+  slow = run ? (uint32_t)ctr[CTR_LAST_TRACED] : std::accumulate(shard_counts.begin(), shard_counts.end(), 0u);
   float ms = 0;
   HIP_TRY(hipEventElapsedTime(&ms, c->ev0, c->ev1));
   c->last_kernel_ms = num_iterations ? ms / num_iterations : 0;
@@ -428,7 +445,7 @@ int free_step(mcg_ctx* c, uint32_t first_iteration, uint32_t num_iterations, mcg
     stats->reactions = 0;
     stats->kernel_ms = ms;
     stats->wall_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-    stats->kernel_launches = 3 * num_iterations;
+    stats->kernel_launches = launches;
     stats->slow_path_last = slow;
   }
   if (err) {
@@ -467,6 +484,13 @@ int mcg_step(mcg_ctx* c, uint32_t first_iteration, uint32_t num_iterations, doub
                     : free_step(c, first_iteration, num_iterations, stats);
   if (st == MCG_OK) c->clock = (uint64_t)first_iteration + num_iterations;
   return step_failed(c, st);
+}
+
+int mcg_barriers_matter(mcg_ctx* c, uint32_t* matter) {
+  if (!c || !matter) return fail(MCG_E_INVALID, "null argument");
+  MCG_ALIVE(c);
+  *matter = (c->rx.on || c->custom_steps() || (c->surface_diffusion() && c->rx.total_tiles)) ? 1u : 0u;
+  return MCG_OK;
 }
 
 int mcg_set_surface_classes(mcg_ctx* c, uint32_t num_classes, const uint8_t* action) {

@@ -287,7 +287,7 @@ int run_iterations(mcg_ctx* c, ReactPipeline<PosT>& p, uint32_t first, uint32_t 
   }
   if (propose_only) r.log_count = h[kHdrLog];
   if (stats) {
-    unsigned long long ctr[CTR_WORDS] = {0, 0};
+    unsigned long long ctr[CTR_WORDS] = {};
     HIP_TRY(hipMemcpy(ctr, c->counters.p, sizeof(ctr), hipMemcpyDeviceToHost));
     stats->molecule_steps = steps;
     stats->reactions = reactions;

@@ -62,6 +62,18 @@ hipError_t launch_diffuse_reflect32(hipStream_t s, const MolView32& m, uint32_t 
                                     float max_abs_coord, uint64_t seed, uint32_t iteration, SlowQueue MQ,
                                     SlowQueue Q, uint32_t* err, const HitTrace& trace, unsigned long long* ctr);
 
+// Iterations first .. first + num - 1 of every molecule in one launch
+// (molecules that react with nothing); CTR_LAST_TRACED gets the molecules
+// whose last step took the full ray trace.  run_pays: whether that is faster
+// than the passes of single iterations for n molecules.
+bool run_pays(uint32_t n);
+hipError_t launch_run64(hipStream_t s, const MolView64& m, uint32_t n, SpeciesTable species, const SurfaceClasses& SC,
+                        const PartitionParams& P, const WallView64& W, uint64_t seed, uint32_t first, uint32_t num,
+                        uint32_t* err, unsigned long long* ctr);
+hipError_t launch_run32(hipStream_t s, const MolView32& m, uint32_t n, SpeciesTable species, const SurfaceClasses& SC,
+                        const PartitionParams& P, const WallView64& W, const WallRec32* w32, float max_abs_coord,
+                        uint64_t seed, uint32_t first, uint32_t num, uint32_t* err, unsigned long long* ctr);
+
 hipError_t launch_copy(hipStream_t s, const void* src, void* dst, size_t bytes);
 
 }  // namespace mcg

@@ -89,6 +89,40 @@ __device__ __forceinline__ bool clear_move64(const PartitionParams32& Q, const W
                      [&](uint32_t k) { return wall_certain_miss64(W.ent[k], pos, disp); });
 }
 
+// One molecule's step on the light path: whether it commits (pos moved), or
+// who takes it: its displacement is off the Ziggurat's fast path (the full
+// draw decides), or a wall may stop it (the full ray trace).
+enum : uint32_t { kStepDone = 0, kStepMid = 1, kStepHard = 2 };
+
+__device__ __forceinline__ uint32_t light_step64(const FastZiggurat& T, const PartitionParams32& Q,
+                                                 const WallView64& W, uint64_t seed, uint32_t id, uint32_t iteration,
+                                                 uint32_t replica, double space_step, D3& pos) {
+  uint32_t r0, r1, r2, r3;
+  philox_block0(seed, id, iteration, replica, 0, r0, r1, r2, r3);
+  D3 disp;
+  if (!fast_displacement(r0, r1, r2, T, space_step, disp.x, disp.y, disp.z)) return kStepMid;
+  const D3 end = {pos.x + disp.x, pos.y + disp.y, pos.z + disp.z};
+  if (!clear_move64(Q, W, pos, disp, end)) return kStepHard;
+  pos = end;
+  return kStepDone;
+}
+
+struct F3 {
+  float x, y, z;
+};
+__device__ __forceinline__ uint32_t light_step32(const FastZiggurat& T, const PartitionParams32& Q,
+                                                 const Walls32View& W, const FilterParams& F, float band,
+                                                 uint64_t seed, uint32_t id, uint32_t iteration, uint32_t replica,
+                                                 double space_step, F3& pos) {
+  uint32_t r0, r1, r2, r3;
+  philox_block0(seed, id, iteration, replica, 0, r0, r1, r2, r3);
+  float mx, my, mz;
+  if (!fast_displacement32(r0, r1, r2, T, (float)(space_step * 0.70710678118654752440), mx, my, mz)) return kStepMid;
+  if (!clear_move32(Q, W, F, band, pos.x, pos.y, pos.z, mx, my, mz)) return kStepHard;
+  pos = {pos.x + mx, pos.y + my, pos.z + mz};
+  return kStepDone;
+}
+
 // ------------------------------------------------------------------- FP64 --
 // Every molecule whose three Gaussians are on the Ziggurat's fast path and
 // whose straight move certainly meets no wall (FP64 collide_wall of every
@@ -108,20 +142,16 @@ __global__ __launch_bounds__(256) void k_light64(MolView64 m, uint32_t n, Specie
       const D3 pos = {m.x[i], m.y[i], m.z[i]};
       const SpeciesRec sp = species.of(tag);
       if (!(tag_flags(tag) & MF_DEFUNCT) && sp.space_step > 0) {
-        uint32_t r0, r1, r2, r3;
-        philox_block0(seed, idv, iteration, tag_replica(tag), 0, r0, r1, r2, r3);
-        D3 disp;
-        mid = !fast_displacement(r0, r1, r2, T, sp.space_step, disp.x, disp.y, disp.z);
-        bool clear = !mid;
-        const D3 end = {pos.x + disp.x, pos.y + disp.y, pos.z + disp.z};
-        clear = clear && clear_move64(Q, W, pos, disp, end);
-        if (clear) {
-          m.x[i] = end.x;
-          m.y[i] = end.y;
-          m.z[i] = end.z;
+        D3 at = pos;
+        const uint32_t r = light_step64(T, Q, W, seed, idv, iteration, tag_replica(tag), sp.space_step, at);
+        if (r == kStepDone) {
+          m.x[i] = at.x;
+          m.y[i] = at.y;
+          m.z[i] = at.z;
           if (trace.enabled) trace.count[i] = 0;
         }
-        hard = !clear && !mid;
+        mid = r == kStepMid;
+        hard = r == kStepHard;
       }
     }
     append_light(mid, hard, i, tile, MQ, HQ);
@@ -222,18 +252,16 @@ __global__ __launch_bounds__(256) void k_light32(MolView32 m, uint32_t n, Specie
       const float px = m.x[i], py = m.y[i], pz = m.z[i];
       const SpeciesRec sp = species.of(tag);
       if (!(tag_flags(tag) & MF_DEFUNCT) && sp.space_step > 0) {
-        uint32_t r0, r1, r2, r3;
-        philox_block0(seed, idv, iteration, tag_replica(tag), 0, r0, r1, r2, r3);
-        float mx, my, mz;
-        mid = !fast_displacement32(r0, r1, r2, T, (float)(sp.space_step * 0.70710678118654752440), mx, my, mz);
-        const bool clear = !mid && clear_move32(Q, W, F, band, px, py, pz, mx, my, mz);
-        if (clear) {
-          m.x[i] = px + mx;
-          m.y[i] = py + my;
-          m.z[i] = pz + mz;
+        F3 at = {px, py, pz};
+        const uint32_t r = light_step32(T, Q, W, F, band, seed, idv, iteration, tag_replica(tag), sp.space_step, at);
+        if (r == kStepDone) {
+          m.x[i] = at.x;
+          m.y[i] = at.y;
+          m.z[i] = at.z;
           if (trace.enabled) trace.count[i] = 0;
         }
-        hard = !clear && !mid;
+        mid = r == kStepMid;
+        hard = r == kStepHard;
       }
     }
     append_light(mid, hard, i, tile, MQ, HQ);
@@ -323,6 +351,145 @@ __global__ __launch_bounds__(256) void k_hard32(MolView32 m, SpeciesTable specie
   wave_count(ctr + CTR_CROSSINGS, n_cross);
 }
 
+// ------------------------------------------------- several iterations at once --
+// Molecules that react with nothing do not see each other, so a wave keeps
+// up to 64 molecules in registers and takes them through all iterations of
+// the call: memory is read and written once per call, and no launch, queue or
+// synchronisation lies between two steps.  Every lane counts its own
+// iterations.  Steps off the light path wait until half of the wave's
+// unfinished lanes wait for one, and are then taken together: a full step's
+// chain costs the wave many light steps however many lanes take it, and
+// about one step in ten needs one.  Few molecules are spread over all the
+// waves the chip holds (kRunWaves; 223 registers, two waves per SIMD): a
+// wave's chains are then shorter and fewer.  Same steps, same order per
+// molecule: the results equal those of single iterations bit for bit.
+// Bound by the chains' latency; 10,000 molecules in a box take 11 us an
+// iteration in calls of 64 (the three passes: 80), 262,144 take 42 (100).
+struct FreeForm64 {
+  using Pos = D3;
+  MolView64 m;
+  WallView64 W;
+  __device__ __forceinline__ Pos load(uint32_t i) const { return {m.x[i], m.y[i], m.z[i]}; }
+  __device__ __forceinline__ void store(uint32_t i, const Pos& p) const {
+    m.x[i] = p.x;
+    m.y[i] = p.y;
+    m.z[i] = p.z;
+  }
+  __device__ __forceinline__ uint32_t light(const FastZiggurat& T, const PartitionParams32& Q, uint64_t seed,
+                                            uint32_t id, uint32_t it, uint32_t rep, double step, Pos& p) const {
+    return light_step64(T, Q, W, seed, id, it, rep, step, p);
+  }
+  // the move of a full draw, if it certainly meets no wall
+  __device__ __forceinline__ bool clear(const PartitionParams32& Q, const D3& disp, Pos& p) const {
+    const D3 end = {p.x + disp.x, p.y + disp.y, p.z + disp.z};
+    if (!clear_move64(Q, W, p, disp, end)) return false;
+    p = end;
+    return true;
+  }
+  __device__ __forceinline__ bool trace(const PartitionParams& P, const SurfaceClasses& SC, uint32_t species,
+                                        const D3& disp, PhiloxStream& rng, Pos& p, uint32_t& err, uint32_t& n_reflect,
+                                        uint32_t& n_cross) const {
+    uint32_t tn = 0;
+    return diffuse_reflect64(P, W.walls, W.off, W.idx, W.box, SC, species, p, disp, rng, err, nullptr, tn, n_reflect,
+                             n_cross);
+  }
+};
+
+struct FreeForm32 {
+  using Pos = F3;
+  MolView32 m;
+  Walls32View W;
+  FilterParams F;
+  float band;
+  __device__ __forceinline__ Pos load(uint32_t i) const { return {m.x[i], m.y[i], m.z[i]}; }
+  __device__ __forceinline__ void store(uint32_t i, const Pos& p) const {
+    m.x[i] = p.x;
+    m.y[i] = p.y;
+    m.z[i] = p.z;
+  }
+  __device__ __forceinline__ uint32_t light(const FastZiggurat& T, const PartitionParams32& Q, uint64_t seed,
+                                            uint32_t id, uint32_t it, uint32_t rep, double step, Pos& p) const {
+    return light_step32(T, Q, W, F, band, seed, id, it, rep, step, p);
+  }
+  __device__ __forceinline__ bool clear(const PartitionParams32& Q, const D3& disp, Pos& p) const {
+    const float mx = (float)disp.x, my = (float)disp.y, mz = (float)disp.z;
+    if (!clear_move32(Q, W, F, band, p.x, p.y, p.z, mx, my, mz)) return false;
+    p = {p.x + mx, p.y + my, p.z + mz};
+    return true;
+  }
+  __device__ __forceinline__ bool trace(const PartitionParams& P, const SurfaceClasses& SC, uint32_t species,
+                                        const D3& disp, PhiloxStream& rng, Pos& p, uint32_t& err, uint32_t& n_reflect,
+                                        uint32_t& n_cross) const {
+    uint32_t tn = 0;
+    D3 q = {(double)p.x, (double)p.y, (double)p.z};
+    const bool alive = diffuse_reflect64(P, W.w64, W.off, W.idx, W.box, SC, species, q, disp, rng, err, nullptr, tn,
+                                         n_reflect, n_cross);
+    if (!round_to_fp32_same_side(Solo{}, P, W.w64, W.off, W.idx, W.box, q.x, q.y, q.z, &p.x, &p.y, &p.z))
+      err |= ERR_ROUND32;
+    return alive;
+  }
+};
+
+template <class Form>
+__global__ __launch_bounds__(64, 2) void k_run(Form S, uint32_t n, uint32_t per_wave, SpeciesTable species,
+                                               SurfaceClasses SC, PartitionParams P, PartitionParams32 Q,
+                                               uint64_t seed, uint32_t first, uint32_t num, uint32_t* __restrict__ err_out,
+                                               unsigned long long* __restrict__ ctr) {
+  __shared__ FastZiggurat F;
+  __shared__ ZigguratTables T;
+  stage_fast_ziggurat(F, c_zig);
+  stage_ziggurat(T);
+  const uint32_t i = blockIdx.x * per_wave + threadIdx.x;
+  uint32_t tag = 0, id = 0, it = num;
+  typename Form::Pos pos = {0, 0, 0};
+  double step = 0;
+  if (threadIdx.x < per_wave && i < n) {
+    tag = S.m.tag[i];
+    id = S.m.id[i];
+    pos = S.load(i);
+    step = species.of(tag).space_step;
+    if (!(tag_flags(tag) & MF_DEFUNCT) && step > 0) it = 0;
+  }
+  const bool moves = it == 0 && num > 0;
+  const uint32_t rep = tag_replica(tag);
+  uint32_t wait = kStepDone, err = 0, n_reflect = 0, n_cross = 0, n_last = 0;
+  for (;;) {
+    for (;;) {
+      const bool go = it < num && wait == kStepDone;
+      const uint32_t going = (uint32_t)__popcll(__ballot(go));
+      const uint32_t waiting = (uint32_t)__popcll(__ballot(wait != kStepDone));
+      if (going <= waiting) break;  // (also when none goes)
+      if (go) {
+        wait = S.light(F, Q, seed, id, first + it, rep, step, pos);
+        if (wait == kStepDone) ++it;
+      }
+    }
+    if (__ballot(wait != kStepDone) == 0) break;  // every lane is through
+    if (wait != kStepDone) {
+      PhiloxStream rng;
+      rng.init(seed, id, first + it, rep, 0);
+      const D3 disp = draw_displacement(rng, T, step);
+      bool alive = true;
+      if (!(wait == kStepMid && S.clear(Q, disp, pos))) {
+        if (it + 1 == num) ++n_last;
+        alive = S.trace(P, SC, tag_species(tag), disp, rng, pos, err, n_reflect, n_cross);
+      }
+      if (!alive) {
+        S.m.tag[i] = tag | (MF_DEFUNCT << 8);
+        it = num;
+      } else {
+        ++it;
+      }
+      wait = kStepDone;
+    }
+  }
+  if (moves) S.store(i, pos);
+  if (err) atomicOr(err_out, err);
+  wave_count(ctr + CTR_REFLECTIONS, n_reflect);
+  wave_count(ctr + CTR_CROSSINGS, n_cross);
+  wave_count(ctr + CTR_LAST_TRACED, n_last);
+}
+
 // Copy kernel of known size (device-to-device bandwidth reference).
 __global__ __launch_bounds__(256) void k_copy(const float4* __restrict__ src, float4* __restrict__ dst, size_t n) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -359,6 +526,41 @@ uint32_t shard_capacity(uint32_t n, uint32_t shards) {
   return 256u * ((blocks + shards - 1) / shards);
 }
 
+
+constexpr uint32_t kRunWaves = 2048;  // waves of k_run the chip holds (256 CUs x 4 SIMDs x 2)
+static inline uint32_t run_per_wave(uint32_t n) {
+  return std::max<uint32_t>(1u, std::min<uint32_t>(64u, (n + kRunWaves - 1) / kRunWaves));
+}
+
+// Two turns of the waves the chip holds.  Above, the three passes' full
+// waves win: at 10^6 molecules 141 us an iteration against 132 in calls of
+// 64 iterations and 422 against 218 in single ones, at 3 * 10^5 53 against
+// 101 and 179 against 192.
+bool run_pays(uint32_t n) { return n <= 2u * 64u * kRunWaves; }
+
+hipError_t launch_run64(hipStream_t s, const MolView64& m, uint32_t n, SpeciesTable species, const SurfaceClasses& SC,
+                        const PartitionParams& P, const WallView64& W, uint64_t seed, uint32_t first, uint32_t num,
+                        uint32_t* err, unsigned long long* ctr) {
+  if (n == 0 || num == 0) return hipSuccess;
+  const uint32_t per = run_per_wave(n);
+  hipLaunchKernelGGL(k_run<FreeForm64>, dim3((n + per - 1) / per), dim3(64), 0, s, FreeForm64{m, W}, n, per, species, SC, P,
+                     make_partition32(P), seed, first, num, err, ctr);
+  return hipGetLastError();
+}
+
+hipError_t launch_run32(hipStream_t s, const MolView32& m, uint32_t n, SpeciesTable species, const SurfaceClasses& SC,
+                        const PartitionParams& P, const WallView64& W, const WallRec32* w32, float max_abs_coord,
+                        uint64_t seed, uint32_t first, uint32_t num, uint32_t* err, unsigned long long* ctr) {
+  if (n == 0 || num == 0) return hipSuccess;
+  const uint32_t per = run_per_wave(n);
+  const FilterParams F = make_filter_params(max_abs_coord, kMoveUlps);
+  const float band = 2.0f * F.e_dd + 8.0f * F.eps * max_abs_coord;
+  const Walls32View W32{W.walls, reinterpret_cast<const FilterWall*>(w32), W.off, W.idx,
+                        reinterpret_cast<const FilterWall*>(W.ent32), W.box};
+  hipLaunchKernelGGL(k_run<FreeForm32>, dim3((n + per - 1) / per), dim3(64), 0, s, FreeForm32{m, W32, F, band}, n, per, species,
+                     SC, P, make_partition32(P), seed, first, num, err, ctr);
+  return hipGetLastError();
+}
 
 hipError_t launch_diffuse_reflect64(hipStream_t s, const MolView64& m, uint32_t n, SpeciesTable species,
                                     const SurfaceClasses& SC,
