@@ -34,8 +34,6 @@ mcg_ctx::~mcg_ctx() {
   if (rx.hdr_host) (void)hipHostFree(rx.hdr_host);
   if (ev0) (void)hipEventDestroy(ev0);
   if (ev1) (void)hipEventDestroy(ev1);
-  if (evm0) (void)hipEventDestroy(evm0);
-  if (evm1) (void)hipEventDestroy(evm1);
   if (stream) (void)hipStreamDestroy(stream);
 }
 
@@ -118,9 +116,12 @@ int mcg_create(const mcg_config* cfg, mcg_ctx** out) {
   };
   hipError_t e;
   if ((e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) != hipSuccess ||
-      (e = hipEventCreate(&c->ev0)) != hipSuccess || (e = hipEventCreate(&c->ev1)) != hipSuccess ||
-      (e = hipEventCreate(&c->evm0)) != hipSuccess || (e = hipEventCreate(&c->evm1)) != hipSuccess)
+      (e = hipEventCreate(&c->ev0)) != hipSuccess || (e = hipEventCreate(&c->ev1)) != hipSuccess)
     return cleanup_fail(fail(MCG_E_HIP, std::string("stream/event creation: ") + hipGetErrorString(e)));
+  int dev = 0, khz = 0;
+  if (hipGetDevice(&dev) == hipSuccess &&
+      hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) == hipSuccess && khz > 0)
+    c->clock_khz = khz;
   size_t cap = cfg->molecule_capacity;
   bool pos_fail = c->fp32() ? (c->xf.alloc(cap) || c->yf.alloc(cap) || c->zf.alloc(cap))
                             : (c->x.alloc(cap) || c->y.alloc(cap) || c->z.alloc(cap));

@@ -101,7 +101,15 @@ struct ReactState {
   bool grid_dirty = true;
   std::vector<uint32_t> next_id_host;  // per replica: 1 + largest id seen
   bool next_id_dirty = true;
-  uint32_t* hdr_host = nullptr;        // pinned mirror of hdr
+  uint32_t* hdr_host = nullptr;        // pinned mirror of hdr, written by the kernels (kHdrSeq: the copy's number)
+  uint32_t* hdr_host_d = nullptr;      // its device address
+  uint32_t hdr_seq = 0;                // number of the last copy asked for
+  // launch sizes: what the last rounds of each kind led to expect ([0]: list
+  // moves, [1], [2]: an iteration's first moves by the drain's form), never
+  // what a kernel may do
+  static constexpr uint32_t kUnknown = 1u << 30;
+  uint32_t expect_props[3] = {kUnknown, kUnknown, kUnknown}, expect_deferred[3] = {kUnknown, kUnknown, kUnknown};
+  bool volume_products = false;        // some class makes volume molecules or keeps a unimolecular reactant
   // the drain's form (1 exact_disk in place, 2 deferred): fixed by a flag,
   // else timed on the first iterations after the geometry or the molecules
   // are set (0 while undecided; the trials alternate the forms)
@@ -151,7 +159,8 @@ struct mcg_ctx {
   mcg_config cfg{};
   mcg::PartitionParams P{};
   hipStream_t stream = nullptr;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr, evm0 = nullptr, evm1 = nullptr;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  double clock_khz = 100000;  // the device's wall clock (wall_clock64)
 
   // geometry
   std::vector<mcg::WallRec64> walls_host;

@@ -130,15 +130,31 @@ ReactPipeline<PosT> make_pipeline(mcg_ctx* c, PosT* x, PosT* y, PosT* z, PosT* s
   p.head = r.head.p;
   p.next_id = r.next_id.p;
   p.hdr = r.hdr.p;
+  p.hdr_host = r.hdr_host_d;
   p.scan_tmp = r.scan_tmp.p;
   p.scan_tmp_bytes = r.scan_tmp.n;
   return p;
 }
 
-int read_hdr(mcg_ctx* c) {
-  HIP_TRY(hipMemcpyAsync(c->rx.hdr_host, c->rx.hdr.p, kHdrWords * 4, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  return MCG_OK;
+// Waits for the header's copy number c->rx.hdr_seq: the kernel that ends the
+// round writes it to host memory.  Polls (the wait is tens of microseconds,
+// which a stream synchronisation would add half again to), with a look at the
+// stream now and then: a copy that does not come although the stream is idle
+// or in error is an error.
+int wait_hdr(mcg_ctx* c) {
+  const uint32_t want = c->rx.hdr_seq;
+  const uint32_t* const seq = c->rx.hdr_host + kHdrSeq;
+  for (;;) {
+    for (int k = 0; k < 20000; ++k) {
+      if (__atomic_load_n(seq, __ATOMIC_ACQUIRE) == want) return MCG_OK;
+      __builtin_ia32_pause();
+    }
+    const hipError_t e = hipStreamQuery(c->stream);
+    if (e == hipErrorNotReady) continue;
+    if (e != hipSuccess) return fail(MCG_E_HIP, std::string("waiting for a round: ") + hipGetErrorString(e));
+    if (__atomic_load_n(seq, __ATOMIC_ACQUIRE) == want) return MCG_OK;
+    return fail(MCG_E_HIP, "a round ended without its counters");
+  }
 }
 
 // The drain's form for the next iteration: the flag's, the decided one, or
@@ -169,19 +185,24 @@ void drain_form_timed(ReactState& r, uint32_t form, float ms) {
 // read once per round, after the claims are settled.
 template <typename PosT>
 int settle_rounds(mcg_ctx* c, ReactPipeline<PosT>& p, bool snapshot_src, double barrier, uint32_t* err,
-                  uint32_t& rounds, uint32_t max_props) {
-  uint32_t* h = c->rx.hdr_host;
+                  uint32_t& rounds, uint32_t max_props, uint32_t form, bool timed) {
+  const uint32_t* const h = c->rx.hdr_host;
+  uint32_t kind = snapshot_src ? form : 0u;  // an iteration's first moves, or a list's
   for (uint32_t r = 0;; ++r) {
     if (r > 100000) return fail(MCG_E_LIMIT, "reaction settling did not converge");
     uint32_t* rl = (r & 1) ? p.rlist1 : p.rlist0;
     uint32_t* rc = p.hdr + ((r & 1) ? kHdrRerun1 : kHdrRerun0);
-    HIP_TRY(p.settle(c->stream, max_props, rl, rc));
-    int st = read_hdr(c);
-    if (st) return st;
+    p.expect_props = c->rx.expect_props[kind];
+    HIP_TRY(p.settle(c->stream, max_props, rl, rc, timed && r == 0, ++c->rx.hdr_seq));
+    if (int st = wait_hdr(c)) return st;
+    c->rx.expect_props[kind] = h[kHdrProposals];
+    c->rx.expect_deferred[kind] = h[kHdrExd];
+    kind = 0;
     if (h[kHdrProposals] == 0) return MCG_OK;
     ++rounds;
     const uint32_t nr = h[(r & 1) ? kHdrRerun1 : kHdrRerun0];
     if (nr == 0) return MCG_OK;
+    p.expect_deferred = c->rx.expect_deferred[0];
     HIP_TRY(p.move(c->stream, snapshot_src, rl, rc, nr, barrier, false, err));
     max_props = nr;
   }
@@ -191,10 +212,10 @@ template <typename PosT>
 int run_iterations(mcg_ctx* c, ReactPipeline<PosT>& p, uint32_t first, uint32_t num, double time_up,
                    mcg_step_stats* stats, double& move_ms) {
   ReactState& r = c->rx;
-  uint32_t* h = r.hdr_host;
+  const uint32_t* const h = r.hdr_host;
   const bool propose_only = (c->cfg.flags & MCG_FLAG_PROPOSE_ONLY) != 0;
   const uint64_t cap = c->cfg.molecule_capacity;
-  uint64_t reactions = 0, steps = 0;
+  uint64_t steps = 0;
   uint32_t rounds = 0;
   r.log_count = 0;
   HIP_TRY(launch_fill_u32(c->stream, p.hdr, 0u, kHdrWords));
@@ -211,68 +232,60 @@ int run_iterations(mcg_ctx* c, ReactPipeline<PosT>& p, uint32_t first, uint32_t 
     p.R.iteration = it;
     const uint32_t n_in = (uint32_t)c->n;
     HIP_TRY(p.sort(c->stream, n_in, r.num_cells, err));
-    HIP_TRY(launch_copy_u32(c->stream, p.cell_start + r.num_cells, p.hdr + kHdrNumOut));
-    HIP_TRY(launch_copy_u32(c->stream, p.cell_start + r.num_cells, p.hdr + kHdrSnapshot));
-    HIP_TRY(launch_fill_u32(c->stream, p.hdr + kHdrAccepted, 0u, 1u));
     const uint32_t form = drain_form_for(c);
     p.drain_inline = form == 1;
-    HIP_TRY(hipEventRecord(c->evm0, c->stream));
+    p.expect_deferred = r.expect_deferred[form];
     HIP_TRY(p.move(c->stream, true, nullptr, p.cell_start + r.num_cells, n_in, barrier, propose_only, err));
-    HIP_TRY(hipEventRecord(c->evm1, c->stream));
+    const bool timed = n_in != 0;
     if (propose_only) {
       HIP_TRY(p.log_proposals(c->stream, n_in, it, r.log.p, p.hdr + kHdrLog, (uint32_t)r.log_cap));
+      HIP_TRY(p.publish(c->stream, timed, ++r.hdr_seq));
+      if (int st = wait_hdr(c)) return st;
+      r.expect_deferred[form] = h[kHdrExd];
     } else {
       bool snapshot_src = true;
       uint32_t phase_movers = n_in;
       for (;;) {
-        int st = settle_rounds(c, p, snapshot_src, barrier, err, rounds, phase_movers);
-        if (st) return st;
-        if (h[kHdrUnimolDue]) {
-          HIP_TRY(p.fire_unimol(c->stream, h[kHdrUnimolDue]));
-          HIP_TRY(launch_fill_u32(c->stream, p.hdr + kHdrUnimolDue, 0u, 1u));
-          st = read_hdr(c);
-          if (st) return st;
-        }
-        // the next phase's movers: the products that move in this
-        // iteration, then the movers that diffuse again (the phase's moves
-        // are over, so the header's count of those is final)
-        const uint32_t na = h[kHdrAccepted], nc = h[kHdrContinue];
+        if (int st = settle_rounds(c, p, snapshot_src, barrier, err, rounds, phase_movers, form, timed && snapshot_src))
+          return st;
+        if (!snapshot_src) steps += h[kHdrProductMovers];
+        // the phase's reactions (at most: a due unimolecular event only
+        // happens to a molecule that is still there) and the movers that
+        // diffuse again in this iteration
+        const uint32_t due = h[kHdrUnimolDue], nc = h[kHdrContinue];
+        uint32_t na = h[kHdrAccepted] + due;
         if (na == 0 && nc == 0) break;
-        HIP_TRY(launch_fill_u32(c->stream, p.hdr + kHdrProductMovers, 0u, 1u));
-        if (na) {
-          reactions += na;
-          const uint64_t log_base = std::min<uint64_t>(r.log_count, 0xFFFFFFFFull);
-          HIP_TRY(p.products(c->stream, na, (uint32_t)cap, r.log.p, (uint32_t)log_base, (uint32_t)r.log_cap,
-                             snapshot_src, err));
-          r.log_count += na;
-          HIP_TRY(launch_fill_u32(c->stream, p.hdr + kHdrAccepted, 0u, 1u));
+        if (due) HIP_TRY(p.fire_unimol(c->stream, due));
+        if (na > kSmallBatch && due) {
+          // the sort of a large batch needs its exact length
+          HIP_TRY(p.publish(c->stream, false, ++r.hdr_seq));
+          if (int st = wait_hdr(c)) return st;
+          na = h[kHdrAccepted];
         }
-        HIP_TRY(p.continuations(c->stream, nc));
-        uint32_t nm = nc;
-        if (na) {
-          st = read_hdr(c);
-          if (st) return st;
-          nm = h[kHdrProductMovers];
+        HIP_TRY(p.products(c->stream, na, (uint32_t)cap, r.log.p, (uint32_t)r.log_cap, snapshot_src, err));
+        HIP_TRY(p.continuations(c->stream, nc, na != 0));
+        // the next phase's movers: the products that move in this iteration,
+        // then the movers that diffuse again (how many the device counts)
+        const uint64_t movers = nc + (r.volume_products ? (uint64_t)kMaxProducts * na : 0u);
+        if (movers == 0) {
+          HIP_TRY(p.publish(c->stream, false, ++r.hdr_seq));
+          if (int st = wait_hdr(c)) return st;
+          break;
         }
-        if (nm == 0) break;
         snapshot_src = false;
-        phase_movers = nm;
-        steps += nm;
-        HIP_TRY(p.move(c->stream, false, p.mlist, p.hdr + kHdrProductMovers, nm, barrier, false, err));
+        phase_movers = (uint32_t)std::min<uint64_t>(movers, cap);
+        p.expect_deferred = r.expect_deferred[0];
+        HIP_TRY(p.move(c->stream, false, p.mlist, p.hdr + kHdrProductMovers, phase_movers, barrier, false, err));
       }
       // the surface molecules' steps follow the volume phases
       if (r.surf_on)
         if (int st = surface_phase(c, it, barrier, err)) return st;
     }
-    // the settling loop ends on a header read; the proposal log does not
-    if (propose_only) {
-      int st = read_hdr(c);
-      if (st) return st;
-    }
-    float ms = 0;
-    HIP_TRY(hipEventElapsedTime(&ms, c->evm0, c->evm1));
-    move_ms += ms;
-    if (n_in) drain_form_timed(r, form, ms);
+    unsigned long long ticks;
+    std::memcpy(&ticks, h + kHdrMoveTicks, sizeof(ticks));
+    const double total_ms = (double)ticks / c->clock_khz;
+    if (n_in) drain_form_timed(r, form, (float)(total_ms - move_ms));
+    move_ms = total_ms;
     r.last_form = form;
     const uint32_t e = h[kHdrErr];
     if (e) {
@@ -281,11 +294,13 @@ int run_iterations(mcg_ctx* c, ReactPipeline<PosT>& p, uint32_t first, uint32_t 
       if (e & ERR_QUEUE) return fail(MCG_E_CAPACITY, "molecule capacity exceeded by reaction products");
       return fail(MCG_E_LIMIT, "per-step limit exceeded (error bits " + std::to_string(e) + ")");
     }
-    // k_bump_ids keeps the used slots within the capacity
+    // book_batch keeps the used slots within the capacity
     c->n = std::min<uint64_t>(h[kHdrNumOut], cap);
     steps += h[kHdrSnapshot];
   }
-  if (propose_only) r.log_count = h[kHdrLog];
+  const uint64_t reactions = num ? h[kHdrReacted] : 0u;
+  r.log_count = reactions;
+  if (propose_only) r.log_count = num ? h[kHdrLog] : 0u;
   if (stats) {
     unsigned long long ctr[CTR_WORDS] = {};
     HIP_TRY(hipMemcpy(ctr, c->counters.p, sizeof(ctr), hipMemcpyDeviceToHost));
@@ -326,7 +341,11 @@ int ensure_react_buffers(mcg_ctx* c) {
     bad = c->fp32() ? (r.sxf.alloc(cap) || r.syf.alloc(cap) || r.szf.alloc(cap))
                     : (r.sx.alloc(cap) || r.sy.alloc(cap) || r.sz.alloc(cap));
   if (bad) return fail(MCG_E_NOMEM, "reaction buffers");
-  if (!r.hdr_host) HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r.hdr_host), kHdrWords * 4, hipHostMallocDefault));
+  if (!r.hdr_host) {
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r.hdr_host), kHdrHostWords * 4, hipHostMallocDefault));
+    std::memset(r.hdr_host, 0, kHdrHostWords * 4);
+    HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void**>(&r.hdr_host_d), r.hdr_host, 0));
+  }
   std::vector<int32_t> none((size_t)ns * ns, -1);
   if (r.pair.empty()) r.pair = none;
   HIP_TRY(hipMemcpy(r.pair_d.p, r.pair.data(), r.pair.size() * 4, hipMemcpyHostToDevice));
@@ -368,6 +387,7 @@ int react_step(mcg_ctx* c, uint32_t first_iteration, uint32_t num_iterations, do
     if (r.num_cells == 0) return fail(MCG_E_LIMIT, "reaction grid too large (cells x replicas x species)");
     if (r.cell_count.alloc((size_t)r.num_cells + 1) || r.cell_start.alloc((size_t)r.num_cells + 1))
       return fail(MCG_E_NOMEM, "cell grid");
+    HIP_TRY(launch_fill_u32(c->stream, r.cell_count.p, 0u, r.num_cells + 1));  // (from here on k_scatter clears it)
     size_t tmp = ReactPipeline<double>::scan_bytes(r.num_cells, (uint32_t)c->cfg.molecule_capacity);
     if (tmp > r.scan_tmp.n && r.scan_tmp.alloc(tmp)) return fail(MCG_E_NOMEM, "scan scratch");
     r.grid_dirty = false;
@@ -388,6 +408,15 @@ int react_step(mcg_ctx* c, uint32_t first_iteration, uint32_t num_iterations, do
     if (r.rxn_counts.alloc(std::max<size_t>(n, 1))) return fail(MCG_E_NOMEM, "reaction counts");
     HIP_TRY(hipMemset(r.rxn_counts.p, 0, std::max<size_t>(n, 1) * 8));
   }
+  r.volume_products = false;
+  for (const RxnRec& x : r.rxns)
+    for (uint32_t q = 0; q < x.num_pathways; ++q) r.volume_products |= x.num_products[q] > 0;
+  for (const UnimolRec& x : r.unimol)
+    for (uint32_t q = 0; q < x.num_pathways; ++q) r.volume_products |= x.num_products[q] > 0 || x.keep[q] != 0;
+  for (const VolSurfRec& x : r.vs)
+    for (uint32_t q = 0; q < x.num_pathways; ++q)
+      for (uint32_t i = 0; i < x.num_products[q]; ++i)
+        r.volume_products |= !((x.surf_mask[q] >> i) & 1u) && x.keep_vol[q] != i + 1;
   HIP_TRY(hipEventRecord(c->ev0, c->stream));
   double move_ms = 0;
   int st;
@@ -1047,10 +1076,12 @@ int surface_phase(mcg_ctx* c, uint32_t iteration, double barrier, uint32_t* err)
     P.pass = pass;
     P.clist = conts[pass & 1];
     P.ccount = r.hdr.p + cwords[pass & 1];
-    HIP_TRY(launch_zero_word(c->stream, P.ccount));
+    HIP_TRY(launch_clear_words(c->stream, r.hdr.p, kHdrSurfProps, words[0], cwords[pass & 1]));
     HIP_TRY(surf_round(c->stream, P, in_list, in_count, n_in, lists[0], r.hdr.p + words[0]));
     for (uint32_t round = 0;; ++round) {
-      if (int st = read_hdr(c)) return st;
+      // (the copy clears the counter of the list the next round appends to)
+      HIP_TRY(launch_publish(c->stream, r.hdr.p, r.hdr_host_d, ++r.hdr_seq, false, words[(round + 1) & 1]));
+      if (int st = wait_hdr(c)) return st;
       const uint32_t nl = h[words[round & 1]];
       if (nl == 0) break;
       if (round > 100000) return fail(MCG_E_LIMIT, "surface moves did not settle");

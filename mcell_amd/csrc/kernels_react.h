@@ -56,8 +56,23 @@ enum : uint32_t {
   kHdrSurfLose1 = 14,
   kHdrSurfCont0 = 15,     // surface phase: molecules that step again in this iteration (two lists)
   kHdrSurfCont1 = 16,
-  kHdrWords = 18,
+  kHdrOutBase = 17,       // products: the first output slot of the phase's new molecules
+  kHdrBatch = 18,         // products: the phase's reactions
+  kHdrReacted = 19,       // reactions of the call
+  kHdrLogBase = 20,       // products: reactions of the call before the phase
+  kHdrMoveStart = 22,     // (64 bits) device clock at the start of the iteration's first move
+  kHdrMoveTicks = 24,     // (64 bits) device clock ticks the call's first moves took
+  kHdrWords = 26,
 };
+// The host's copy of the counters, written by the kernels that end a round:
+// the words, then the number of the copy.
+constexpr uint32_t kHdrSeq = 32;
+constexpr uint32_t kHdrHostWords = 64;
+
+// Phases of up to this many reactions are put in order by one workgroup.
+constexpr uint32_t kSmallBatch = 1024;
+// Rounds expected to have up to this many proposals are settled by one.
+constexpr uint32_t kSmallSettle = 2048;
 
 template <typename PosT>
 struct ReactPipeline {
@@ -82,17 +97,29 @@ struct ReactPipeline {
   void* scan_tmp;
   size_t scan_tmp_bytes;
 
+  uint32_t* hdr_host;  // the host copy, as the device sees it
+  // what earlier rounds led to expect (launch sizes only)
+  uint32_t expect_props;     // proposals of the round
+  uint32_t expect_deferred;  // movers the round's move defers
+
   static size_t scan_bytes(uint32_t num_cells, uint32_t capacity);
+  // the snapshot in bin order; also clears the iteration's counters, claim
+  // words and queues
   hipError_t sort(hipStream_t s, uint32_t n_in, uint32_t num_cells, uint32_t* err);
   hipError_t move(hipStream_t s, bool snapshot_src, const uint32_t* list, const uint32_t* count, uint32_t max_movers,
                   double barrier, bool propose_only, uint32_t* err);
-  hipError_t settle(hipStream_t s, uint32_t max_props, uint32_t* rlist, uint32_t* rcount);
+  // settles the round's claims and hands the host the counters as copy
+  // `seq`; timed: the move's end by the device clock
+  hipError_t settle(hipStream_t s, uint32_t max_props, uint32_t* rlist, uint32_t* rcount, bool timed, uint32_t seq);
+  hipError_t publish(hipStream_t s, bool timed, uint32_t seq);
   hipError_t fire_unimol(hipStream_t s, uint32_t max_due);
-  hipError_t products(hipStream_t s, uint32_t n_acc, uint32_t capacity, RxnEvent* log, uint32_t log_base,
-                      uint32_t log_cap, bool first_phase, uint32_t* err);
+  // the phase's accepted reactions (hdr[kHdrAccepted], at most max_acc;
+  // exactly that many above kSmallBatch): order, ids, new molecules
+  hipError_t products(hipStream_t s, uint32_t max_acc, uint32_t capacity, RxnEvent* log, uint32_t log_cap,
+                      bool first_phase, uint32_t* err);
   // appends the phase's continuing movers to the next phase's mover list
-  // (after its products) and clears their count
-  hipError_t continuations(hipStream_t s, uint32_t max_cont);
+  // (after its products, or to an empty one) and clears their count
+  hipError_t continuations(hipStream_t s, uint32_t max_cont, bool after_products);
   hipError_t log_proposals(hipStream_t s, uint32_t max_props, uint32_t iteration, RxnEvent* log, uint32_t* log_count,
                            uint32_t log_cap);
   hipError_t count_species(hipStream_t s, uint32_t n, uint32_t num_species, uint32_t num_replicas, uint64_t* counts);
@@ -110,6 +137,8 @@ hipError_t launch_count_by_volume(hipStream_t s, const uint32_t* cvol, const uin
                                   uint32_t num_species, uint32_t num_replicas, uint32_t num_volumes,
                                   uint64_t* counts);
 hipError_t launch_fill_u64(hipStream_t s, unsigned long long* p, unsigned long long v, uint32_t n);
-hipError_t launch_copy_u32(hipStream_t s, const uint32_t* src, uint32_t* dst);
+// Copies the counters to the host's copy and clears the round's; also word
+// `clear` (a counter the next round appends to) unless it is kHdrWords.
+hipError_t launch_publish(hipStream_t s, uint32_t* hdr, uint32_t* host, uint32_t seq, bool timed, uint32_t clear);
 
 }  // namespace mcg

@@ -19,16 +19,25 @@
 //                                    movers); a mover whose reaction test
 //                                    succeeds stops with a proposal and claims
 //                                    itself and its partner (atomicMin of its id)
-//   k_accept                         a proposal is accepted when it holds both
-//                                    claims; its reactants are consumed
-//   k_requeue                        claims are released; movers whose proposal
-//                                    lost and that were not consumed move again
-//                                    (same stream, consumed partners skipped)
+//   k_settle (or k_accept,           a proposal is accepted when it holds both
+//   k_requeue, k_publish)            claims, its reactants are consumed; claims
+//                                    are released, movers whose proposal lost
+//                                    and that were not consumed move again
+//                                    (same stream, consumed partners skipped);
+//                                    the counters go to host memory
 //   k_unimol_fire                    due unimolecular events of unconsumed molecules
-//   products                         accepted reactions in (replica, mover id)
-//                                    order get product ids per replica; products
+//   k_order_small (or a sort and     accepted reactions in (replica, mover id)
+//   scans), k_products               order get product ids per replica; products
 //                                    move for the rest of the step as new movers;
 //                                    a surface product takes its receptor's tile
+//
+// An iteration of some 10^5 molecules is bound by the length of this chain,
+// not by its work: small rounds and batches are one workgroup's, the
+// iteration's counters are cleared by kernels that run anyway, and the host
+// waits twice (after the first moves, after the products' moves).  40
+// launches, three copies with a synchronisation and two timing events became
+// 18 launches: A + B -> C with 4,000 molecules 268 -> 177 us an iteration,
+// 50,000 E <-> A + B 500 -> 350 us.
 //
 // The smallest mover id among open proposals always wins its claims, so every
 // round settles at least one proposal.  Molecules leave the snapshot order in
@@ -98,12 +107,35 @@ __global__ __launch_bounds__(256) void k_cell_keys(RMolView<PosT> m, uint32_t n,
   if (i < n && c != kInvalid) rank[i] = base + (uint32_t)(lane - my_head);
 }
 
+// The scatter into bin order.  Its threads also clear what the iteration
+// starts with: the claim words of the slots (in slot order; n bounds the
+// snapshot), the bin counts (the scan has read them) for the next iteration,
+// the queue's counters and the header's.
 template <typename PosT>
 __global__ __launch_bounds__(256) void k_scatter(RMolView<PosT> m, uint32_t n, const uint32_t* __restrict__ key,
                                                  const uint32_t* __restrict__ rank,
-                                                 const uint32_t* __restrict__ cell_start, RMolView<PosT> s) {
+                                                 const uint32_t* __restrict__ cell_start, RMolView<PosT> s,
+                                                 uint32_t* __restrict__ cell_count, uint32_t num_cells,
+                                                 uint32_t* __restrict__ consumed, uint32_t* __restrict__ owner,
+                                                 uint32_t* __restrict__ kept, uint32_t* __restrict__ born,
+                                                 uint32_t* __restrict__ qcount, uint32_t* __restrict__ hdr) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t threads = gridDim.x * blockDim.x;
+  for (uint32_t c = i; c <= num_cells; c += threads) cell_count[c] = 0;
+  for (uint32_t q = i; q < kQueueShards; q += threads) qcount[q] = 0;
+  if (i == 0) {
+    const uint32_t live = cell_start[num_cells];
+    hdr[kHdrNumOut] = live;
+    hdr[kHdrSnapshot] = live;
+    hdr[kHdrAccepted] = 0;
+    hdr[kHdrProposals] = 0;
+    hdr[kHdrExd] = 0;
+  }
   if (i >= n) return;
+  consumed[i] = 0;
+  owner[i] = kInvalid;
+  if (kept) kept[i] = 0;
+  if (born) born[i] = 0;
   const uint32_t c = key[i];
   if (c == kInvalid) return;
   const uint32_t j = cell_start[c] + rank[i];
@@ -117,6 +149,44 @@ __global__ __launch_bounds__(256) void k_scatter(RMolView<PosT> m, uint32_t n, c
   if (s.utime) s.utime[j] = m.utime[i];
   if (s.cvol) s.cvol[j] = m.cvol[i];
   if (s.birth) s.birth[j] = m.birth[i];
+}
+
+// The device clock of the first move's start and end (the drain's form is
+// chosen by it, and it is the time the ABI reports).
+__device__ __forceinline__ void move_started(uint32_t* hdr) {
+  *reinterpret_cast<unsigned long long*>(hdr + kHdrMoveStart) = wall_clock64();
+}
+__device__ __forceinline__ void move_ended(uint32_t* hdr) {
+  unsigned long long* const t = reinterpret_cast<unsigned long long*>(hdr + kHdrMoveStart);
+  t[1] += wall_clock64() - t[0];
+}
+
+// The header to the host's copy, by one workgroup: the words, then -- once
+// they are visible to the host -- the copy's number, which the host waits
+// for.  A blit copy and a stream synchronisation cost 12 us here, this 6.
+__device__ __forceinline__ void publish_header(uint32_t* hdr, uint32_t* host, uint32_t seq, uint32_t clear) {
+  if (threadIdx.x < kHdrWords) {
+    // (the words were counted by atomics, this workgroup's among them: read past the L1)
+    const uint32_t v = __hip_atomic_load(hdr + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(host + threadIdx.x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __threadfence_system();
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(host + kHdrSeq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    // the round's counters, for the next move
+    hdr[kHdrProposals] = 0;
+    hdr[kHdrExd] = 0;
+    hdr[kHdrSurfProps] = 0;
+    if (clear < kHdrWords) hdr[clear] = 0;
+  }
+}
+
+__global__ __launch_bounds__(64) void k_publish(uint32_t* hdr, uint32_t* host, uint32_t seq, uint32_t timed,
+                                                uint32_t clear) {
+  if (timed && threadIdx.x == 0) move_ended(hdr);
+  __syncthreads();
+  publish_header(hdr, host, seq, clear);
 }
 
 // ----------------------------------------------------------------- moves --
@@ -414,8 +484,10 @@ __global__ __launch_bounds__(256, 2) void k_move_drain(ReactParams R, Snapshot<P
 template <typename PosT>
 __global__ __launch_bounds__(256, 4) void k_move_light(ReactParams R, Snapshot<PosT> S, RMolView<PosT> out,
                                                     const uint32_t* __restrict__ count, SpeciesTable species,
-                                                    double barrier, SlowQueue Q, uint32_t* __restrict__ err_out) {
+                                                    double barrier, SlowQueue Q, uint32_t* __restrict__ hdr,
+                                                    uint32_t* __restrict__ err_out) {
   constexpr bool kF32 = sizeof(PosT) == 4;
+  if (blockIdx.x == 0 && threadIdx.x == 0) move_started(hdr);
   __shared__ ZigguratTables T;
   stage_zig(T);
   const uint32_t n = *count;
@@ -646,30 +718,40 @@ __device__ __forceinline__ void append_accepted(bool acc, uint32_t j, const Prop
   }
 }
 
+// What settling a round's claims reads and writes.
+struct SettleArgs {
+  const uint32_t* __restrict__ plist;
+  Proposal* __restrict__ prop;
+  uint32_t* __restrict__ owner;
+  uint32_t* __restrict__ tile_owner;
+  uint32_t* __restrict__ consumed;
+  uint32_t* __restrict__ tile_consumed;
+  uint32_t* __restrict__ out_tag;
+  const RxnRec* __restrict__ rxns;
+  uint32_t rxn_stride;
+  const VolSurfRec* __restrict__ vs_rxns;
+  uint32_t* __restrict__ kept;
+  Proposal* __restrict__ aprop;
+  uint32_t* __restrict__ alist;
+  unsigned long long* __restrict__ ctr;
+  uint32_t* __restrict__ rlist;
+  uint32_t* rcount;
+  uint32_t* hdr;
+};
+
 // A proposal whose mover and partner both carry its claim is accepted.
-template <typename PosT>
-__global__ __launch_bounds__(256) void k_accept(const uint32_t* __restrict__ plist, const uint32_t* __restrict__ pcount,
-                                                Proposal* __restrict__ prop, const uint32_t* __restrict__ owner,
-                                                const uint32_t* __restrict__ tile_owner,
-                                                uint32_t* __restrict__ consumed, uint32_t* __restrict__ tile_consumed,
-                                                uint32_t* __restrict__ out_tag,
-                                                const RxnRec* __restrict__ rxns, uint32_t rxn_stride,
-                                                const VolSurfRec* __restrict__ vs_rxns,
-                                                uint32_t* __restrict__ kept, Proposal* __restrict__ aprop,
-                                                uint32_t* __restrict__ alist,
-                                                uint32_t* __restrict__ acount, unsigned long long* __restrict__ ctr) {
-  const uint32_t n = *pcount;
+__device__ __forceinline__ void accept_claims(const SettleArgs& A, uint32_t n) {
   uint32_t n_reflect = 0, n_cross = 0;
   for (uint32_t q0 = blockIdx.x * blockDim.x; q0 < n; q0 += gridDim.x * blockDim.x) {
   const uint32_t q = q0 + threadIdx.x;
   bool acc = false;
   uint32_t j = 0;
   if (q < n) {
-    j = plist[q];
-    const Proposal& p = prop[j];
+    j = A.plist[q];
+    const Proposal& p = A.prop[j];
     const bool tile = (p.partner_slot & kTileBit) != 0;
     const uint32_t ps = p.partner_slot & ~kTileBit;
-    if (owner[j] == p.mover_id && (tile ? tile_owner[ps] : owner[ps]) == p.mover_id) {
+    if (A.owner[j] == p.mover_id && (tile ? A.tile_owner[ps] : A.owner[ps]) == p.mover_id) {
       acc = true;
       // outcome_bimolecular (diffuse_react_event.cpp:1833-1895): the
       // reactants are consumed unless the pathway keeps them (bit 0: the
@@ -678,36 +760,37 @@ __global__ __launch_bounds__(256) void k_accept(const uint32_t* __restrict__ pli
       // mover's id + 1.
       uint32_t keep = 0;
       if (!tile) {
-        const uint32_t k = rxns[p.replica * rxn_stride + p.rxn].keep[p.pathway];
+        const uint32_t k = A.rxns[p.replica * A.rxn_stride + p.rxn].keep[p.pathway];
         keep = (p.pad & kPadMoverIsB) ? ((k >> 1) & 1u) | ((k & 1u) << 1) : k;
-      } else if (vs_rxns[p.rxn & ~kVolSurfBit].keep_vol[p.pathway & kPathwayMask]) {
+      } else if (A.vs_rxns[p.rxn & ~kVolSurfBit].keep_vol[p.pathway & kPathwayMask]) {
         keep = 1u;
       }
       if (keep & 1u) {
         // the mover stays: its step is repeated through this reaction and
         // goes on (the repeat counts its walls)
-        ++kept[j];
+        ++A.kept[j];
       } else {
         n_reflect += p.pad & 0xFFFFu;  // the walls the mover met before the reaction
         n_cross += (p.pad >> 16) & 0x7FFFu;
-        consumed[j] = p.mover_id + 1;
-        out_tag[j] = out_tag[j] | (MF_DEFUNCT << 8);
+        A.consumed[j] = p.mover_id + 1;
+        A.out_tag[j] = A.out_tag[j] | (MF_DEFUNCT << 8);
       }
       if (tile) {
         // the surface reactant stays when a product of its species keeps it;
         // a consumed tile names its consumer (a kept mover's repeated step
         // passes through it)
-        if (!vs_rxns[p.rxn & ~kVolSurfBit].keep_surf[p.pathway & kPathwayMask]) tile_consumed[ps] = p.mover_id + 1;
+        if (!A.vs_rxns[p.rxn & ~kVolSurfBit].keep_surf[p.pathway & kPathwayMask])
+          A.tile_consumed[ps] = p.mover_id + 1;
       } else if (!(keep & 2u)) {
-        consumed[ps] = p.mover_id + 1;
-        out_tag[ps] = out_tag[ps] | (MF_DEFUNCT << 8);
+        A.consumed[ps] = p.mover_id + 1;
+        A.out_tag[ps] = A.out_tag[ps] | (MF_DEFUNCT << 8);
       }
     }
   }
-  append_accepted(acc, j, prop, aprop, alist, acount);
+  append_accepted(acc, j, A.prop, A.aprop, A.alist, A.hdr + kHdrAccepted);
   }
-  wave_count(ctr + CTR_REFLECTIONS, n_reflect);
-  wave_count(ctr + CTR_CROSSINGS, n_cross);
+  wave_count(A.ctr + CTR_REFLECTIONS, n_reflect);
+  wave_count(A.ctr + CTR_CROSSINGS, n_cross);
 }
 
 // Unimolecular events of the phase (react_unimol_single_molecule +
@@ -754,35 +837,53 @@ __global__ __launch_bounds__(256) void k_unimol_fire(ReactParams R, const uint32
 
 // Releases the claims of every proposal of the round and queues the movers
 // of lost proposals that are still alive.
-__global__ __launch_bounds__(256) void k_requeue(const uint32_t* __restrict__ plist,
-                                                 const uint32_t* __restrict__ pcount,
-                                                 const Proposal* __restrict__ prop, uint32_t* __restrict__ owner,
-                                                 uint32_t* __restrict__ tile_owner,
-                                                 const uint32_t* __restrict__ consumed, uint32_t* __restrict__ rlist,
-                                                 uint32_t* __restrict__ rcount) {
-  const uint32_t n = *pcount;
+__device__ __forceinline__ void requeue_losers(const SettleArgs& A, uint32_t n) {
   for (uint32_t q0 = blockIdx.x * blockDim.x; q0 < n; q0 += gridDim.x * blockDim.x) {
   const uint32_t q = q0 + threadIdx.x;
   bool again = false;
   uint32_t j = 0;
   if (q < n) {
-    j = plist[q];
-    owner[j] = kInvalid;
-    const uint32_t ps = prop[j].partner_slot;
-    if (ps & kTileBit) tile_owner[ps & ~kTileBit] = kInvalid;
-    else owner[ps] = kInvalid;
-    again = consumed[j] == 0;
+    j = A.plist[q];
+    A.owner[j] = kInvalid;
+    const uint32_t ps = A.prop[j].partner_slot;
+    if (ps & kTileBit) A.tile_owner[ps & ~kTileBit] = kInvalid;
+    else A.owner[ps] = kInvalid;
+    again = A.consumed[j] == 0;
   }
   const uint64_t mask = __ballot(again);
   if (mask) {
     const int lane = __lane_id();
     const int leader = __ffsll((long long)mask) - 1;
     uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(rcount, (uint32_t)__popcll(mask));
+    if (lane == leader) base = atomicAdd(A.rcount, (uint32_t)__popcll(mask));
     base = __shfl(base, leader);
-    if (again) rlist[base + __popcll(mask & ((1ull << lane) - 1))] = j;
+    if (again) A.rlist[base + __popcll(mask & ((1ull << lane) - 1))] = j;
   }
   }
+}
+
+__global__ __launch_bounds__(256) void k_accept(SettleArgs A, uint32_t timed) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (timed) move_ended(A.hdr);
+    *A.rcount = 0;
+  }
+  accept_claims(A, A.hdr[kHdrProposals]);
+}
+__global__ __launch_bounds__(256) void k_requeue(SettleArgs A) { requeue_losers(A, A.hdr[kHdrProposals]); }
+
+// A whole round by one workgroup: at up to a few thousand proposals the
+// launches between the steps cost more than the steps.
+__global__ __launch_bounds__(1024) void k_settle(SettleArgs A, uint32_t timed, uint32_t* host, uint32_t seq) {
+  if (threadIdx.x == 0) {
+    if (timed) move_ended(A.hdr);
+    *A.rcount = 0;
+  }
+  const uint32_t n = A.hdr[kHdrProposals];
+  accept_claims(A, n);
+  __syncthreads();
+  requeue_losers(A, n);
+  __syncthreads();
+  publish_header(A.hdr, host, seq, kHdrWords);
 }
 
 // ---------------------------------------------------------------- products --
@@ -798,23 +899,36 @@ __global__ __launch_bounds__(256) void k_requeue(const uint32_t* __restrict__ pl
 // stable).  key = replica << 36 | pass << 33 | late << 32 | mover id.
 __device__ __forceinline__ uint32_t key_replica(uint64_t key) { return (uint32_t)(key >> 36); }
 
+__device__ __forceinline__ uint64_t accepted_key(const Proposal& p, const uint32_t* __restrict__ stag,
+                                                 const double* __restrict__ stoff, uint32_t snapshot,
+                                                 uint32_t first_phase) {
+  const uint32_t j = p.mover_slot;
+  const bool snap = j < snapshot;
+  const bool late = first_phase ? (snap && load_toff(stoff, stag[j], j) != 0.0) : snap;
+  // a fired unimolecular event keeps its draw's pass in pad (k_unimol_fire)
+  const uint32_t pass = (first_phase && (p.rxn & kUnimolBit)) ? min(p.pad & 0xFFu, 7u) : 0u;
+  return ((uint64_t)p.replica << 36) | ((uint64_t)pass << 33) | ((uint64_t)late << 32) | p.mover_id;
+}
+
 __global__ __launch_bounds__(256) void k_acc_keys(const uint32_t* __restrict__ alist, uint32_t n,
                                                   const Proposal* __restrict__ prop, const uint32_t* __restrict__ stag,
                                                   const double* __restrict__ stoff, const uint32_t* __restrict__ hdr,
                                                   uint32_t first_phase, uint64_t* __restrict__ keys) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
-  const Proposal& p = prop[alist[k]];
-  const uint32_t j = p.mover_slot;
-  const bool snap = j < hdr[kHdrSnapshot];
-  const bool late = first_phase ? (snap && load_toff(stoff, stag[j], j) != 0.0) : snap;
-  // a fired unimolecular event keeps its draw's pass in pad (k_unimol_fire)
-  const uint32_t pass = (first_phase && (p.rxn & kUnimolBit)) ? min(p.pad & 0xFFu, 7u) : 0u;
-  keys[k] = ((uint64_t)p.replica << 36) | ((uint64_t)pass << 33) | ((uint64_t)late << 32) | p.mover_id;
+  keys[k] = accepted_key(prop[alist[k]], stag, stoff, hdr[kHdrSnapshot], first_phase);
 }
 
 __device__ __forceinline__ uint32_t new_products(const RxnRec& r, uint32_t pathway) {
   return r.num_products[pathway];
+}
+
+__device__ __forceinline__ uint32_t product_count(const Proposal& p, const RxnRec* __restrict__ rxns,
+                                                  uint32_t rxn_stride, const UnimolRec* __restrict__ unimol,
+                                                  const VolSurfRec* __restrict__ vs_rxns) {
+  return (p.rxn & kUnimolBit)    ? unimol[p.rxn & ~kUnimolBit].num_products[p.pathway]
+         : (p.rxn & kVolSurfBit) ? vs_rxns[p.rxn & ~kVolSurfBit].num_new[p.pathway & kPathwayMask]
+                                 : new_products(rxns[p.replica * rxn_stride + p.rxn], p.pathway);
 }
 
 __global__ __launch_bounds__(256) void k_prod_counts(const uint32_t* __restrict__ sorted_slots, uint32_t n,
@@ -825,14 +939,7 @@ __global__ __launch_bounds__(256) void k_prod_counts(const uint32_t* __restrict_
                                                      uint32_t* __restrict__ cnt) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k > n) return;
-  if (k == n) {
-    cnt[k] = 0;
-    return;
-  }
-  const Proposal& p = prop[sorted_slots[k]];
-  cnt[k] = (p.rxn & kUnimolBit)    ? unimol[p.rxn & ~kUnimolBit].num_products[p.pathway]
-           : (p.rxn & kVolSurfBit) ? vs_rxns[p.rxn & ~kVolSurfBit].num_new[p.pathway & kPathwayMask]
-                                   : new_products(rxns[p.replica * rxn_stride + p.rxn], p.pathway);
+  cnt[k] = k == n ? 0u : product_count(prop[sorted_slots[k]], rxns, rxn_stride, unimol, vs_rxns);
 }
 
 __global__ __launch_bounds__(256) void k_seg_heads(const uint64_t* __restrict__ keys, uint32_t n,
@@ -843,9 +950,102 @@ __global__ __launch_bounds__(256) void k_seg_heads(const uint64_t* __restrict__ 
   if (k == 0 || key_replica(keys[k - 1]) != rep) head[rep] = k;
 }
 
-// Products of accepted reaction k (in (replica, mover id) order) get ids
-// next_id[replica] + (products of earlier reactions of that replica) + i and
-// output slots base + pre[k] + i.  Products created before the iteration's
+// The id of the first product of every reaction: next_id[replica] + the
+// products of that replica's earlier reactions (before k_bump_ids raises
+// next_id).
+__global__ __launch_bounds__(256) void k_first_ids(const uint64_t* __restrict__ keys, uint32_t n,
+                                                   const uint32_t* __restrict__ pre,
+                                                   const uint32_t* __restrict__ head,
+                                                   const uint32_t* __restrict__ next_id,
+                                                   uint32_t* __restrict__ first_id) {
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const uint32_t rep = key_replica(keys[k]);
+  first_id[k] = next_id[rep] + pre[k] - pre[head[rep]];
+}
+
+// The header after the phase's reactions are in order (one thread): their
+// `total` new molecules take the output slots from the used ones on, never
+// past the capacity (k_products reports what does not fit).
+__device__ __forceinline__ void book_batch(uint32_t* __restrict__ hdr, uint32_t n, uint32_t total, uint32_t capacity) {
+  const uint32_t base = hdr[kHdrNumOut];
+  const uint64_t used = (uint64_t)base + total;
+  hdr[kHdrOutBase] = base;
+  hdr[kHdrNumOut] = used < capacity ? (uint32_t)used : capacity;
+  hdr[kHdrBatch] = n;
+  hdr[kHdrLogBase] = hdr[kHdrReacted];
+  hdr[kHdrReacted] += n;
+  hdr[kHdrAccepted] = 0;
+  hdr[kHdrUnimolDue] = 0;
+  hdr[kHdrProductMovers] = 0;
+}
+
+// Order, ids and slots of a phase of at most kSmallBatch reactions by one
+// workgroup: a reaction's place is the number of smaller keys (equal ones in
+// acceptance order, as the stable sort gives them).  One launch for the
+// eight of the sort, scans and updates: 15 us of radix sort alone.
+__global__ __launch_bounds__(kSmallBatch) void k_order_small(
+    const uint32_t* __restrict__ alist, const Proposal* __restrict__ prop, const uint32_t* __restrict__ stag,
+    const double* __restrict__ stoff, const RxnRec* __restrict__ rxns, uint32_t rxn_stride,
+    const UnimolRec* __restrict__ unimol, const VolSurfRec* __restrict__ vs_rxns, uint32_t first_phase,
+    uint32_t capacity, uint32_t* __restrict__ sorted_slots, uint64_t* __restrict__ keys, uint32_t* __restrict__ pre,
+    uint32_t* __restrict__ first_id, uint32_t* head, uint32_t* next_id, uint32_t* hdr) {
+  __shared__ uint64_t skey[kSmallBatch], okey[kSmallBatch];
+  __shared__ uint32_t oslot[kSmallBatch], scan[kSmallBatch + 1];
+  __shared__ uint32_t wave_sum[kSmallBatch / 64];
+  const uint32_t k = threadIdx.x;
+  const uint32_t n = min(hdr[kHdrAccepted], kSmallBatch);
+  const uint32_t slot = k < n ? alist[k] : 0u;
+  uint64_t key = 0;
+  if (k < n) {
+    key = accepted_key(prop[slot], stag, stoff, hdr[kHdrSnapshot], first_phase);
+    skey[k] = key;
+  }
+  __syncthreads();
+  if (k < n) {
+    uint32_t place = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+      const uint64_t o = skey[i];
+      place += (o < key || (o == key && i < k)) ? 1u : 0u;
+    }
+    okey[place] = key;
+    oslot[place] = slot;
+  }
+  __syncthreads();
+  // thread k is now reaction k of the order
+  uint32_t count = 0, rep = 0;
+  if (k < n) {
+    key = okey[k];
+    rep = key_replica(key);
+    sorted_slots[k] = oslot[k];
+    keys[k] = key;
+    count = product_count(prop[oslot[k]], rxns, rxn_stride, unimol, vs_rxns);
+    if (k == 0 || key_replica(okey[k - 1]) != rep) head[rep] = k;
+  }
+  uint32_t incl = count;
+  for (uint32_t o = 1; o < 64; o <<= 1) {
+    const uint32_t v = __shfl_up(incl, o);
+    if (__lane_id() >= o) incl += v;
+  }
+  if (__lane_id() == 63) wave_sum[k / 64] = incl;
+  __syncthreads();
+  uint32_t excl = incl - count;
+  for (uint32_t w = 0; w < k / 64; ++w) excl += wave_sum[w];
+  if (k < n) {
+    scan[k] = excl;
+    pre[k] = excl;
+    if (k == n - 1) scan[n] = excl + count;
+  }
+  __syncthreads();
+  const uint32_t from = k < n ? scan[head[rep]] : 0u;
+  if (k < n) first_id[k] = next_id[rep] + scan[k] - from;
+  __syncthreads();
+  if (k < n && (k == n - 1 || key_replica(okey[k + 1]) != rep)) next_id[rep] += scan[k + 1] - from;
+  if (k == 0) book_batch(hdr, n, n ? scan[n] : 0u, capacity);
+}
+
+// Products of accepted reaction k of the phase's order get ids first_id[k] +
+// i and output slots base + pre[k] + i.  Products created before the iteration's
 // end move in this iteration (diffuse_react_event.cpp:2883-2886).
 // The counter of one carried-out reaction (the volume the mover was in; 0
 // without counted volumes), or ~0.
@@ -874,17 +1074,18 @@ __device__ __forceinline__ void wave_add_counters(unsigned long long* __restrict
 
 template <typename PosT>
 __global__ __launch_bounds__(256) void k_products(ReactParams R, const uint32_t* __restrict__ sorted_slots,
-                                                  const uint64_t* __restrict__ keys, uint32_t n,
+                                                  const uint64_t* __restrict__ keys,
                                                   const Proposal* __restrict__ prop, const uint32_t* __restrict__ pre,
-                                                  const uint32_t* __restrict__ head,
-                                                  const uint32_t* __restrict__ next_id, const uint32_t* __restrict__ hdr,
+                                                  const uint32_t* __restrict__ first_ids,
+                                                  const uint32_t* __restrict__ hdr,
                                                   uint32_t capacity, RMolView<PosT> out, uint32_t* __restrict__ consumed,
                                                   uint32_t* __restrict__ owner, uint32_t* __restrict__ mlist,
                                                   uint32_t* __restrict__ mcount, RxnEvent* __restrict__ log,
-                                                  uint32_t log_base, uint32_t log_cap, uint32_t* __restrict__ err,
+                                                  uint32_t log_cap, uint32_t* __restrict__ err,
                                                   uint32_t* __restrict__ tiles, uint32_t* __restrict__ tile_id,
                                                   uint32_t* __restrict__ tile_consumed, uint32_t* __restrict__ kept) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t n = hdr[kHdrBatch], log_base = hdr[kHdrLogBase];
   // reaction counts, with every lane of the wave present
   wave_add_counters(R.rxn_counts, k < n ? reaction_counter(R, prop[sorted_slots[k]], key_replica(keys[k])) : ~0ull);
   if (k >= n) return;
@@ -898,7 +1099,7 @@ __global__ __launch_bounds__(256) void k_products(ReactParams R, const uint32_t*
     const VolSurfRec& vs = R.vs_rxns[p.rxn & ~kVolSurfBit];
     const uint32_t pw = p.pathway & kPathwayMask, drawn = p.pathway >> 8;
     const uint32_t rep = key_replica(keys[k]);
-    const uint32_t first_id = next_id[rep] + pre[k] - pre[head[rep]];
+    const uint32_t first_id = first_ids[k];
     const uint32_t ts = p.partner_slot & ~kTileBit;
     const uint32_t wall = R.tile_wall[ts - rep * R.total_tiles];
     // a given orientation flips when S is not oriented as in the rule (:2636-2658)
@@ -914,7 +1115,7 @@ __global__ __launch_bounds__(256) void k_products(ReactParams R, const uint32_t*
       }
       if (vs.keep_vol[pw] == q + 1) continue;  // the mover, which goes on with its step
       const uint32_t id = first_id + i;
-      const uint32_t slot = hdr[kHdrNumOut] + pre[k] + i;
+      const uint32_t slot = hdr[kHdrOutBase] + pre[k] + i;
       ++i;
       if (slot >= capacity) {
         atomicOr(err, ERR_QUEUE);
@@ -981,8 +1182,8 @@ __global__ __launch_bounds__(256) void k_products(ReactParams R, const uint32_t*
   const uint32_t np = uni ? R.unimol[p.rxn & ~kUnimolBit].num_products[p.pathway]
                           : R.rxns[p.replica * R.rxn_stride + p.rxn].num_products[p.pathway];
   const uint32_t rep = key_replica(keys[k]);
-  const uint32_t base = hdr[kHdrNumOut];
-  const uint32_t first_id = next_id[rep] + pre[k] - pre[head[rep]];
+  const uint32_t base = hdr[kHdrOutBase];
+  const uint32_t first_id = first_ids[k];
   const bool moves_now = cmp_lt_d(p.time, (double)R.iteration + 1.0, 1e-12);
   for (uint32_t i = 0; i < np; ++i) {
     const uint32_t slot = base + pre[k] + i;
@@ -1034,8 +1235,6 @@ __global__ __launch_bounds__(256) void k_products(ReactParams R, const uint32_t*
   }
 }
 
-// The used output slots never exceed the capacity: k_products wrote no
-// product past it (and reported ERR_QUEUE).
 __global__ void k_bump_ids(const uint64_t* __restrict__ keys, uint32_t n, const uint32_t* __restrict__ pre,
                            const uint32_t* __restrict__ head, uint32_t* __restrict__ next_id,
                            uint32_t* __restrict__ hdr, uint32_t capacity) {
@@ -1043,10 +1242,7 @@ __global__ void k_bump_ids(const uint64_t* __restrict__ keys, uint32_t n, const 
   if (k >= n) return;
   const uint32_t rep = key_replica(keys[k]);
   if (k == n - 1 || key_replica(keys[k + 1]) != rep) next_id[rep] += pre[k + 1] - pre[head[rep]];
-  if (k == n - 1) {
-    const uint64_t used = (uint64_t)hdr[kHdrNumOut] + pre[n];
-    hdr[kHdrNumOut] = used < capacity ? (uint32_t)used : capacity;
-  }
+  if (k == n - 1) book_batch(hdr, n, pre[n], capacity);
 }
 
 // Proposals logged without being carried out (the snapshot parity mode).
@@ -1142,21 +1338,15 @@ static inline dim3 move_grid(uint32_t max_movers) { return dim3(std::min<uint32_
 
 template <typename PosT>
 hipError_t ReactPipeline<PosT>::sort(hipStream_t s, uint32_t n_in, uint32_t num_cells, uint32_t* err) {
-  hipLaunchKernelGGL(k_fill_u32, blocks_for(num_cells + 1), dim3(256), 0, s, cell_count, 0u, num_cells + 1);
+  // the bin counts are zero: cleared when the grid is made, then by every scatter
   if (n_in)
     hipLaunchKernelGGL(k_cell_keys<PosT>, blocks_for(n_in), dim3(256), 0, s, M, n_in, R.P, R.G, key, rank, cell_count,
                        err);
   size_t tmp = scan_tmp_bytes;
   hipError_t e = hipcub::DeviceScan::ExclusiveSum(scan_tmp, tmp, cell_count, cell_start, num_cells + 1, s);
   if (e != hipSuccess) return e;
-  if (n_in) {
-    hipLaunchKernelGGL(k_scatter<PosT>, blocks_for(n_in), dim3(256), 0, s, M, n_in, key, rank, cell_start, Sm);
-    // claim words of the snapshot's slots (n_in bounds it), written in order
-    hipLaunchKernelGGL(k_fill_u32, blocks_for(n_in), dim3(256), 0, s, consumed, 0u, n_in);
-    if (kept) hipLaunchKernelGGL(k_fill_u32, blocks_for(n_in), dim3(256), 0, s, kept, 0u, n_in);
-    if (R.born) hipLaunchKernelGGL(k_fill_u32, blocks_for(n_in), dim3(256), 0, s, R.born, 0u, n_in);
-    hipLaunchKernelGGL(k_fill_u32, blocks_for(n_in), dim3(256), 0, s, owner, kInvalid, n_in);
-  }
+  hipLaunchKernelGGL(k_scatter<PosT>, blocks_for(n_in), dim3(256), 0, s, M, n_in, key, rank, cell_start, Sm,
+                     cell_count, num_cells, consumed, owner, kept, R.born, queue.count, hdr);
   return hipGetLastError();
 }
 
@@ -1186,8 +1376,6 @@ hipError_t ReactPipeline<PosT>::move(hipStream_t s, bool snapshot_src, const uin
   if (max_movers == 0) return hipSuccess;
   Snapshot<PosT> S{Sm.x, Sm.y, Sm.z, Sm.id, Sm.tag, consumed, Sm.toff, Sm.utime, Sm.cvol, Sm.birth};
   const uint32_t po = propose_only ? 1u : 0u;
-  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, hdr + kHdrProposals, 0u, 1u);
-  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, hdr + kHdrExd, 0u, 1u);
   // the deferred steps go to a list that is free during this move: mlist
   // until the products are listed, else the rerun list settle() does not
   // read next
@@ -1197,9 +1385,8 @@ hipError_t ReactPipeline<PosT>::move(hipStream_t s, bool snapshot_src, const uin
   if (list == nullptr && snapshot_src) {
     // every snapshot slot: light pass, then the queued movers in full
     Q.shard_cap = shard_capacity(max_movers, kQueueShards / 2);
-    hipLaunchKernelGGL(k_fill_u32, dim3(kQueueShards / 256), dim3(256), 0, s, Q.count, 0u, kQueueShards);
     hipLaunchKernelGGL(k_move_light<PosT>, blocks_for(max_movers), dim3(256), 0, s, R, S, M, count, species, barrier,
-                       Q, err);
+                       Q, hdr, err);
     Q.nshards = kQueueShards / 2 + std::min<uint32_t>(kQueueShards / 2, blocks_for(max_movers).x);
   } else {
     Q.nshards = 0;
@@ -1218,8 +1405,9 @@ hipError_t ReactPipeline<PosT>::move(hipStream_t s, bool snapshot_src, const uin
       hipLaunchKernelGGL((k_move<PosT, kListPool, TeamT>), move_grid(max_movers), dim3(256), 0, s, R, S, src, M, list,
                          count, species, barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err, ulist,
                          hdr + kHdrUnimolDue, xlist, hdr + kHdrExd);
-    // the deferred steps, with the large pool
-    hipLaunchKernelGGL((k_move<PosT, exd::kPool, TeamT>), move_grid(max_movers), dim3(256), 0, s, R, S, src, M, xlist,
+    // the deferred steps, with the large pool (mostly none: a grid for twice
+    // the last round's)
+    hipLaunchKernelGGL((k_move<PosT, exd::kPool, TeamT>), move_grid(std::min(max_movers, 64 + 2 * expect_deferred)), dim3(256), 0, s, R, S, src, M, xlist,
                        hdr + kHdrExd, species, barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err,
                        ulist, hdr + kHdrUnimolDue, nullptr, nullptr);
   };
@@ -1229,16 +1417,24 @@ hipError_t ReactPipeline<PosT>::move(hipStream_t s, bool snapshot_src, const uin
 }
 
 template <typename PosT>
-hipError_t ReactPipeline<PosT>::settle(hipStream_t s, uint32_t max_props, uint32_t* rlist, uint32_t* rcount) {
+hipError_t ReactPipeline<PosT>::settle(hipStream_t s, uint32_t max_props, uint32_t* rlist, uint32_t* rcount,
+                                       bool timed, uint32_t seq) {
+  const SettleArgs A{plist,  prop,      owner,        tile_owner, consumed, tile_consumed, M.tag, R.rxns, R.rxn_stride,
+                     R.vs_rxns, kept,   aprop,        alist,      R.ctr,    rlist,         rcount, hdr};
+  if (std::min(max_props, expect_props) <= kSmallSettle) {
+    hipLaunchKernelGGL(k_settle, dim3(1), dim3(1024), 0, s, A, timed ? 1u : 0u, hdr_host, seq);
+    return hipGetLastError();
+  }
   // grid-stride over the device's proposal count; max_props bounds it
-  const dim3 grid = dim3(std::min<uint32_t>(blocks_for(max_props).x, 1024u));
-  hipLaunchKernelGGL(k_accept<PosT>, grid, dim3(256), 0, s, plist, hdr + kHdrProposals, prop, owner,
-                     tile_owner, consumed, tile_consumed, M.tag, R.rxns, R.rxn_stride, R.vs_rxns, kept, aprop,
-                     alist, hdr + kHdrAccepted, R.ctr);
-  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, rcount, 0u, 1u);
-  hipLaunchKernelGGL(k_requeue, grid, dim3(256), 0, s, plist, hdr + kHdrProposals, prop, owner,
-                     tile_owner, consumed, rlist, rcount);
-  return hipGetLastError();
+  const dim3 grid = dim3(std::min<uint32_t>(blocks_for(std::min(max_props, 2 * expect_props)).x, 1024u));
+  hipLaunchKernelGGL(k_accept, grid, dim3(256), 0, s, A, timed ? 1u : 0u);
+  hipLaunchKernelGGL(k_requeue, grid, dim3(256), 0, s, A);
+  return publish(s, false, seq);
+}
+
+template <typename PosT>
+hipError_t ReactPipeline<PosT>::publish(hipStream_t s, bool timed, uint32_t seq) {
+  return launch_publish(s, hdr, hdr_host, seq, timed, kHdrWords);
 }
 
 template <typename PosT>
@@ -1250,53 +1446,58 @@ hipError_t ReactPipeline<PosT>::fire_unimol(hipStream_t s, uint32_t max_due) {
 }
 
 template <typename PosT>
-hipError_t ReactPipeline<PosT>::products(hipStream_t s, uint32_t n_acc, uint32_t capacity, RxnEvent* log,
-                                         uint32_t log_base, uint32_t log_cap, bool first_phase, uint32_t* err) {
-  if (n_acc == 0) return hipSuccess;
+hipError_t ReactPipeline<PosT>::products(hipStream_t s, uint32_t max_acc, uint32_t capacity, RxnEvent* log,
+                                         uint32_t log_cap, bool first_phase, uint32_t* err) {
+  if (max_acc == 0) return hipSuccess;
   // the accepted proposals: copies when movers can stay, else in place
   const Proposal* const P = aprop ? aprop : prop;
-  hipLaunchKernelGGL(k_acc_keys, blocks_for(n_acc), dim3(256), 0, s, alist, n_acc, P, Sm.tag, Sm.toff, hdr,
-                     first_phase ? 1u : 0u, keys_a);
-  size_t tmp = scan_tmp_bytes;
-  hipError_t e =
-      hipcub::DeviceRadixSort::SortPairs(scan_tmp, tmp, keys_a, keys_b, alist, alist_sorted, n_acc, 0, 64, s);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_prod_counts, blocks_for(n_acc + 1), dim3(256), 0, s, alist_sorted, n_acc, P, R.rxns,
-                     R.rxn_stride, R.unimol, R.vs_rxns, cnt);
-  tmp = scan_tmp_bytes;
-  e = hipcub::DeviceScan::ExclusiveSum(scan_tmp, tmp, cnt, pre, n_acc + 1, s);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_seg_heads, blocks_for(n_acc), dim3(256), 0, s, keys_b, n_acc, head);
-  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, hdr + kHdrProductMovers, 0u, 1u);
-  hipLaunchKernelGGL(k_products<PosT>, blocks_for(n_acc), dim3(256), 0, s, R, alist_sorted, keys_b, n_acc, P, pre,
-                     head, next_id, hdr, capacity, M, consumed, owner, mlist, hdr + kHdrProductMovers, log, log_base,
-                     log_cap, err, tiles, tile_id, tile_consumed, kept);
-  hipLaunchKernelGGL(k_bump_ids, blocks_for(n_acc), dim3(256), 0, s, keys_b, n_acc, pre, head, next_id, hdr,
-                     capacity);
+  const uint32_t first = first_phase ? 1u : 0u;
+  uint32_t* const first_id = cnt;  // (after the scan has read the counts)
+  if (max_acc <= kSmallBatch) {
+    hipLaunchKernelGGL(k_order_small, dim3(1), dim3(kSmallBatch), 0, s, alist, P, Sm.tag, Sm.toff, R.rxns,
+                       R.rxn_stride, R.unimol, R.vs_rxns, first, capacity, alist_sorted, keys_b, pre, first_id, head,
+                       next_id, hdr);
+  } else {
+    const uint32_t n = max_acc;
+    hipLaunchKernelGGL(k_acc_keys, blocks_for(n), dim3(256), 0, s, alist, n, P, Sm.tag, Sm.toff, hdr, first, keys_a);
+    size_t tmp = scan_tmp_bytes;
+    hipError_t e =
+        hipcub::DeviceRadixSort::SortPairs(scan_tmp, tmp, keys_a, keys_b, alist, alist_sorted, n, 0, 64, s);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_prod_counts, blocks_for(n + 1), dim3(256), 0, s, alist_sorted, n, P, R.rxns, R.rxn_stride,
+                       R.unimol, R.vs_rxns, cnt);
+    tmp = scan_tmp_bytes;
+    e = hipcub::DeviceScan::ExclusiveSum(scan_tmp, tmp, cnt, pre, n + 1, s);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_seg_heads, blocks_for(n), dim3(256), 0, s, keys_b, n, head);
+    hipLaunchKernelGGL(k_first_ids, blocks_for(n), dim3(256), 0, s, keys_b, n, pre, head, next_id, first_id);
+    hipLaunchKernelGGL(k_bump_ids, blocks_for(n), dim3(256), 0, s, keys_b, n, pre, head, next_id, hdr, capacity);
+  }
+  hipLaunchKernelGGL(k_products<PosT>, blocks_for(max_acc), dim3(256), 0, s, R, alist_sorted, keys_b, P, pre, first_id,
+                     hdr, capacity, M, consumed, owner, mlist, hdr + kHdrProductMovers, log, log_cap, err, tiles,
+                     tile_id, tile_consumed, kept);
   return hipGetLastError();
 }
 
-// dst[*dst_count + i] = src[i] for i < *src_count (the counts are read on
-// the device; max bounds the grid).
-__global__ __launch_bounds__(256) void k_append_list(const uint32_t* __restrict__ src,
-                                                     const uint32_t* __restrict__ src_count,
-                                                     uint32_t* __restrict__ dst, const uint32_t* __restrict__ dst_count) {
-  const uint32_t n = *src_count, base = *dst_count;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) dst[base + i] = src[i];
-}
-__global__ void k_take_count(uint32_t* __restrict__ dst_count, uint32_t* __restrict__ src_count) {
+// The continuing movers after the list's *count entries, by one workgroup
+// (one launch instead of two; lists of tens of thousands take it a few us).
+__global__ __launch_bounds__(1024) void k_append_list(const uint32_t* __restrict__ src, uint32_t* src_count,
+                                                      uint32_t* __restrict__ dst, uint32_t* dst_count,
+                                                      uint32_t after_products) {
+  const uint32_t n = *src_count, base = after_products ? *dst_count : 0u;
+  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) dst[base + i] = src[i];
+  __syncthreads();
   if (threadIdx.x == 0) {
-    *dst_count += *src_count;
+    *dst_count = base + n;
     *src_count = 0;
   }
 }
 
 template <typename PosT>
-hipError_t ReactPipeline<PosT>::continuations(hipStream_t s, uint32_t max_cont) {
+hipError_t ReactPipeline<PosT>::continuations(hipStream_t s, uint32_t max_cont, bool after_products) {
   if (max_cont == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_append_list, dim3(std::min<uint32_t>(blocks_for(max_cont).x, 2048u)), dim3(256), 0, s, clist,
-                     hdr + kHdrContinue, mlist, hdr + kHdrProductMovers);
-  hipLaunchKernelGGL(k_take_count, dim3(1), dim3(64), 0, s, hdr + kHdrProductMovers, hdr + kHdrContinue);
+  hipLaunchKernelGGL(k_append_list, dim3(1), dim3(1024), 0, s, clist, hdr + kHdrContinue, mlist,
+                     hdr + kHdrProductMovers, after_products ? 1u : 0u);
   return hipGetLastError();
 }
 
@@ -1391,12 +1592,8 @@ hipError_t launch_fill_u64(hipStream_t s, unsigned long long* p, unsigned long l
   return hipGetLastError();
 }
 
-__global__ void k_copy_u32(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst) {
-  if (threadIdx.x == 0) *dst = *src;
-}
-
-hipError_t launch_copy_u32(hipStream_t s, const uint32_t* src, uint32_t* dst) {
-  hipLaunchKernelGGL(k_copy_u32, dim3(1), dim3(64), 0, s, src, dst);
+hipError_t launch_publish(hipStream_t s, uint32_t* hdr, uint32_t* host, uint32_t seq, bool timed, uint32_t clear) {
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s, hdr, host, seq, timed ? 1u : 0u, clear);
   return hipGetLastError();
 }
 

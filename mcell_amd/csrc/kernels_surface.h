@@ -51,10 +51,12 @@ constexpr uint32_t kSurfPasses = 8;          // steps per iteration (time steps 
 // first round; else the molecules stepping again in this pass, or the
 // movers of the previous round that lost a tile or waited), then the
 // claims' settlement: winners move, losers are listed for the next round.
+// The counters of the proposals and of lose_list are zero on entry.
 hipError_t surf_round(hipStream_t s, const SurfPhase& P, const uint32_t* list, const uint32_t* count,
                       uint32_t max_movers, uint32_t* lose_list, uint32_t* lose_count);
 hipError_t launch_fill_done(hipStream_t s, uint32_t* done, uint32_t n);
-hipError_t launch_zero_word(hipStream_t s, uint32_t* word);
+// Zeroes three words of the header.
+hipError_t launch_clear_words(hipStream_t s, uint32_t* hdr, uint32_t a, uint32_t b, uint32_t c);
 hipError_t launch_fill_claims(hipStream_t s, unsigned long long* claim, uint32_t n);
 
 }  // namespace mcg

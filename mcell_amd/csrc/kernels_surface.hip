@@ -235,8 +235,8 @@ __global__ void k_fill_ones(uint32_t* p, uint32_t n) {
   if (i < n) p[i] = ~0u;
 }
 
-__global__ void k_zero_word(uint32_t* p) {
-  if (threadIdx.x == 0) *p = 0;
+__global__ void k_clear_words(uint32_t* hdr, uint32_t a, uint32_t b, uint32_t c) {
+  if (threadIdx.x == 0) hdr[a] = hdr[b] = hdr[c] = 0;
 }
 
 }  // namespace
@@ -247,8 +247,8 @@ hipError_t launch_fill_done(hipStream_t s, uint32_t* done, uint32_t n) {
   return hipGetLastError();
 }
 
-hipError_t launch_zero_word(hipStream_t s, uint32_t* word) {
-  hipLaunchKernelGGL(k_zero_word, dim3(1), dim3(64), 0, s, word);
+hipError_t launch_clear_words(hipStream_t s, uint32_t* hdr, uint32_t a, uint32_t b, uint32_t c) {
+  hipLaunchKernelGGL(k_clear_words, dim3(1), dim3(64), 0, s, hdr, a, b, c);
   return hipGetLastError();
 }
 
@@ -261,8 +261,6 @@ hipError_t surf_round(hipStream_t s, const SurfPhase& P, const uint32_t* list, c
                       uint32_t max_movers, uint32_t* lose_list, uint32_t* lose_count) {
   if (max_movers == 0) return hipSuccess;
   const uint32_t n_all = P.total_tiles * P.num_replicas;
-  hipLaunchKernelGGL(k_zero_word, dim3(1), dim3(64), 0, s, P.hdr + kHdrSurfProps);
-  hipLaunchKernelGGL(k_zero_word, dim3(1), dim3(64), 0, s, lose_count);
   hipLaunchKernelGGL(k_surf_move, blocks_for(max_movers), dim3(256), 0, s, P, list, count, n_all, lose_list,
                      lose_count);
   const dim3 grid = dim3(std::min<uint32_t>(blocks_for(max_movers).x, 2048u));
