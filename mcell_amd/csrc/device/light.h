@@ -153,6 +153,12 @@ __device__ __forceinline__ bool move_index_box(const PartitionParams& P, D3 pos,
   return true;
 }
 
+// Whether any wall is listed in subpartition s or one of its 26 neighbours
+// (the bit the host sets up with the lists).
+__device__ __forceinline__ bool walls_around(const uint32_t* __restrict__ near_walls, uint32_t s) {
+  return (near_walls[s >> 5] >> (s & 31u)) & 1u;
+}
+
 // FP64: every wall of the index box is an exact WALL_MISS of collide_wall
 // (no hit, no re-draw).  Exact in the reference's arithmetic.
 // `ent` holds the wall records in list order (ent[k] = walls[idx[k]]).

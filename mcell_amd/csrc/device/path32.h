@@ -22,6 +22,7 @@ struct Walls32View {
   const uint32_t* __restrict__ idx;
   const FilterWall* __restrict__ ent32;  // w32[idx[k]] for every list entry k
   const uint32_t* __restrict__ box;      // sub-cell box of every list entry k
+  const WallRec64* __restrict__ ent64;   // w64[idx[k]]
 };
 
 // Rounds the FP64 end point to FP32 keeping it on the same side of the plane

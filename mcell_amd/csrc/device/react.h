@@ -140,20 +140,50 @@ struct Snapshot {
 __device__ __forceinline__ uint32_t pack_sp(int x, int y, int z) {
   return (uint32_t)x | ((uint32_t)y << 10) | ((uint32_t)z << 20);
 }
+//
+// Membership is a bit per cell of a window of 5 x 5 x 5 subpartitions around
+// the move (its index box and one cell more, unless the move spans more than
+// three cells on an axis): an insertion is a bit test, where a search of the
+// list was a chain of LDS reads per cell (22 us for a set of twenty, a third
+// of the longest full step).  Cells outside the window are searched for.
 struct SubpartSet {
   static constexpr int kCap = 48;
+  static constexpr uint32_t kEdge = 5;
   uint32_t* v;
   uint32_t stride;
   int n;
   bool overflow;
+  int x0, y0, z0;    // the window's low corner
+  uint64_t in0, in1; // its cells in the set
   __device__ __forceinline__ uint32_t at(int k) const { return v[(uint32_t)k * stride]; }
   __device__ __forceinline__ void clear() {
     n = 0;
     overflow = false;
+    x0 = y0 = z0 = 0;
+    in0 = in1 = 0;
   }
-  __device__ __forceinline__ void insert(uint32_t s) {
-    for (int k = 0; k < n; ++k)
-      if (at(k) == s) return;
+  __device__ __forceinline__ void window(const int a[3], const int b[3]) {
+    x0 = (a[0] < b[0] ? a[0] : b[0]) - 1;
+    y0 = (a[1] < b[1] ? a[1] : b[1]) - 1;
+    z0 = (a[2] < b[2] ? a[2] : b[2]) - 1;
+  }
+  __device__ __forceinline__ void insert(int x, int y, int z) {
+    const uint32_t dx = (uint32_t)(x - x0), dy = (uint32_t)(y - y0), dz = (uint32_t)(z - z0);
+    const uint32_t s = pack_sp(x, y, z);
+    if (dx < kEdge && dy < kEdge && dz < kEdge) {
+      const uint32_t c = dx + kEdge * dy + kEdge * kEdge * dz;
+      const uint64_t bit = 1ull << (c & 63u);
+      if (c < 64u) {
+        if (in0 & bit) return;
+        in0 |= bit;
+      } else {
+        if (in1 & bit) return;
+        in1 |= bit;
+      }
+    } else {
+      for (int k = 0; k < n; ++k)
+        if (at(k) == s) return;
+    }
     if (n < kCap) v[(uint32_t)(n++) * stride] = s;
     else overflow = true;
   }
@@ -168,16 +198,16 @@ __device__ __forceinline__ void collect_neighbors(const PartitionParams& P, D3 p
   D3 minus = {rel.x - r, rel.y - r, rel.z - r};
   D3 b = {(double)idx[0] * P.sp_len, (double)idx[1] * P.sp_len, (double)idx[2] * P.sp_len};
   int xd = 0, yd = 0, zd = 0;
-  if (minus.x < b.x && minus.x > 0.0) { out.insert(pack_sp(idx[0] - 1, idx[1], idx[2])); xd = -1; }
-  else if (plus.x > b.x + P.sp_len && plus.x < part_len) { out.insert(pack_sp(idx[0] + 1, idx[1], idx[2])); xd = 1; }
-  if (minus.y < b.y && minus.y > 0.0) { out.insert(pack_sp(idx[0], idx[1] - 1, idx[2])); yd = -1; }
-  else if (plus.y > b.y + P.sp_len && plus.y < part_len) { out.insert(pack_sp(idx[0], idx[1] + 1, idx[2])); yd = 1; }
-  if (minus.z < b.z && minus.z > 0.0) { out.insert(pack_sp(idx[0], idx[1], idx[2] - 1)); zd = -1; }
-  else if (plus.z > b.z + P.sp_len && plus.z < part_len) { out.insert(pack_sp(idx[0], idx[1], idx[2] + 1)); zd = 1; }
-  if (xd && yd) out.insert(pack_sp(idx[0] + xd, idx[1] + yd, idx[2]));
-  if (xd && zd) out.insert(pack_sp(idx[0] + xd, idx[1], idx[2] + zd));
-  if (yd && zd) out.insert(pack_sp(idx[0], idx[1] + yd, idx[2] + zd));
-  if (xd && yd && zd) out.insert(pack_sp(idx[0] + xd, idx[1] + yd, idx[2] + zd));
+  if (minus.x < b.x && minus.x > 0.0) { out.insert(idx[0] - 1, idx[1], idx[2]); xd = -1; }
+  else if (plus.x > b.x + P.sp_len && plus.x < part_len) { out.insert(idx[0] + 1, idx[1], idx[2]); xd = 1; }
+  if (minus.y < b.y && minus.y > 0.0) { out.insert(idx[0], idx[1] - 1, idx[2]); yd = -1; }
+  else if (plus.y > b.y + P.sp_len && plus.y < part_len) { out.insert(idx[0], idx[1] + 1, idx[2]); yd = 1; }
+  if (minus.z < b.z && minus.z > 0.0) { out.insert(idx[0], idx[1], idx[2] - 1); zd = -1; }
+  else if (plus.z > b.z + P.sp_len && plus.z < part_len) { out.insert(idx[0], idx[1], idx[2] + 1); zd = 1; }
+  if (xd && yd) out.insert(idx[0] + xd, idx[1] + yd, idx[2]);
+  if (xd && zd) out.insert(idx[0] + xd, idx[1], idx[2] + zd);
+  if (yd && zd) out.insert(idx[0], idx[1] + yd, idx[2] + zd);
+  if (xd && yd && zd) out.insert(idx[0] + xd, idx[1] + yd, idx[2] + zd);
 }
 
 // collect_crossed_subparts with collect_for_molecules (and not for walls):
@@ -189,21 +219,20 @@ __device__ __forceinline__ void collect_molecule_subparts(const PartitionParams&
   out.clear();
   int src[3];
   subpart_3d(P, pos, src[0], src[1], src[2]);  // the subpartition `start` names
-  out.insert(pack_sp(src[0], src[1], src[2]));
+  const D3 dst = {pos.x + disp.x, pos.y + disp.y, pos.z + disp.z};
+  int d[3];
+  subpart_3d(P, dst, d[0], d[1], d[2]);
+  out.window(src, d);
+  out.insert(src[0], src[1], src[2]);
   const double r_nb = P.rxn_radius * 1.41421356238;  // POS_SQRT2, defines.h:148
   if (P.use_expanded_list) collect_neighbors(P, pos, src, r_nb, out);
   SubpartWalk64 walk;
   walk.init(P, pos, start, disp);
   while (walk.next(P, err)) {
-    out.insert(pack_sp(walk.ci[0], walk.ci[1], walk.ci[2]));
+    out.insert(walk.ci[0], walk.ci[1], walk.ci[2]);
     if (P.use_expanded_list) collect_neighbors(P, walk.cp, walk.ci, r_nb, out);
   }
-  if (P.use_expanded_list) {
-    D3 dst = {pos.x + disp.x, pos.y + disp.y, pos.z + disp.z};
-    int d[3];
-    subpart_3d(P, dst, d[0], d[1], d[2]);
-    collect_neighbors(P, dst, d, r_nb, out);
-  }
+  if (P.use_expanded_list) collect_neighbors(P, dst, d, r_nb, out);
   if (out.overflow) err |= ERR_CELLS;
 }
 

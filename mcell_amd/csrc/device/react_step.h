@@ -24,6 +24,7 @@ struct ReactParams {
   const FilterWall* __restrict__ ent32;  // FP32 records in list order (FP32 form)
   const WallRec64* __restrict__ ent64;   // FP64 records in list order
   const uint32_t* __restrict__ ent_box;  // sub-cell box of every list entry
+  const uint32_t* __restrict__ near_walls;  // bit per subpartition (walls_around)
   CellGrid G;
   const RxnRec* __restrict__ rxns;
   uint32_t rxn_stride;                   // reaction classes per replica table (0: one shared table)
@@ -118,7 +119,7 @@ __device__ __forceinline__ bool segment_first_wall(const ReactParams& R, D3 pos,
     return false;
   }
   const uint32_t start = subpart_of(R.P, sx, sy, sz);
-  if (closest_wall_in_subpart64(Solo{}, R.P, R.walls, R.off, R.idx, R.ent_box, start, skip, pos, disp, rng, hit, err))
+  if (closest_wall_in_subpart64(Solo{}, R.P, R.ent64, R.off, R.idx, R.ent_box, start, skip, pos, disp, rng, hit, err))
     return true;
   const D3 dst = {pos.x + part_disp.x, pos.y + part_disp.y, pos.z + part_disp.z};
   int dx, dy, dz;
@@ -127,7 +128,7 @@ __device__ __forceinline__ bool segment_first_wall(const ReactParams& R, D3 pos,
   SubpartWalk64 walk;
   walk.init(R.P, pos, start, part_disp);
   while (walk.next(R.P, err))
-    if (closest_wall_in_subpart64(Solo{}, R.P, R.walls, R.off, R.idx, R.ent_box, walk.cur, skip, pos, disp, rng, hit,
+    if (closest_wall_in_subpart64(Solo{}, R.P, R.ent64, R.off, R.idx, R.ent_box, walk.cur, skip, pos, disp, rng, hit,
                                   err))
       return true;
   return false;
@@ -174,7 +175,7 @@ constexpr uint32_t kPadMoverIsB = 1u << 31;  // the mover is the class's reactan
 template <class TeamT>
 __device__ __forceinline__ bool closest_wall(const TeamT& T, const ReactParams& R, uint32_t s, uint32_t last_hit,
                                              D3 pos, D3& disp, PhiloxStream& rng, WallHit& hit, uint32_t& err) {
-  return closest_wall_in_subpart64(T, R.P, R.walls, R.off, R.idx, R.ent_box, s, last_hit, pos, disp, rng, hit, err);
+  return closest_wall_in_subpart64(T, R.P, TeamT::kShared ? R.walls : R.ent64, R.off, R.idx, R.ent_box, s, last_hit, pos, disp, rng, hit, err);
 }
 
 // The snapshot range of species t's molecules in the k-th subpartition of the

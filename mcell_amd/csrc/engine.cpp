@@ -207,8 +207,12 @@ int mcg_set_geometry(mcg_ctx* c, const double* vertices, uint32_t nv, const uint
   std::vector<uint32_t> eb;
   const uint64_t scanned = entry_boxes(P, c->walls_host, c->off_host, c->idx_host, eb);
   c->long_wall_lists = !c->idx_host.empty() && scanned >= 64 * (uint64_t)c->idx_host.size();
-  if (c->ent64.alloc(e64.size()) || c->ent32.alloc(e32.size()) || c->ent_box.alloc(eb.size()))
+  std::vector<uint32_t> nw_bits;
+  cells_near_walls(P, c->off_host, nw_bits);
+  if (c->ent64.alloc(e64.size()) || c->ent32.alloc(e32.size()) || c->ent_box.alloc(eb.size()) ||
+      c->near_walls.alloc(nw_bits.size()))
     return fail(MCG_E_NOMEM, "wall entry buffers");
+  HIP_TRY(hipMemcpy(c->near_walls.p, nw_bits.data(), nw_bits.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(c->ent64.p, e64.data(), e64.size() * sizeof(WallRec64), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(c->ent32.p, e32.data(), e32.size() * sizeof(WallRec32), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(c->ent_box.p, eb.data(), eb.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
@@ -402,7 +406,8 @@ int free_step(mcg_ctx* c, uint32_t first_iteration, uint32_t num_iterations, mcg
   // species time step 1, so the barrier (>= 1 ahead) never clips a step
   const bool run = !tr.enabled && run_pays(n);
   // launches of some 2.7e8 steps: about ten milliseconds each
-  const uint32_t per_launch = run ? (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(4096, (1ull << 28) / std::max(n, 1u))) : 1u;
+  const uint64_t most = std::min<uint64_t>(4096, (1ull << 28) / std::max(n, 1u));
+  const uint32_t per_launch = run ? (uint32_t)std::max<uint64_t>(1, most) : 1u;
   uint32_t launches = 0;
   for (uint32_t k = 0; k < num_iterations; k += per_launch, launches += run ? 1 : 3) {
     const uint32_t first = first_iteration + k, num = std::min(per_launch, num_iterations - k);

@@ -207,4 +207,20 @@ uint64_t entry_boxes(const PartitionParams& P, const std::vector<WallRec64>& wal
   return scanned;
 }
 
+void cells_near_walls(const PartitionParams& P, const std::vector<uint32_t>& off, std::vector<uint32_t>& bits) {
+  const int n = (int)P.n;
+  const size_t n3 = off.size() - 1;
+  bits.assign((n3 + 31) / 32, 0u);
+  for (size_t s = 0; s < n3; ++s) {
+    if (off[s + 1] == off[s]) continue;
+    const int x = (int)(s % P.n), y = (int)((s / P.n) % P.n), z = (int)(s / P.n2);
+    for (int c = std::max(z - 1, 0); c <= std::min(z + 1, n - 1); ++c)
+      for (int b = std::max(y - 1, 0); b <= std::min(y + 1, n - 1); ++b)
+        for (int a = std::max(x - 1, 0); a <= std::min(x + 1, n - 1); ++a) {
+          const size_t q = (size_t)a + (size_t)b * P.n + (size_t)c * P.n2;
+          bits[q >> 5] |= 1u << (q & 31);
+        }
+  }
+}
+
 }  // namespace mcg

@@ -25,4 +25,8 @@ void bin_walls(const PartitionParams& P, const std::vector<WallRec64>& walls, st
 uint64_t entry_boxes(const PartitionParams& P, const std::vector<WallRec64>& walls, const std::vector<uint32_t>& off,
                  const std::vector<uint32_t>& idx, std::vector<uint32_t>& box);
 
+// One bit per subpartition: whether a wall is listed in it or in one of its
+// 26 neighbours (device/light.h, walls_around).
+void cells_near_walls(const PartitionParams& P, const std::vector<uint32_t>& off, std::vector<uint32_t>& bits);
+
 }  // namespace mcg

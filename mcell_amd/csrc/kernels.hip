@@ -218,8 +218,8 @@ __global__ __launch_bounds__(256) void k_hard64(MolView64 m, SpeciesTable specie
     const D3 disp = draw_displacement(rng, T, sp.space_step);
     uint32_t err = 0, tn = 0;
     uint32_t* tw = trace.enabled ? trace.wall + (size_t)i * kTraceHits : nullptr;
-    const bool alive = diffuse_reflect64(P, W.walls, W.off, W.idx, W.box, SC, tag_species(tag), pos, disp, rng, err,
-                                         tw, tn, n_reflect, n_cross);
+    const bool alive = diffuse_reflect64(P, W.walls, W.ent, W.off, W.idx, W.box, SC, tag_species(tag), pos, disp, rng,
+                                         err, tw, tn, n_reflect, n_cross);
     m.x[i] = pos.x;
     m.y[i] = pos.y;
     m.z[i] = pos.z;
@@ -335,8 +335,8 @@ __global__ __launch_bounds__(256) void k_hard32(MolView32 m, SpeciesTable specie
     // entry-box pre-test; the FP32 filter in front of them cost more than
     // it saved), then the end point rounded to FP32 on its side of nearby
     // wall planes
-    const bool alive = diffuse_reflect64(P, W.w64, W.off, W.idx, W.box, SC, tag_species(tag), pos, disp, rng, err,
-                                         tw, tn, n_reflect, n_cross);
+    const bool alive = diffuse_reflect64(P, W.w64, W.ent64, W.off, W.idx, W.box, SC, tag_species(tag), pos, disp,
+                                         rng, err, tw, tn, n_reflect, n_cross);
     if (!alive) m.tag[i] = tag | (MF_DEFUNCT << 8);
     float fx, fy, fz;
     if (!round_to_fp32_same_side(Solo{}, P, W.w64, W.off, W.idx, W.box, pos.x, pos.y, pos.z, &fx, &fy, &fz))
@@ -390,8 +390,8 @@ struct FreeForm64 {
                                         const D3& disp, PhiloxStream& rng, Pos& p, uint32_t& err, uint32_t& n_reflect,
                                         uint32_t& n_cross) const {
     uint32_t tn = 0;
-    return diffuse_reflect64(P, W.walls, W.off, W.idx, W.box, SC, species, p, disp, rng, err, nullptr, tn, n_reflect,
-                             n_cross);
+    return diffuse_reflect64(P, W.walls, W.ent, W.off, W.idx, W.box, SC, species, p, disp, rng, err, nullptr, tn,
+                             n_reflect, n_cross);
   }
 };
 
@@ -422,8 +422,8 @@ struct FreeForm32 {
                                         uint32_t& n_cross) const {
     uint32_t tn = 0;
     D3 q = {(double)p.x, (double)p.y, (double)p.z};
-    const bool alive = diffuse_reflect64(P, W.w64, W.off, W.idx, W.box, SC, species, q, disp, rng, err, nullptr, tn,
-                                         n_reflect, n_cross);
+    const bool alive = diffuse_reflect64(P, W.w64, W.ent64, W.off, W.idx, W.box, SC, species, q, disp, rng, err,
+                                         nullptr, tn, n_reflect, n_cross);
     if (!round_to_fp32_same_side(Solo{}, P, W.w64, W.off, W.idx, W.box, q.x, q.y, q.z, &p.x, &p.y, &p.z))
       err |= ERR_ROUND32;
     return alive;
@@ -433,7 +433,8 @@ struct FreeForm32 {
 template <class Form>
 __global__ __launch_bounds__(64, 2) void k_run(Form S, uint32_t n, uint32_t per_wave, SpeciesTable species,
                                                SurfaceClasses SC, PartitionParams P, PartitionParams32 Q,
-                                               uint64_t seed, uint32_t first, uint32_t num, uint32_t* __restrict__ err_out,
+                                               uint64_t seed, uint32_t first, uint32_t num,
+                                               uint32_t* __restrict__ err_out,
                                                unsigned long long* __restrict__ ctr) {
   __shared__ FastZiggurat F;
   __shared__ ZigguratTables T;
@@ -543,8 +544,8 @@ hipError_t launch_run64(hipStream_t s, const MolView64& m, uint32_t n, SpeciesTa
                         uint32_t* err, unsigned long long* ctr) {
   if (n == 0 || num == 0) return hipSuccess;
   const uint32_t per = run_per_wave(n);
-  hipLaunchKernelGGL(k_run<FreeForm64>, dim3((n + per - 1) / per), dim3(64), 0, s, FreeForm64{m, W}, n, per, species, SC, P,
-                     make_partition32(P), seed, first, num, err, ctr);
+  hipLaunchKernelGGL(k_run<FreeForm64>, dim3((n + per - 1) / per), dim3(64), 0, s, FreeForm64{m, W}, n, per,
+                     species, SC, P, make_partition32(P), seed, first, num, err, ctr);
   return hipGetLastError();
 }
 
@@ -556,9 +557,9 @@ hipError_t launch_run32(hipStream_t s, const MolView32& m, uint32_t n, SpeciesTa
   const FilterParams F = make_filter_params(max_abs_coord, kMoveUlps);
   const float band = 2.0f * F.e_dd + 8.0f * F.eps * max_abs_coord;
   const Walls32View W32{W.walls, reinterpret_cast<const FilterWall*>(w32), W.off, W.idx,
-                        reinterpret_cast<const FilterWall*>(W.ent32), W.box};
-  hipLaunchKernelGGL(k_run<FreeForm32>, dim3((n + per - 1) / per), dim3(64), 0, s, FreeForm32{m, W32, F, band}, n, per, species,
-                     SC, P, make_partition32(P), seed, first, num, err, ctr);
+                        reinterpret_cast<const FilterWall*>(W.ent32), W.box, W.ent};
+  hipLaunchKernelGGL(k_run<FreeForm32>, dim3((n + per - 1) / per), dim3(64), 0, s, FreeForm32{m, W32, F, band}, n, per,
+                     species, SC, P, make_partition32(P), seed, first, num, err, ctr);
   return hipGetLastError();
 }
 
@@ -593,7 +594,7 @@ hipError_t launch_diffuse_reflect32(hipStream_t s, const MolView32& m, uint32_t 
   FilterParams F = make_filter_params(max_abs_coord, kMoveUlps);
   float band = 2.0f * F.e_dd + 8.0f * F.eps * max_abs_coord;
   Walls32View W32{W.walls, reinterpret_cast<const FilterWall*>(w32), W.off, W.idx,
-                  reinterpret_cast<const FilterWall*>(W.ent32), W.box};
+                  reinterpret_cast<const FilterWall*>(W.ent32), W.box, W.ent};
   const PartitionParams32 P32 = make_partition32(P);
   MQ.shard_cap = shard_capacity(n);
   MQ.nshards = kQueueShards;

@@ -223,14 +223,12 @@ __device__ __forceinline__ uint32_t store_pos(const TeamT& T, const ReactParams&
 }
 
 // The snapshot range of species t's molecules in the row of cells
-// (x0 .. x0 + nx, y, z) of replica rep (bins of one row are consecutive).
+// (x0 .. x0 + nx, y, z), all inside the grid, of replica rep (bins of one row
+// are consecutive).
 __device__ __forceinline__ void row_range(const CellGrid& G, uint32_t rep, uint32_t t, int x0, int y, int z, int nx,
                                           uint32_t& k0, uint32_t& k1) {
-  uint32_t c0;
-  if (!cell_of(G, x0, y, z, c0)) {
-    k0 = k1 = 0;
-    return;
-  }
+  const uint32_t c0 = (uint32_t)(x0 - G.lo[0]) +
+                      (uint32_t)G.dim[0] * ((uint32_t)(y - G.lo[1]) + (uint32_t)G.dim[1] * (uint32_t)(z - G.lo[2]));
   const uint32_t b0 = bin_of(G, rep, t, c0);
   k0 = G.start[b0];
   k1 = G.start[b0 + (uint32_t)nx + 1];
@@ -281,8 +279,8 @@ __device__ __forceinline__ void append_slot(bool want, uint32_t j, uint32_t* __r
 // The team's lanes call it together; the leader writes and returns the
 // outcome, the others return false with nothing due or deferred.
 template <typename PosT, int kPoolN, class TeamT>
-__device__ __forceinline__ bool move_one(const TeamT& L, const ReactParams& R, const Snapshot<PosT>& S, const RMolView<PosT>& src,
-                                         const RMolView<PosT>& out, uint32_t j, SpeciesTable species,
+__device__ __forceinline__ bool move_one(const TeamT& L, const ReactParams& R, const Snapshot<PosT>& S,
+                                         const RMolView<PosT>& src, const RMolView<PosT>& out, uint32_t j, SpeciesTable species,
                                          const ZigguratTables& T, double barrier, uint32_t propose_only,
                                          Proposal* __restrict__ prop, uint32_t* __restrict__ owner,
                                          uint32_t* __restrict__ tile_owner, uint32_t* __restrict__ err_out,
@@ -479,16 +477,25 @@ __global__ __launch_bounds__(256, 2) void k_move_drain(ReactParams R, Snapshot<P
 // partners in the start or end subpartition, which the reference always
 // collects, are processed here in the reference's order when no wall is near
 // the collision point: exact_disk is then exactly 1, and a failed
-// test_bimolecular draw leaves the move as it was.  Registers are capped at
-// 128 (4 waves per SIMD); one register more costs a wave.
+// test_bimolecular draw leaves the move as it was.  Bound by instruction
+// issue: half of the vector issue slots at three or four waves per SIMD,
+// which run alike (three spill nothing in either form).  With one bit for
+// moves away from all walls, the partner rows read as one list, the class
+// table in LDS and collisions kept as time, class and slot the replica batch
+// (1.1e7 molecules, FP32) takes 1.36 ms for 1.53 before.
 template <typename PosT>
-__global__ __launch_bounds__(256, 4) void k_move_light(ReactParams R, Snapshot<PosT> S, RMolView<PosT> out,
+__global__ __launch_bounds__(256, 3) void k_move_light(ReactParams R, Snapshot<PosT> S, RMolView<PosT> out,
                                                     const uint32_t* __restrict__ count, SpeciesTable species,
                                                     double barrier, SlowQueue Q, uint32_t* __restrict__ hdr,
                                                     uint32_t* __restrict__ err_out) {
   constexpr bool kF32 = sizeof(PosT) == 4;
   if (blockIdx.x == 0 && threadIdx.x == 0) move_started(hdr);
   __shared__ ZigguratTables T;
+  // the class of a species pair, for tables of up to sixteen species in LDS:
+  // a mover asks for every species in turn
+  __shared__ int32_t pairs[256];
+  const bool pairs_staged = R.num_species <= 16;
+  if (pairs_staged && threadIdx.x < R.num_species * R.num_species) pairs[threadIdx.x] = R.pair_rxn[threadIdx.x];
   stage_zig(T);
   const uint32_t n = *count;
   const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
@@ -532,7 +539,12 @@ __global__ __launch_bounds__(256, 4) void k_move_light(ReactParams R, Snapshot<P
       int lo[3], hi[3];
       bool clear = move_index_box(R.P, pos, end, lo, hi);
       bool near_plane = false;
-      if (clear) {
+      // most moves stay within a cell of their start and start two cells or
+      // more from any wall: one bit says so, instead of the lists of up to
+      // eight cells one after the other
+      const bool open = clear && hi[0] - lo[0] <= 1 && hi[1] - lo[1] <= 1 && hi[2] - lo[2] <= 1 &&
+                        !walls_around(R.near_walls, subpart_index(R.P, pos));
+      if (clear && !open) {
         if (kF32) clear = all_walls_miss32(R.P, R.ent32, R.off, R.ent_box, R.F, R.band, pos, disp, lo, hi, near_plane);
         else clear = all_walls_miss64(R.P, R.ent64, R.off, R.ent_box, pos, disp, lo, hi);
       }
@@ -558,54 +570,56 @@ __global__ __launch_bounds__(256, 4) void k_move_light(ReactParams R, Snapshot<P
         const PartnerBox<PosT> box((a[0] < b[0] ? a[0] : b[0]) - R1, (a[0] < b[0] ? b[0] : a[0]) + R1,
                                    (a[1] < b[1] ? a[1] : b[1]) - R1, (a[1] < b[1] ? b[1] : a[1]) + R1,
                                    (a[2] < b[2] ? a[2] : b[2]) - R1, (a[2] < b[2] ? b[2] : a[2]) + R1);
-        // up to two collisions are resolved here when both partners sit in the
-        // start or end subpartition (cells every collection of the reference holds)
-        int ss[3], se[3];
-        subpart_3d(R.P, pos, ss[0], ss[1], ss[2]);
-        subpart_3d(R.P, end, se[0], se[1], se[2]);
+        // up to two collisions, by time, class and partner slot: the rest of
+        // them is worked out again for the few movers that have one
         int ncand = 0;
-        double ct[2];
-        uint32_t cid[2];
-        int32_t crx[2];
-        D3 ccp[2];
-        bool cok[2];
+        double t0 = 0, t1 = 0;
+        uint32_t s0 = 0, s1 = 0;
+        int32_t x0 = 0, x1 = 0;
         // one species' partners in a row of cells along x are one range of the
-        // snapshot; the next row's range is loaded while the current row's
-        // partners are tested, and partner positions are loaded kGroup at a
-        // time, so that the dependent loads overlap (the candidates' order
+        // snapshot; the ranges of up to four rows are loaded together and
+        // their partners read as one list, kGroup at a time, so that a scan
+        // is a few rounds of loads in flight together (the candidates' order
         // does not matter: at most two are kept and they are sorted below)
-        constexpr int kGroup = kF32 ? 4 : 2;
+        constexpr int kGroup = 4;
         const int nx = chi[0] - clo[0];
         const bool rows = nx >= 0 && chi[1] >= clo[1] && chi[2] >= clo[2];
         for (uint32_t t = 0; t < R.G.ns && rows && clear; ++t) {
-          const int32_t rx = R.pair_rxn[my_sp * R.num_species + t];
+          const uint32_t pair = my_sp * R.num_species + t;
+          const int32_t rx = pairs_staged ? pairs[pair] : R.pair_rxn[pair];
           if (rx < 0) continue;
           int y = clo[1], z = clo[2];
-          uint32_t n0, n1;
-          row_range(R.G, rep, t, clo[0], y, z, nx, n0, n1);
-          while (clear) {
-            const uint32_t k0 = n0, k1 = n1;
-            const bool last = y == chi[1] && z == chi[2];
-            if (!last) {
-              if (++y > chi[1]) {
-                y = clo[1];
-                ++z;
-              }
-              row_range(R.G, rep, t, clo[0], y, z, nx, n0, n1);
+          while (z <= chi[2] && clear) {
+            uint32_t from[4], len[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const bool have = z <= chi[2];
+              uint32_t k0, k1;
+              row_range(R.G, rep, t, clo[0], y, have ? z : chi[2], nx, k0, k1);
+              from[q] = k0;
+              len[q] = have ? k1 - k0 : 0u;
+              const bool wrap = y == chi[1];
+              y = wrap ? clo[1] : y + 1;
+              z += wrap ? 1 : 0;
             }
-            for (uint32_t kb = k0; kb < k1 && clear; kb += kGroup) {
+            const uint32_t c1 = len[0], c2 = c1 + len[1], c3 = c2 + len[2], total = c3 + len[3];
+            const uint32_t o1 = from[1] - c1, o2 = from[2] - c2, o3 = from[3] - c3;
+            for (uint32_t mb = 0; mb < total && clear; mb += kGroup) {
+              uint32_t gk[kGroup];
               PosT gx[kGroup], gy[kGroup], gz[kGroup];
 #pragma unroll
               for (int u = 0; u < kGroup; ++u) {
-                const uint32_t k = kb + u < k1 ? kb + u : k1 - 1;
+                const uint32_t m = mb + u < total ? mb + u : total - 1;
+                const uint32_t k = m + (m < c1 ? from[0] : m < c2 ? o1 : m < c3 ? o2 : o3);
+                gk[u] = k;
                 gx[u] = S.x[k];
                 gy[u] = S.y[k];
                 gz[u] = S.z[k];
               }
 #pragma unroll
               for (int u = 0; u < kGroup; ++u) {
-                const uint32_t k = kb + u;
-                if (k >= k1 || !clear) break;
+                const uint32_t k = gk[u];
+                if (mb + u >= total || !clear) break;
                 if (box.outside(gx[u], gy[u], gz[u])) continue;
                 const double qx = (double)gx[u], qy = (double)gy[u], qz = (double)gz[u];
                 double tc;
@@ -616,50 +630,63 @@ __global__ __launch_bounds__(256, 4) void k_move_light(ReactParams R, Snapshot<P
                   clear = false;
                   break;
                 }
-                int q3[3];
-                subpart_3d(R.P, D3{qx, qy, qz}, q3[0], q3[1], q3[2]);
-                ct[ncand] = tc;
-                cid[ncand] = S.id[k];
-                crx[ncand] = rx;
-                ccp[ncand] = cp;
-                cok[ncand] = (q3[0] == ss[0] && q3[1] == ss[1] && q3[2] == ss[2]) ||
-                             (q3[0] == se[0] && q3[1] == se[1] && q3[2] == se[2]);
+                if (ncand == 0) {
+                  t0 = tc;
+                  s0 = k;
+                  x0 = rx;
+                } else {
+                  t1 = tc;
+                  s1 = k;
+                  x1 = rx;
+                }
                 ++ncand;
               }
             }
-            if (last) break;
           }
         }
         if (clear && ncand > 0) {
           // the reference's order: time, then the larger partner id first
-          if (ncand == 2 && (ct[1] < ct[0] || (ct[1] == ct[0] && cid[1] > cid[0]))) {
-            const double tt = ct[0]; ct[0] = ct[1]; ct[1] = tt;
-            const uint32_t ti = cid[0]; cid[0] = cid[1]; cid[1] = ti;
-            const int32_t tr = crx[0]; crx[0] = crx[1]; crx[1] = tr;
-            const D3 tp = ccp[0]; ccp[0] = ccp[1]; ccp[1] = tp;
-            const bool tb = cok[0]; cok[0] = cok[1]; cok[1] = tb;
+          if (ncand == 2 && (t1 < t0 || (t1 == t0 && S.id[s1] > S.id[s0]))) {
+            const double tt = t0; t0 = t1; t1 = tt;
+            const uint32_t ts = s0; s0 = s1; s1 = ts;
+            const int32_t tx = x0; x0 = x1; x1 = tx;
           }
+          // resolved here when the partners sit in the start or end
+          // subpartition (cells every collection of the reference holds)
+          int ss[3], se[3];
+          subpart_3d(R.P, pos, ss[0], ss[1], ss[2]);
+          subpart_3d(R.P, end, se[0], se[1], se[2]);
+#pragma unroll 1
           for (int q = 0; q < ncand && clear; ++q) {
-            if (!cok[q]) {
+            const double tq = q == 0 ? t0 : t1;
+            const uint32_t sq = q == 0 ? s0 : s1;
+            const int32_t xq = q == 0 ? x0 : x1;
+            int q3[3];
+            subpart_3d(R.P, D3{(double)S.x[sq], (double)S.y[sq], (double)S.z[sq]}, q3[0], q3[1], q3[2]);
+            if (!((q3[0] == ss[0] && q3[1] == ss[1] && q3[2] == ss[2]) ||
+                  (q3[0] == se[0] && q3[1] == se[1] && q3[2] == se[2]))) {
               clear = false;
               break;
             }
-            if (ct[q] < STIME_EPS) continue;  // is_immediate_collision (collision_utils.inl:814-816)
+            const D3 cpq = {pos.x + tq * disp.x, pos.y + tq * disp.y, pos.z + tq * disp.z};  // as collide_mol has it
+            if (tq < STIME_EPS) continue;  // is_immediate_collision (collision_utils.inl:814-816)
             // exact_disk is exactly 1 when no wall of the collision point's
             // subpartition comes within R of it (no wall is processed)
-            int qx, qy, qz;
-            subpart_3d(R.P, ccp[q], qx, qy, qz);
-            const uint32_t csp = subpart_of(R.P, qx, qy, qz);
-            const uint32_t db = region_box(R.P, csp, ccp[q].x - R1, ccp[q].y - R1, ccp[q].z - R1, ccp[q].x + R1,
-                                           ccp[q].y + R1, ccp[q].z + R1);
-            const uint32_t e1 = R.off[csp + 1];
-            if (next_overlap<kLightOverlapGroup>(R.ent_box, R.off[csp], e1, db) < e1) {
-              clear = false;
-              break;
+            if (!open) {
+              int qx, qy, qz;
+              subpart_3d(R.P, cpq, qx, qy, qz);
+              const uint32_t csp = subpart_of(R.P, qx, qy, qz);
+              const uint32_t db = region_box(R.P, csp, cpq.x - R1, cpq.y - R1, cpq.z - R1, cpq.x + R1,
+                                             cpq.y + R1, cpq.z + R1);
+              const uint32_t e1 = R.off[csp + 1];
+              if (next_overlap<kLightOverlapGroup>(R.ent_box, R.off[csp], e1, db) < e1) {
+                clear = false;
+                break;
+              }
             }
             // test_bimolecular with factor 1: a reaction goes to the full step,
             // which re-draws the same numbers and proposes it
-            if (test_bimolecular(R.rxns[rep * R.rxn_stride + crx[q]], r_rate_factor, rng) >= 0) clear = false;
+            if (test_bimolecular(R.rxns[rep * R.rxn_stride + xq], r_rate_factor, rng) >= 0) clear = false;
           }
         }
       }
@@ -1407,8 +1434,8 @@ hipError_t ReactPipeline<PosT>::move(hipStream_t s, bool snapshot_src, const uin
                          hdr + kHdrUnimolDue, xlist, hdr + kHdrExd);
     // the deferred steps, with the large pool (mostly none: a grid for twice
     // the last round's)
-    hipLaunchKernelGGL((k_move<PosT, exd::kPool, TeamT>), move_grid(std::min(max_movers, 64 + 2 * expect_deferred)), dim3(256), 0, s, R, S, src, M, xlist,
-                       hdr + kHdrExd, species, barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err,
+    const dim3 grid = move_grid(std::min(max_movers, 64 + 2 * expect_deferred));
+    hipLaunchKernelGGL((k_move<PosT, exd::kPool, TeamT>), grid, dim3(256), 0, s, R, S, src, M, xlist, hdr + kHdrExd, species, barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err,
                        ulist, hdr + kHdrUnimolDue, nullptr, nullptr);
   };
   if (teams) full_steps(Team{1, 0});
