@@ -486,8 +486,8 @@ __global__ __launch_bounds__(256, 2) void k_move_drain(ReactParams R, Snapshot<P
 template <typename PosT>
 __global__ __launch_bounds__(256, 3) void k_move_light(ReactParams R, Snapshot<PosT> S, RMolView<PosT> out,
                                                     const uint32_t* __restrict__ count, SpeciesTable species,
-                                                    double barrier, SlowQueue Q, uint32_t* __restrict__ hdr,
-                                                    uint32_t* __restrict__ err_out) {
+                                                    double barrier, SlowQueue Q, uint32_t per_wave,
+                                                    uint32_t* __restrict__ hdr, uint32_t* __restrict__ err_out) {
   constexpr bool kF32 = sizeof(PosT) == 4;
   if (blockIdx.x == 0 && threadIdx.x == 0) move_started(hdr);
   __shared__ ZigguratTables T;
@@ -498,10 +498,10 @@ __global__ __launch_bounds__(256, 3) void k_move_light(ReactParams R, Snapshot<P
   if (pairs_staged && threadIdx.x < R.num_species * R.num_species) pairs[threadIdx.x] = R.pair_rxn[threadIdx.x];
   stage_zig(T);
   const uint32_t n = *count;
-  const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t j = (blockIdx.x * (blockDim.x / 64u) + threadIdx.x / 64u) * per_wave + __lane_id();
   bool hard = false, partner_hard = false;
   uint32_t err = 0;
-  if (j < n) {
+  if (__lane_id() < per_wave && j < n) {
     const uint32_t tag = S.tag[j];
     const uint32_t idv = S.id[j];
     const double toff = load_toff(S.toff, tag, j);
@@ -1396,6 +1396,13 @@ size_t ReactPipeline<PosT>::scan_bytes(uint32_t num_cells, uint32_t capacity) {
 // second, sparse pass over the deferred steps.
 constexpr int kDrainPool = 48;
 constexpr int kListPool = 48;
+// Lists of at most this many movers take the large pool at once: the second
+// launch, mostly empty, cost more than the smaller pool saved (the products'
+// moves of 50,000 E <-> A + B: 44 + 10 us for the two, 44 in one).
+constexpr uint32_t kFewMovers = 8192;
+// Waves the light pass spreads few molecules over (256 CUs x 4 SIMDs x 2):
+// 4,000 molecules take it 16 us for 23 with full waves, 50,000 22 for 24.
+constexpr uint32_t kLightWaves = 2048;
 
 template <typename PosT>
 hipError_t ReactPipeline<PosT>::move(hipStream_t s, bool snapshot_src, const uint32_t* list, const uint32_t* count,
@@ -1412,9 +1419,14 @@ hipError_t ReactPipeline<PosT>::move(hipStream_t s, bool snapshot_src, const uin
   if (list == nullptr && snapshot_src) {
     // every snapshot slot: light pass, then the queued movers in full
     Q.shard_cap = shard_capacity(max_movers, kQueueShards / 2);
-    hipLaunchKernelGGL(k_move_light<PosT>, blocks_for(max_movers), dim3(256), 0, s, R, S, M, count, species, barrier,
-                       Q, hdr, err);
-    Q.nshards = kQueueShards / 2 + std::min<uint32_t>(kQueueShards / 2, blocks_for(max_movers).x);
+    // few molecules are spread over the waves the chip holds, for the same
+    // reason as the full steps (a workgroup of four waves still has a shard of
+    // its own)
+    const uint32_t per_wave = std::min(64u, (max_movers + kLightWaves - 1) / kLightWaves);
+    const uint32_t blocks = (max_movers + 4 * per_wave - 1) / (4 * per_wave);
+    hipLaunchKernelGGL(k_move_light<PosT>, dim3(blocks), dim3(256), 0, s, R, S, M, count, species, barrier, Q,
+                       per_wave, hdr, err);
+    Q.nshards = kQueueShards / 2 + std::min<uint32_t>(kQueueShards / 2, blocks);
   } else {
     Q.nshards = 0;
   }
@@ -1428,7 +1440,12 @@ hipError_t ReactPipeline<PosT>::move(hipStream_t s, bool snapshot_src, const uin
       hipLaunchKernelGGL((k_move_drain<PosT, 0, TeamT>), move_grid(max_movers), dim3(256), 0, s, R, S, Sm, M, Q,
                          species, barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err, ulist,
                          hdr + kHdrUnimolDue, xlist, hdr + kHdrExd);
-    else
+    else if (max_movers <= kFewMovers) {
+      hipLaunchKernelGGL((k_move<PosT, exd::kPool, TeamT>), move_grid(max_movers), dim3(256), 0, s, R, S, src, M, list,
+                         count, species, barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err, ulist,
+                         hdr + kHdrUnimolDue, nullptr, nullptr);
+      return;
+    } else
       hipLaunchKernelGGL((k_move<PosT, kListPool, TeamT>), move_grid(max_movers), dim3(256), 0, s, R, S, src, M, list,
                          count, species, barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err, ulist,
                          hdr + kHdrUnimolDue, xlist, hdr + kHdrExd);

@@ -61,3 +61,39 @@ def test_many_species(gpu_available, precision):
     assert got[0][0] == got[1][0] > 100
     for k in got[0][1]:
         assert np.array_equal(got[0][1][k], got[1][1][k]), k
+
+
+@pytest.mark.parametrize("n_a,n_b", [(1, 0), (1, 1), (1024, 1024), (1025, 1024), (65536, 65536), (65537, 65536)])
+def test_waves_shares_of_the_light_pass(gpu_available, oracle_lib, n_a, n_b):
+    """One molecule a wave up to 2,048, a full wave from 131,009 on: the
+    positions after two snapshot iterations equal the oracle's."""
+    from oracle import pyoracle as po
+    wl = W.bimol_box(n_a=n_a, n_b=n_b, iterations=2, seed=4)
+    eng = DiffuseReactEngine.from_workload(wl, seed=5, propose_only=True, log_capacity=1 << 12)
+    w = po.world_from_workload(wl, draw_mode=po.DRAW_PHILOX, seed=5)
+    w.set_snapshot(True)
+    w.set_barrier_interval(wl.barrier_interval)
+    eng.step(0, 2)
+    w.run(2)
+    m = eng.molecules()
+    assert len(m["id"]) == n_a + n_b
+    assert np.abs(m["pos"][np.argsort(m["id"])] - w.molecules()["pos"]).max() <= 1e-10
+    w.close()
+    eng.close()
+
+
+@pytest.mark.parametrize("n", [500, 20000])
+def test_list_moves_short_and_long(gpu_available, oracle_lib, n):
+    """Second half steps of every molecule: lists below and above the length
+    up to which the list moves take the large pool at once."""
+    from oracle import pyoracle as po
+    wl = W.with_time_steps(W.free_diffusion_box(scale=n / 10000, iterations=4), [0.5])
+    eng = DiffuseReactEngine.from_workload(wl)
+    w = po.world_from_workload(wl, draw_mode=po.DRAW_PHILOX)
+    eng.step(0, 4)
+    w.run(4)
+    m = eng.molecules()
+    got, want = m["pos"][np.argsort(m["id"])], w.molecules()["pos"]
+    assert np.abs(got - want).max() <= 1e-10
+    w.close()
+    eng.close()
