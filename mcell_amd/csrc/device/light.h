@@ -159,11 +159,19 @@ __device__ __forceinline__ bool walls_around(const uint32_t* __restrict__ near_w
   return (near_walls[s >> 5] >> (s & 31u)) & 1u;
 }
 
+// The light passes' walk of a wall list: through the boxes of groups where
+// the context keeps them (long lists), else entry by entry.
+__device__ __forceinline__ uint32_t light_overlap(const uint32_t* __restrict__ box, const uint32_t* __restrict__ group,
+                                                  uint32_t k, uint32_t k1, uint32_t sb) {
+  return group ? next_overlap_grouped(box, group, k, k1, sb) : next_overlap<kLightOverlapGroup>(box, k, k1, sb);
+}
+
 // FP64: every wall of the index box is an exact WALL_MISS of collide_wall
 // (no hit, no re-draw).  Exact in the reference's arithmetic.
 // `ent` holds the wall records in list order (ent[k] = walls[idx[k]]).
 __device__ __forceinline__ bool all_walls_miss64(const PartitionParams& P, const WallRec64* __restrict__ ent,
                                                  const uint32_t* __restrict__ off, const uint32_t* __restrict__ box,
+                                                  const uint32_t* __restrict__ group,
                                                  D3 pos, D3 disp, const int lo[3], const int hi[3]) {
   for (int z = lo[2]; z <= hi[2]; ++z)
     for (int y = lo[1]; y <= hi[1]; ++y)
@@ -172,8 +180,8 @@ __device__ __forceinline__ bool all_walls_miss64(const PartitionParams& P, const
         const uint32_t k0 = off[s], k1 = off[s + 1];
         if (k0 == k1) continue;
         const uint32_t sb = segment_box(P, s, pos.x, pos.y, pos.z, disp.x, disp.y, disp.z);
-        for (uint32_t k = next_overlap<kLightOverlapGroup>(box, k0, k1, sb); k < k1;
-             k = next_overlap<kLightOverlapGroup>(box, k + 1, k1, sb))
+        for (uint32_t k = light_overlap(box, group, k0, k1, sb); k < k1;
+             k = light_overlap(box, group, k + 1, k1, sb))
           if (!wall_certain_miss64(ent[k], pos, disp)) return false;
       }
   return true;
@@ -183,6 +191,7 @@ __device__ __forceinline__ bool all_walls_miss64(const PartitionParams& P, const
 // within `band` of some wall plane.
 __device__ __forceinline__ bool all_walls_miss32(const PartitionParams& P, const FilterWall* __restrict__ ent,
                                                  const uint32_t* __restrict__ off, const uint32_t* __restrict__ box,
+                                                  const uint32_t* __restrict__ group,
                                                  const FilterParams& F, float band, D3 pos, D3 disp,
                                                  const int lo[3], const int hi[3], bool& near_plane) {
   const float px = (float)pos.x, py = (float)pos.y, pz = (float)pos.z;
@@ -194,8 +203,8 @@ __device__ __forceinline__ bool all_walls_miss32(const PartitionParams& P, const
         const uint32_t k0 = off[s], k1 = off[s + 1];
         if (k0 == k1) continue;
         const uint32_t sb = segment_box(P, s, pos.x, pos.y, pos.z, disp.x, disp.y, disp.z);
-        for (uint32_t k = next_overlap<kLightOverlapGroup>(box, k0, k1, sb); k < k1;
-             k = next_overlap<kLightOverlapGroup>(box, k + 1, k1, sb)) {
+        for (uint32_t k = light_overlap(box, group, k0, k1, sb); k < k1;
+             k = light_overlap(box, group, k + 1, k1, sb)) {
           float de;
           if (!certain_miss32(ent[k], F, px, py, pz, mx, my, mz, &de)) return false;
           if (fabs_f(de) < band) near_plane = true;

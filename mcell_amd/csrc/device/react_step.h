@@ -24,6 +24,7 @@ struct ReactParams {
   const FilterWall* __restrict__ ent32;  // FP32 records in list order (FP32 form)
   const WallRec64* __restrict__ ent64;   // FP64 records in list order
   const uint32_t* __restrict__ ent_box;  // sub-cell box of every list entry
+  const uint32_t* __restrict__ ent_group;   // boxes of groups of entries (next_overlap_grouped), or null
   const uint32_t* __restrict__ near_walls;  // bit per subpartition (walls_around)
   CellGrid G;
   const RxnRec* __restrict__ rxns;

@@ -114,4 +114,44 @@ MCG_BOX_HD uint32_t next_overlap(const uint32_t* __restrict__ box, uint32_t k, u
   return k1;
 }
 
+// The box around two boxes: per axis the lower low and the higher high cell.
+MCG_BOX_HD uint32_t box_union(uint32_t a, uint32_t b) {
+  uint32_t r = 0;
+  for (uint32_t s = 0; s < 24; s += 8) {
+    const uint32_t al = (a >> s) & 15u, bl = (b >> s) & 15u, ah = (a >> (s + 4)) & 15u, bh = (b >> (s + 4)) & 15u;
+    r |= (al < bl ? al : bl) << s | (ah < bh ? bh : ah) << (s + 4);
+  }
+  return r;
+}
+
+// next_overlap through the boxes of aligned groups of eight entries
+// (group[g] is the box around box[8 g .. 8 g + 7], used where all eight lie
+// in the list): walls next to each other in a mesh's order mostly lie next to
+// each other in space, so a list of hundreds is left at one read per eight
+// entries where no wall is near.
+constexpr uint32_t kBoxGroup = 8;
+MCG_BOX_HD uint32_t next_overlap_grouped(const uint32_t* __restrict__ box, const uint32_t* __restrict__ group,
+                                         uint32_t k, uint32_t k1, uint32_t sb) {
+  while (k < k1) {
+    if ((k & (kBoxGroup - 1)) == 0 && k + kBoxGroup <= k1) {
+      const uint32_t g = k / kBoxGroup, g1 = k1 / kBoxGroup;
+      uint32_t bx[4], first = 4;
+      for (uint32_t u = 0; u < 4; ++u) bx[u] = group[g + u < g1 ? g + u : g1 - 1];
+      for (uint32_t u = 4; u-- > 0;)
+        if (g + u < g1 && boxes_overlap(bx[u], sb)) first = u;
+      k = (g + first < g1 ? g + first : g1) * kBoxGroup;
+      if (first == 4 || g + first >= g1) continue;
+    }
+    // entries up to the group's end
+    const uint32_t e = (k / kBoxGroup + 1) * kBoxGroup, end = e < k1 ? e : k1;
+    uint32_t bx[kBoxGroup], first = kBoxGroup;
+    for (uint32_t u = 0; u < kBoxGroup; ++u) bx[u] = box[k + u < end ? k + u : end - 1];
+    for (uint32_t u = kBoxGroup; u-- > 0;)
+      if (k + u < end && boxes_overlap(bx[u], sb)) first = u;
+    if (first < kBoxGroup) return k + first;
+    k = end;
+  }
+  return k1;
+}
+
 }  // namespace mcg

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "engine.h"
+#include "device/wallbox.h"
 #include "geometry.h"
 
 using namespace mcg;
@@ -207,6 +208,15 @@ int mcg_set_geometry(mcg_ctx* c, const double* vertices, uint32_t nv, const uint
   std::vector<uint32_t> eb;
   const uint64_t scanned = entry_boxes(P, c->walls_host, c->off_host, c->idx_host, eb);
   c->long_wall_lists = !c->idx_host.empty() && scanned >= 64 * (uint64_t)c->idx_host.size();
+  if (c->long_wall_lists) {
+    std::vector<uint32_t> groups(eb.size() / kBoxGroup + 1, 0u);
+    for (size_t g = 0; (g + 1) * kBoxGroup <= eb.size(); ++g) {
+      groups[g] = eb[g * kBoxGroup];
+      for (size_t u = 1; u < kBoxGroup; ++u) groups[g] = box_union(groups[g], eb[g * kBoxGroup + u]);
+    }
+    if (c->ent_group.alloc(groups.size())) return fail(MCG_E_NOMEM, "wall entry buffers");
+    HIP_TRY(hipMemcpy(c->ent_group.p, groups.data(), groups.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+  }
   std::vector<uint32_t> nw_bits;
   cells_near_walls(P, c->off_host, nw_bits);
   if (c->ent64.alloc(e64.size()) || c->ent32.alloc(e32.size()) || c->ent_box.alloc(eb.size()) ||

@@ -172,6 +172,7 @@ struct mcg_ctx {
   mcg::DevBuf<mcg::WallRec64> ent64;  // wall records in list (entry) order
   mcg::DevBuf<mcg::WallRec32> ent32;
   mcg::DevBuf<uint32_t> ent_box;  // sub-cell box of every list entry
+  mcg::DevBuf<uint32_t> ent_group; // boxes of groups of eight entries (long lists only)
   mcg::DevBuf<uint32_t> near_walls;  // bit per subpartition: a wall is listed in it or next to it
   bool have_geometry = false;
   // full steps run by teams of lanes (device/team.h): worth the exchanges

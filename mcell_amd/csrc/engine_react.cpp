@@ -58,6 +58,7 @@ ReactPipeline<PosT> make_pipeline(mcg_ctx* c, PosT* x, PosT* y, PosT* z, PosT* s
   p.R.ent64 = c->ent64.p;
   p.R.ent_box = c->ent_box.p;
   p.R.near_walls = c->near_walls.p;
+  p.R.ent_group = c->long_wall_lists ? c->ent_group.p : nullptr;
   p.queue = SlowQueue{c->queue.p, c->qcount.p, 0};
   p.teams = c->long_wall_lists;
   p.R.G = r.grid;

@@ -545,8 +545,8 @@ __global__ __launch_bounds__(256, 3) void k_move_light(ReactParams R, Snapshot<P
       const bool open = clear && hi[0] - lo[0] <= 1 && hi[1] - lo[1] <= 1 && hi[2] - lo[2] <= 1 &&
                         !walls_around(R.near_walls, subpart_index(R.P, pos));
       if (clear && !open) {
-        if (kF32) clear = all_walls_miss32(R.P, R.ent32, R.off, R.ent_box, R.F, R.band, pos, disp, lo, hi, near_plane);
-        else clear = all_walls_miss64(R.P, R.ent64, R.off, R.ent_box, pos, disp, lo, hi);
+        if (kF32) clear = all_walls_miss32(R.P, R.ent32, R.off, R.ent_box, R.ent_group, R.F, R.band, pos, disp, lo, hi, near_plane);
+        else clear = all_walls_miss64(R.P, R.ent64, R.off, R.ent_box, R.ent_group, pos, disp, lo, hi);
       }
       const bool walls_clear = clear;
       if (clear && (sp.flags & SPF_CAN_VOLVOL) && !(sp.flags & SPF_TARGET_ONLY)) {
@@ -679,7 +679,7 @@ __global__ __launch_bounds__(256, 3) void k_move_light(ReactParams R, Snapshot<P
               const uint32_t db = region_box(R.P, csp, cpq.x - R1, cpq.y - R1, cpq.z - R1, cpq.x + R1,
                                              cpq.y + R1, cpq.z + R1);
               const uint32_t e1 = R.off[csp + 1];
-              if (next_overlap<kLightOverlapGroup>(R.ent_box, R.off[csp], e1, db) < e1) {
+              if (light_overlap(R.ent_box, R.ent_group, R.off[csp], e1, db) < e1) {
                 clear = false;
                 break;
               }
