@@ -442,7 +442,8 @@ int mcg_get_walls(mcg_ctx* ctx, double* wall_constants, uint32_t* offsets, uint3
 int mcg_get_hit_trace(mcg_ctx* ctx, uint32_t* walls, uint32_t* counts, uint64_t capacity);
 
 /* Average device time of the dominant (diffuse) kernel over the last
- * mcg_step call, measured with HIP events on the engine's stream. */
+ * mcg_step call, measured with HIP events on the engine's stream or, with
+ * reaction classes, by the device's clock. */
 int mcg_last_kernel_time(mcg_ctx* ctx, double* avg_ms, uint32_t* launches);
 
 #ifdef __cplusplus
