@@ -190,12 +190,22 @@ void bin_walls(const PartitionParams& P, const std::vector<WallRec64>& walls, st
   for (size_t i = 0; i < pairs.size(); ++i) idx[i] = pairs[i].second;
 }
 
+// The first subpartition from s on that lists walls (the number of
+// subpartitions if none does): most of a partition's millions list none, and
+// the offsets do not decrease.
+static size_t next_listed(const std::vector<uint32_t>& off, size_t s) {
+  const size_t n3 = off.size() - 1;
+  if (s >= n3 || off[s + 1] != off[s]) return s;
+  const auto it = std::upper_bound(off.begin() + (ptrdiff_t)s + 1, off.end(), off[s]);
+  return it == off.end() ? n3 : (size_t)(it - off.begin()) - 1;
+}
+
 uint64_t entry_boxes(const PartitionParams& P, const std::vector<WallRec64>& walls, const std::vector<uint32_t>& off,
                      const std::vector<uint32_t>& idx, std::vector<uint32_t>& box) {
   box.assign(std::max<size_t>(idx.size(), 1), kBoxAll);
   const size_t n3 = off.size() - 1;
   uint64_t scanned = 0;
-  for (size_t s = 0; s < n3; ++s) {
+  for (size_t s = next_listed(off, 0); s < n3; s = next_listed(off, s + 1)) {
     scanned += (uint64_t)(off[s + 1] - off[s]) * (off[s + 1] - off[s]);
     for (uint32_t k = off[s]; k < off[s + 1]; ++k) {
       const WallRec64& w = walls[idx[k]];
@@ -211,8 +221,7 @@ void cells_near_walls(const PartitionParams& P, const std::vector<uint32_t>& off
   const int n = (int)P.n;
   const size_t n3 = off.size() - 1;
   bits.assign((n3 + 31) / 32, 0u);
-  for (size_t s = 0; s < n3; ++s) {
-    if (off[s + 1] == off[s]) continue;
+  for (size_t s = next_listed(off, 0); s < n3; s = next_listed(off, s + 1)) {
     const int x = (int)(s % P.n), y = (int)((s / P.n) % P.n), z = (int)(s / P.n2);
     for (int c = std::max(z - 1, 0); c <= std::min(z + 1, n - 1); ++c)
       for (int b = std::max(y - 1, 0); b <= std::min(y + 1, n - 1); ++b)
