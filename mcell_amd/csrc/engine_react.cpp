@@ -283,9 +283,7 @@ int run_iterations(mcg_ctx* c, ReactPipeline<PosT>& p, uint32_t first, uint32_t 
       if (r.surf_on)
         if (int st = surface_phase(c, it, barrier, err)) return st;
     }
-    unsigned long long ticks;
-    std::memcpy(&ticks, h + kHdrMoveTicks, sizeof(ticks));
-    const double total_ms = (double)ticks / c->clock_khz;
+    const double total_ms = (double)hdr_u64(h, kHdrMoveTicks) / c->clock_khz;
     if (n_in) drain_form_timed(r, form, (float)(total_ms - move_ms));
     move_ms = total_ms;
     r.last_form = form;
@@ -300,7 +298,7 @@ int run_iterations(mcg_ctx* c, ReactPipeline<PosT>& p, uint32_t first, uint32_t 
     c->n = std::min<uint64_t>(h[kHdrNumOut], cap);
     steps += h[kHdrSnapshot];
   }
-  const uint64_t reactions = num ? h[kHdrReacted] : 0u;
+  const uint64_t reactions = num ? hdr_u64(h, kHdrReacted) : 0u;
   r.log_count = reactions;
   if (propose_only) r.log_count = num ? h[kHdrLog] : 0u;
   if (stats) {

@@ -4,6 +4,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "device/header.h"
 #include "device/react_step.h"
 #include "kernels.h"
 
@@ -36,38 +37,6 @@ struct RxnEvent {
   uint32_t first_product_id, num_products;
 };
 static_assert(sizeof(RxnEvent) == 64, "event layout");
-
-// device counters
-enum : uint32_t {
-  kHdrNumOut = 0,         // used output slots (snapshot size + products)
-  kHdrProposals = 1,      // proposals of the current round
-  kHdrAccepted = 2,       // accepted reactions of the current phase
-  kHdrProductMovers = 3,  // products that move in this iteration
-  kHdrRerun0 = 4,         // movers queued for another round (two lists)
-  kHdrRerun1 = 5,
-  kHdrSnapshot = 6,       // molecules in the snapshot (the iteration's movers)
-  kHdrLog = 7,            // events logged (snapshot mode)
-  kHdrUnimolDue = 8,      // molecules whose unimolecular reaction falls in this phase
-  kHdrErr = 9,            // error bits (ERR_*) of the call's kernels
-  kHdrExd = 10,           // movers the full step deferred to its exact_disk pass
-  kHdrContinue = 11,      // movers of the phase that diffuse again in this iteration
-  kHdrSurfProps = 12,     // surface phase: moves to other tiles proposed in the round
-  kHdrSurfLose0 = 13,     // surface phase: movers whose tile went to a smaller id (two lists)
-  kHdrSurfLose1 = 14,
-  kHdrSurfCont0 = 15,     // surface phase: molecules that step again in this iteration (two lists)
-  kHdrSurfCont1 = 16,
-  kHdrOutBase = 17,       // products: the first output slot of the phase's new molecules
-  kHdrBatch = 18,         // products: the phase's reactions
-  kHdrReacted = 19,       // reactions of the call
-  kHdrLogBase = 20,       // products: reactions of the call before the phase
-  kHdrMoveStart = 22,     // (64 bits) device clock at the start of the iteration's first move
-  kHdrMoveTicks = 24,     // (64 bits) device clock ticks the call's first moves took
-  kHdrWords = 26,
-};
-// The host's copy of the counters, written by the kernels that end a round:
-// the words, then the number of the copy.
-constexpr uint32_t kHdrSeq = 32;
-constexpr uint32_t kHdrHostWords = 64;
 
 // Phases of up to this many reactions are put in order by one workgroup.
 constexpr uint32_t kSmallBatch = 1024;

@@ -154,11 +154,10 @@ __global__ __launch_bounds__(256) void k_scatter(RMolView<PosT> m, uint32_t n, c
 // The device clock of the first move's start and end (the drain's form is
 // chosen by it, and it is the time the ABI reports).
 __device__ __forceinline__ void move_started(uint32_t* hdr) {
-  *reinterpret_cast<unsigned long long*>(hdr + kHdrMoveStart) = wall_clock64();
+  hdr_u64(hdr, kHdrMoveStart) = wall_clock64();
 }
 __device__ __forceinline__ void move_ended(uint32_t* hdr) {
-  unsigned long long* const t = reinterpret_cast<unsigned long long*>(hdr + kHdrMoveStart);
-  t[1] += wall_clock64() - t[0];
+  hdr_u64(hdr, kHdrMoveTicks) += wall_clock64() - hdr_u64(hdr, kHdrMoveStart);
 }
 
 // The header to the host's copy, by one workgroup: the words, then -- once
@@ -991,22 +990,6 @@ __global__ __launch_bounds__(256) void k_first_ids(const uint64_t* __restrict__ 
   first_id[k] = next_id[rep] + pre[k] - pre[head[rep]];
 }
 
-// The header after the phase's reactions are in order (one thread): their
-// `total` new molecules take the output slots from the used ones on, never
-// past the capacity (k_products reports what does not fit).
-__device__ __forceinline__ void book_batch(uint32_t* __restrict__ hdr, uint32_t n, uint32_t total, uint32_t capacity) {
-  const uint32_t base = hdr[kHdrNumOut];
-  const uint64_t used = (uint64_t)base + total;
-  hdr[kHdrOutBase] = base;
-  hdr[kHdrNumOut] = used < capacity ? (uint32_t)used : capacity;
-  hdr[kHdrBatch] = n;
-  hdr[kHdrLogBase] = hdr[kHdrReacted];
-  hdr[kHdrReacted] += n;
-  hdr[kHdrAccepted] = 0;
-  hdr[kHdrUnimolDue] = 0;
-  hdr[kHdrProductMovers] = 0;
-}
-
 // Order, ids and slots of a phase of at most kSmallBatch reactions by one
 // workgroup: a reaction's place is the number of smaller keys (equal ones in
 // acceptance order, as the stable sort gives them).  One launch for the
@@ -1112,7 +1095,8 @@ __global__ __launch_bounds__(256) void k_products(ReactParams R, const uint32_t*
                                                   uint32_t* __restrict__ tiles, uint32_t* __restrict__ tile_id,
                                                   uint32_t* __restrict__ tile_consumed, uint32_t* __restrict__ kept) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t n = hdr[kHdrBatch], log_base = hdr[kHdrLogBase];
+  const uint32_t n = hdr[kHdrBatch];
+  const uint64_t row = log_row(hdr, k);
   // reaction counts, with every lane of the wave present
   wave_add_counters(R.rxn_counts, k < n ? reaction_counter(R, prop[sorted_slots[k]], key_replica(keys[k])) : ~0ull);
   if (k >= n) return;
@@ -1186,8 +1170,8 @@ __global__ __launch_bounds__(256) void k_products(ReactParams R, const uint32_t*
       if (R.born) R.born[slot] = moves_now ? ts + 1 : 0u;
       if (moves_now) mlist[atomicAdd(mcount, 1u)] = slot;
     }
-    if (log && log_base + k < log_cap) {
-      RxnEvent& e = log[log_base + k];
+    if (log && row < log_cap) {
+      RxnEvent& e = log[row];
       e.time = p.time;
       e.x = p.x;
       e.y = p.y;
@@ -1245,8 +1229,8 @@ __global__ __launch_bounds__(256) void k_products(ReactParams R, const uint32_t*
       mlist[atomicAdd(mcount, 1u)] = j;
     }
   }
-  if (log && log_base + k < log_cap) {
-    RxnEvent& e = log[log_base + k];
+  if (log && row < log_cap) {
+    RxnEvent& e = log[row];
     e.time = p.time;
     e.x = p.x;
     e.y = p.y;
