@@ -302,8 +302,14 @@ int run_iterations(mcg_ctx* c, ReactPipeline<PosT>& p, uint32_t first, uint32_t 
   r.log_count = reactions;
   if (propose_only) r.log_count = num ? h[kHdrLog] : 0u;
   if (stats) {
+    // the header's copy says nothing about the kernels' other writes: these
+    // reads are queued behind the kernels, on their stream
     unsigned long long ctr[CTR_WORDS] = {};
-    HIP_TRY(hipMemcpy(ctr, c->counters.p, sizeof(ctr), hipMemcpyDeviceToHost));
+    std::vector<uint32_t> q(kNumQueueShards, 0);
+    HIP_TRY(hipMemcpyAsync(ctr, c->counters.p, sizeof(ctr), hipMemcpyDeviceToHost, c->stream));
+    if (num && c->n)
+      HIP_TRY(hipMemcpyAsync(q.data(), c->qcount.p, kNumQueueShards * 4, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
     stats->molecule_steps = steps;
     stats->reactions = reactions;
     stats->wall_hits = ctr[CTR_REFLECTIONS];
@@ -311,9 +317,6 @@ int run_iterations(mcg_ctx* c, ReactPipeline<PosT>& p, uint32_t first, uint32_t 
     stats->settle_rounds = rounds;
     stats->drain_form = r.last_form;
     // movers of the last iteration that took the full step
-    std::vector<uint32_t> q(kNumQueueShards, 0);
-    if (num && c->n)
-      HIP_TRY(hipMemcpy(q.data(), c->qcount.p, kNumQueueShards * 4, hipMemcpyDeviceToHost));
     uint64_t hard = 0;
     for (uint32_t v : q) hard += v;
     stats->slow_path_last = (uint32_t)hard;

@@ -40,3 +40,23 @@ def test_order_and_ids_of_batches(gpu_available, n, replicas, precision):
     assert np.array_equal(eng.next_molecule_ids(), next_id)
     assert n < 20000 or (max(sizes) > 2048 and min(sizes) < 1024)  # both ways, and the sizes between them
     eng.close()
+
+
+def test_statistics_of_short_and_long_calls(gpu_available):
+    """The counters of 60 calls of one iteration add up to those of one call,
+    reflections of movers that then react among them (those are counted where
+    the claims are settled, the last thing an iteration does)."""
+    wl = W.receptor_sphere(n_l=20000, n_r=4000, n_t=2000, iterations=60, seed=8, down_fraction=0.0)
+    runs = []
+    for calls in ([(it, 1) for it in range(60)], [(0, 60)]):
+        eng = DiffuseReactEngine.from_workload(wl, seed=2)
+        st = [eng.step_raw(it, num, 100.0 - it) for it, num in calls]
+        total = {f: sum(getattr(s, f) for s in st) for f in ("molecule_steps", "wall_hits", "reactions",
+                                                             "transparent_crossings", "settle_rounds")}
+        m = eng.molecules()
+        runs.append((total, st[-1].slow_path_last, {k: v[np.argsort(m["id"])] for k, v in m.items()}))
+        eng.close()
+    assert runs[0][:2] == runs[1][:2]
+    assert runs[0][0]["reactions"] > 0 and runs[0][0]["wall_hits"] > 0
+    for k in runs[0][2]:
+        assert np.array_equal(runs[0][2][k], runs[1][2][k]), k
