@@ -55,6 +55,7 @@
 #include "device/react_step.h"
 #include "device/schedule.h"
 #include "kernels_react.h"
+#include "launch_sizes.h"
 
 namespace mcg {
 
@@ -121,7 +122,7 @@ __global__ __launch_bounds__(256) void k_scatter(RMolView<PosT> m, uint32_t n, c
                                                  uint32_t* __restrict__ qcount, uint32_t* __restrict__ hdr) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t threads = gridDim.x * blockDim.x;
-  for (uint32_t c = i; c <= num_cells; c += threads) cell_count[c] = 0;
+  for (uint64_t c = i; c <= num_cells; c += threads) cell_count[c] = 0;
   for (uint32_t q = i; q < kQueueShards; q += threads) qcount[q] = 0;
   if (i == 0) {
     const uint32_t live = cell_start[num_cells];
@@ -1356,8 +1357,8 @@ hipError_t ReactPipeline<PosT>::sort(hipStream_t s, uint32_t n_in, uint32_t num_
   size_t tmp = scan_tmp_bytes;
   hipError_t e = hipcub::DeviceScan::ExclusiveSum(scan_tmp, tmp, cell_count, cell_start, num_cells + 1, s);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_scatter<PosT>, blocks_for(n_in), dim3(256), 0, s, M, n_in, key, rank, cell_start, Sm,
-                     cell_count, num_cells, consumed, owner, kept, R.born, queue.count, hdr);
+  hipLaunchKernelGGL(k_scatter<PosT>, dim3(scatter_workgroups(n_in, num_cells)), dim3(256), 0, s, M, n_in, key, rank,
+                     cell_start, Sm, cell_count, num_cells, consumed, owner, kept, R.born, queue.count, hdr);
   return hipGetLastError();
 }
 

@@ -82,6 +82,26 @@ def test_waves_shares_of_the_light_pass(gpu_available, oracle_lib, n_a, n_b):
     eng.close()
 
 
+@pytest.mark.parametrize("n", [1, 100, 3000])
+def test_few_molecules_in_many_bins(gpu_available, oracle_lib, n):
+    """Some 4e5 bins for up to 6,000 molecules: the scatter's grid is sized by
+    the bins it clears, and every iteration finds them cleared."""
+    from oracle import pyoracle as po
+    wl = W.bimol_box(n_a=n, n_b=n, iterations=5, seed=4, subpartition_dimension=0.02)
+    eng = DiffuseReactEngine.from_workload(wl, seed=5, propose_only=True, log_capacity=1 << 12)
+    w = po.world_from_workload(wl, draw_mode=po.DRAW_PHILOX, seed=5)
+    w.set_snapshot(True)
+    w.set_barrier_interval(wl.barrier_interval)
+    st = eng.step_raw(0, 5, 5.0)
+    w.run(5)
+    m = eng.molecules()
+    assert len(m["id"]) == 2 * n and st.molecule_steps == 10 * n
+    # FP64 steps in the reference's operation order, as in the other snapshot comparisons
+    assert np.abs(m["pos"][np.argsort(m["id"])] - w.molecules()["pos"]).max() <= 1e-10
+    w.close()
+    eng.close()
+
+
 @pytest.mark.parametrize("n", [500, 20000])
 def test_list_moves_short_and_long(gpu_available, oracle_lib, n):
     """Second half steps of every molecule: lists below and above the length
