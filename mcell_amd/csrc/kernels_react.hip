@@ -1508,25 +1508,34 @@ hipError_t ReactPipeline<PosT>::products(hipStream_t s, uint32_t max_acc, uint32
   return hipGetLastError();
 }
 
-// The continuing movers after the list's *count entries, by one workgroup
-// (one launch instead of two; lists of tens of thousands take it a few us).
+// The continuing movers after the list's *dst_count entries (from its start
+// unless after_products).  A lone workgroup also moves the counts; after a
+// grid, k_take_count does (append_workgroups, launch_sizes.h).
+__device__ __forceinline__ void take_count(uint32_t* src_count, uint32_t* dst_count, uint32_t after_products) {
+  *dst_count = (after_products ? *dst_count : 0u) + *src_count;
+  *src_count = 0;
+}
 __global__ __launch_bounds__(1024) void k_append_list(const uint32_t* __restrict__ src, uint32_t* src_count,
                                                       uint32_t* __restrict__ dst, uint32_t* dst_count,
                                                       uint32_t after_products) {
   const uint32_t n = *src_count, base = after_products ? *dst_count : 0u;
-  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) dst[base + i] = src[i];
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) dst[base + i] = src[i];
+  if (gridDim.x > 1) return;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    *dst_count = base + n;
-    *src_count = 0;
-  }
+  if (threadIdx.x == 0) take_count(src_count, dst_count, after_products);
+}
+__global__ void k_take_count(uint32_t* src_count, uint32_t* dst_count, uint32_t after_products) {
+  if (threadIdx.x == 0) take_count(src_count, dst_count, after_products);
 }
 
 template <typename PosT>
 hipError_t ReactPipeline<PosT>::continuations(hipStream_t s, uint32_t max_cont, bool after_products) {
   if (max_cont == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_append_list, dim3(1), dim3(1024), 0, s, clist, hdr + kHdrContinue, mlist,
-                     hdr + kHdrProductMovers, after_products ? 1u : 0u);
+  const uint32_t grid = append_workgroups(max_cont), after = after_products ? 1u : 0u;
+  hipLaunchKernelGGL(k_append_list, dim3(grid), dim3(grid > 1 ? 256 : 1024), 0, s, clist, hdr + kHdrContinue, mlist,
+                     hdr + kHdrProductMovers, after);
+  if (grid > 1)
+    hipLaunchKernelGGL(k_take_count, dim3(1), dim3(64), 0, s, hdr + kHdrContinue, hdr + kHdrProductMovers, after);
   return hipGetLastError();
 }
 

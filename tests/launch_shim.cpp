@@ -5,5 +5,6 @@
 extern "C" {
 
 uint32_t scatter(uint32_t molecules, uint32_t bins) { return mcg::scatter_workgroups(molecules, bins); }
+uint32_t append(uint32_t entries) { return mcg::append_workgroups(entries); }
 
 }  // extern "C"

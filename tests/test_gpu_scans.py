@@ -102,10 +102,11 @@ def test_few_molecules_in_many_bins(gpu_available, oracle_lib, n):
     eng.close()
 
 
-@pytest.mark.parametrize("n", [500, 20000])
+@pytest.mark.parametrize("n", [500, 16384, 16385, 20000, 300001])
 def test_list_moves_short_and_long(gpu_available, oracle_lib, n):
     """Second half steps of every molecule: lists below and above the length
-    up to which the list moves take the large pool at once."""
+    up to which the list moves take the large pool at once, and those up to
+    which one workgroup copies the list (16,384)."""
     from oracle import pyoracle as po
     wl = W.with_time_steps(W.free_diffusion_box(scale=n / 10000, iterations=4), [0.5])
     eng = DiffuseReactEngine.from_workload(wl)

@@ -20,7 +20,7 @@ def shim(tmp_path_factory):
     subprocess.check_call([cxx, "-O1", "-std=c++17", "-fPIC", "-shared", os.path.join(HERE, "launch_shim.cpp"),
                            "-o", str(out)])
     lib = ctypes.CDLL(str(out))
-    lib.scatter.restype = ctypes.c_uint32
+    lib.scatter.restype = lib.append.restype = ctypes.c_uint32
     return lib
 
 
@@ -32,3 +32,12 @@ def test_scatter_clears_the_bins_with_enough_threads(shim, molecules, bins):
     assert wg >= own
     assert wg >= 2048 or wg * 256 * 16 >= bins     # at most 16 bins a thread, or the whole chip
     assert wg == own or wg <= 2048 and (wg - 1) * 256 * 16 < bins  # no more than that takes
+
+
+@pytest.mark.parametrize("entries", [1, 256, 16384, 16385, 10 ** 6, 0xFFFFFFFF])
+def test_long_lists_are_copied_by_a_grid(shim, entries):
+    wg = shim.append(ctypes.c_uint32(entries))
+    if wg == 1:
+        assert entries <= 16 * 1024  # sixteen turns of the lone workgroup of 1,024
+    else:
+        assert wg == 2048 or (wg - 1) * 256 < entries <= wg * 256
