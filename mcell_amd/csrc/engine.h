@@ -9,6 +9,7 @@
 #include "kernels.h"
 #include "kernels_react.h"
 #include "kernels_surface.h"
+#include "launch_sizes.h"
 
 namespace mcg {
 
@@ -104,11 +105,7 @@ struct ReactState {
   uint32_t* hdr_host = nullptr;        // pinned mirror of hdr, written by the kernels (kHdrSeq: the copy's number)
   uint32_t* hdr_host_d = nullptr;      // its device address
   uint32_t hdr_seq = 0;                // number of the last copy asked for
-  // launch sizes: what the last rounds of each kind led to expect ([0]: list
-  // moves, [1], [2]: an iteration's first moves by the drain's form), never
-  // what a kernel may do
-  static constexpr uint32_t kUnknown = 1u << 30;
-  uint32_t expect_props[3] = {kUnknown, kUnknown, kUnknown}, expect_deferred[3] = {kUnknown, kUnknown, kUnknown};
+  RoundSizes sizes;                    // launch sizes, never what a kernel may do
   bool volume_products = false;        // some class makes volume molecules or keeps a unimolecular reactant
   // the drain's form (1 exact_disk in place, 2 deferred): fixed by a flag,
   // else timed on the first iterations after the geometry or the molecules

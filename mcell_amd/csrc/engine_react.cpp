@@ -186,26 +186,24 @@ void drain_form_timed(ReactState& r, uint32_t form, float ms) {
 // settling kernels read the actual count on the device, so the header is
 // read once per round, after the claims are settled.
 template <typename PosT>
-int settle_rounds(mcg_ctx* c, ReactPipeline<PosT>& p, bool snapshot_src, double barrier, uint32_t* err,
+int settle_rounds(mcg_ctx* c, ReactPipeline<PosT>& p, uint32_t phase, double barrier, uint32_t* err,
                   uint32_t& rounds, uint32_t max_props, uint32_t form, bool timed) {
   const uint32_t* const h = c->rx.hdr_host;
-  uint32_t kind = snapshot_src ? form : 0u;  // an iteration's first moves, or a list's
+  RoundSizes& sizes = c->rx.sizes;
   for (uint32_t r = 0;; ++r) {
     if (r > 100000) return fail(MCG_E_LIMIT, "reaction settling did not converge");
     uint32_t* rl = (r & 1) ? p.rlist1 : p.rlist0;
     uint32_t* rc = p.hdr + ((r & 1) ? kHdrRerun1 : kHdrRerun0);
-    p.expect_props = c->rx.expect_props[kind];
+    p.expect_props = sizes.expect_props(phase, form, r, max_props);
     HIP_TRY(p.settle(c->stream, max_props, rl, rc, timed && r == 0, ++c->rx.hdr_seq));
     if (int st = wait_hdr(c)) return st;
-    c->rx.expect_props[kind] = h[kHdrProposals];
-    c->rx.expect_deferred[kind] = h[kHdrExd];
-    kind = 0;
+    if (r == 0) sizes.first_round(phase, form, h[kHdrProposals], h[kHdrExd]);
     if (h[kHdrProposals] == 0) return MCG_OK;
     ++rounds;
     const uint32_t nr = h[(r & 1) ? kHdrRerun1 : kHdrRerun0];
     if (nr == 0) return MCG_OK;
-    p.expect_deferred = c->rx.expect_deferred[0];
-    HIP_TRY(p.move(c->stream, snapshot_src, rl, rc, nr, barrier, false, err));
+    p.expect_deferred = sizes.expect_deferred(phase, form, r + 1, nr);
+    HIP_TRY(p.move(c->stream, phase == 0, rl, rc, nr, barrier, false, err));
     max_props = nr;
   }
 }
@@ -236,21 +234,22 @@ int run_iterations(mcg_ctx* c, ReactPipeline<PosT>& p, uint32_t first, uint32_t 
     HIP_TRY(p.sort(c->stream, n_in, r.num_cells, err));
     const uint32_t form = drain_form_for(c);
     p.drain_inline = form == 1;
-    p.expect_deferred = r.expect_deferred[form];
+    p.expect_deferred = r.sizes.expect_deferred(0, form, 0, n_in);
     HIP_TRY(p.move(c->stream, true, nullptr, p.cell_start + r.num_cells, n_in, barrier, propose_only, err));
     const bool timed = n_in != 0;
     if (propose_only) {
       HIP_TRY(p.log_proposals(c->stream, n_in, it, r.log.p, p.hdr + kHdrLog, (uint32_t)r.log_cap));
       HIP_TRY(p.publish(c->stream, timed, ++r.hdr_seq));
       if (int st = wait_hdr(c)) return st;
-      r.expect_deferred[form] = h[kHdrExd];
+      r.sizes.first_round(0, form, h[kHdrProposals], h[kHdrExd]);
     } else {
-      bool snapshot_src = true;
+      // phase 0: the snapshot's moves; then those of products and of movers
+      // that diffuse again
       uint32_t phase_movers = n_in;
-      for (;;) {
-        if (int st = settle_rounds(c, p, snapshot_src, barrier, err, rounds, phase_movers, form, timed && snapshot_src))
+      for (uint32_t phase = 0;; ++phase) {
+        if (int st = settle_rounds(c, p, phase, barrier, err, rounds, phase_movers, form, timed && phase == 0))
           return st;
-        if (!snapshot_src) steps += h[kHdrProductMovers];
+        if (phase) steps += h[kHdrProductMovers];
         // the phase's reactions (at most: a due unimolecular event only
         // happens to a molecule that is still there) and the movers that
         // diffuse again in this iteration
@@ -264,7 +263,7 @@ int run_iterations(mcg_ctx* c, ReactPipeline<PosT>& p, uint32_t first, uint32_t 
           if (int st = wait_hdr(c)) return st;
           na = h[kHdrAccepted];
         }
-        HIP_TRY(p.products(c->stream, na, (uint32_t)cap, r.log.p, (uint32_t)r.log_cap, snapshot_src, err));
+        HIP_TRY(p.products(c->stream, na, (uint32_t)cap, r.log.p, (uint32_t)r.log_cap, phase == 0, err));
         HIP_TRY(p.continuations(c->stream, nc, na != 0));
         // the next phase's movers: the products that move in this iteration,
         // then the movers that diffuse again (how many the device counts)
@@ -274,9 +273,8 @@ int run_iterations(mcg_ctx* c, ReactPipeline<PosT>& p, uint32_t first, uint32_t 
           if (int st = wait_hdr(c)) return st;
           break;
         }
-        snapshot_src = false;
         phase_movers = (uint32_t)std::min<uint64_t>(movers, cap);
-        p.expect_deferred = r.expect_deferred[0];
+        p.expect_deferred = r.sizes.expect_deferred(phase + 1, form, 0, phase_movers);
         HIP_TRY(p.move(c->stream, false, p.mlist, p.hdr + kHdrProductMovers, phase_movers, barrier, false, err));
       }
       // the surface molecules' steps follow the volume phases

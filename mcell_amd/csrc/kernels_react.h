@@ -67,9 +67,9 @@ struct ReactPipeline {
   size_t scan_tmp_bytes;
 
   uint32_t* hdr_host;  // the host copy, as the device sees it
-  // what earlier rounds led to expect (launch sizes only)
-  uint32_t expect_props;     // proposals of the round
-  uint32_t expect_deferred;  // movers the round's move defers
+  // what the round is expected to bring (launch sizes only; RoundSizes)
+  uint32_t expect_props;     // proposals
+  uint32_t expect_deferred;  // movers its move defers
 
   static size_t scan_bytes(uint32_t num_cells, uint32_t capacity);
   // the snapshot in bin order; also clears the iteration's counters, claim

@@ -1435,10 +1435,10 @@ hipError_t ReactPipeline<PosT>::move(hipStream_t s, bool snapshot_src, const uin
                          count, species, barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err, ulist,
                          hdr + kHdrUnimolDue, xlist, hdr + kHdrExd);
     // the deferred steps, with the large pool (mostly none: a grid for twice
-    // the last round's)
-    const dim3 grid = move_grid(std::min(max_movers, 64 + 2 * expect_deferred));
-    hipLaunchKernelGGL((k_move<PosT, exd::kPool, TeamT>), grid, dim3(256), 0, s, R, S, src, M, xlist, hdr + kHdrExd, species, barrier, po, prop, plist, hdr + kHdrProposals, owner, tile_owner, err,
-                       ulist, hdr + kHdrUnimolDue, nullptr, nullptr);
+    // the expected ones)
+    hipLaunchKernelGGL((k_move<PosT, exd::kPool, TeamT>), move_grid(room_for(expect_deferred, max_movers)), dim3(256),
+                       0, s, R, S, src, M, xlist, hdr + kHdrExd, species, barrier, po, prop, plist, hdr + kHdrProposals,
+                       owner, tile_owner, err, ulist, hdr + kHdrUnimolDue, nullptr, nullptr);
   };
   if (teams) full_steps(Team{1, 0});
   else full_steps(Solo{});
@@ -1455,7 +1455,7 @@ hipError_t ReactPipeline<PosT>::settle(hipStream_t s, uint32_t max_props, uint32
     return hipGetLastError();
   }
   // grid-stride over the device's proposal count; max_props bounds it
-  const dim3 grid = dim3(std::min<uint32_t>(blocks_for(std::min(max_props, 2 * expect_props)).x, 1024u));
+  const dim3 grid = dim3(std::min<uint32_t>(blocks_for(room_for(expect_props, max_props)).x, 1024u));
   hipLaunchKernelGGL(k_accept, grid, dim3(256), 0, s, A, timed ? 1u : 0u);
   hipLaunchKernelGGL(k_requeue, grid, dim3(256), 0, s, A);
   return publish(s, false, seq);
