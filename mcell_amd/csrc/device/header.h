@@ -20,9 +20,8 @@ enum : uint32_t {
   kHdrErr = 9,            // error bits (ERR_*) of the call's kernels
   kHdrExd = 10,           // movers the full step deferred to its exact_disk pass
   kHdrContinue = 11,      // movers of the phase that diffuse again in this iteration
-  kHdrSurfProps = 12,     // surface phase: moves to other tiles proposed in the round
-  kHdrSurfLose0 = 13,     // surface phase: movers whose tile went to a smaller id (two lists)
-  kHdrSurfLose1 = 14,
+  kHdrSurfChanged = 12,   // surface phase: movers whose end the round changed
+  kHdrSurfMovers = 13,    // surface phase: the first pass's movers
   kHdrSurfCont0 = 15,     // surface phase: molecules that step again in this iteration (two lists)
   kHdrSurfCont1 = 16,
   kHdrOutBase = 17,       // products: the first output slot of the phase's new molecules

@@ -141,8 +141,10 @@ struct ReactState {
   std::vector<double> tu_host, tv_host, ttoff_host, tbirth_host;
   bool surf_on = false;  // some surface species diffuses: grids on every wall, the surface phase runs
   DevBuf<double> tu, tv, ttoff, tbirth, spu, spv;
-  DevBuf<unsigned long long> sclaim;
-  DevBuf<uint32_t> sprop, splist, slose0, slose1, sdone, scont0, scont1;
+  DevBuf<unsigned long long> sclaim0, sclaim1;
+  DevBuf<uint32_t> sdest0, sdest1, sflags, smoved, smovers, sdone, scont0, scont1;
+  uint32_t surf_code = 0;                   // the claims' code of the last round; 0: the claims are to be cleared
+  uint32_t surf_movers = RoundSizes::kUnknown;  // the last iteration's (launch sizes only)
   DevBuf<WallEdgeRec> edges_d;
   // reaction log of the last mcg_step call
   DevBuf<RxnEvent> log;

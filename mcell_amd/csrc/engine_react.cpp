@@ -892,11 +892,11 @@ int sync_tiles_to_device(mcg_ctx* c, bool allow_alloc) {
     if (r.tu.n != nt) {
       if (!allow_alloc) return fail(MCG_E_STATE, "surface molecules on new walls need tile buffers");
       if (r.tu.alloc(nt) || r.tv.alloc(nt) || r.ttoff.alloc(nt) || r.tbirth.alloc(nt) || r.spu.alloc(nt) ||
-          r.spv.alloc(nt) || r.sclaim.alloc(nt) || r.sprop.alloc(nt) || r.splist.alloc(nt) ||
-          r.slose0.alloc(nt) || r.slose1.alloc(nt) || r.sdone.alloc(nt) || r.scont0.alloc(nt) ||
-          r.scont1.alloc(nt))
+          r.spv.alloc(nt) || r.sclaim0.alloc(nt) || r.sclaim1.alloc(nt) || r.sdest0.alloc(nt) ||
+          r.sdest1.alloc(nt) || r.sflags.alloc(nt) || r.smoved.alloc(nt) || r.smovers.alloc(nt) ||
+          r.sdone.alloc(nt) || r.scont0.alloc(nt) || r.scont1.alloc(nt))
         return fail(MCG_E_NOMEM, "surface phase buffers");
-      HIP_TRY(launch_fill_claims(c->stream, r.sclaim.p, (uint32_t)nt));
+      r.surf_code = 0;
     }
     if (r.sdone.n == nt) {
       // molecules keep their slots' stamps only within an iteration
@@ -1048,11 +1048,10 @@ int surface_phase(mcg_ctx* c, uint32_t iteration, double barrier, uint32_t* err)
   P.tv = r.tv.p;
   P.ttoff = r.ttoff.p;
   P.birth = r.tbirth.p;
-  P.claim = r.sclaim.p;
-  P.prop = r.sprop.p;
   P.pu = r.spu.p;
   P.pv = r.spv.p;
-  P.plist = r.splist.p;
+  P.flags = r.sflags.p;
+  P.moved_id = r.smoved.p;
   P.done = r.sdone.p;
   P.hdr = r.hdr.p;
   P.err = err;
@@ -1064,35 +1063,54 @@ int surface_phase(mcg_ctx* c, uint32_t iteration, double barrier, uint32_t* err)
   P.stamp_base = ((iteration + 1u) % 0x0FFFFFFFu) << 4;
   P.barrier = barrier;
   const uint32_t n_all = r.total_tiles * R;
-  uint32_t* lists[2] = {r.slose0.p, r.slose1.p};
-  const uint32_t words[2] = {kHdrSurfLose0, kHdrSurfLose1};
   uint32_t* conts[2] = {r.scont0.p, r.scont1.p};
   const uint32_t cwords[2] = {kHdrSurfCont0, kHdrSurfCont1};
+  unsigned long long* claims[2] = {r.sclaim0.p, r.sclaim1.p};
+  uint32_t* dests[2] = {r.sdest0.p, r.sdest1.p};
   // pass k: the molecules' k-th steps of the iteration; the first over every
-  // slot, the others over the molecules the previous pass listed
-  const uint32_t* in_list = nullptr;
-  const uint32_t* in_count = nullptr;
-  uint32_t n_in = n_all;
+  // slot (which lists the movers), the others over the molecules the previous
+  // pass listed
+  P.list = r.smovers.p;
+  P.count = r.hdr.p + kHdrSurfMovers;
+  uint32_t movers = room_for(r.surf_movers, n_all);
   for (uint32_t pass = 0; pass < kSurfPasses; ++pass) {
     P.pass = pass;
     P.clist = conts[pass & 1];
     P.ccount = r.hdr.p + cwords[pass & 1];
-    HIP_TRY(launch_clear_words(c->stream, r.hdr.p, kHdrSurfProps, words[0], cwords[pass & 1]));
-    HIP_TRY(surf_round(c->stream, P, in_list, in_count, n_in, lists[0], r.hdr.p + words[0]));
-    for (uint32_t round = 0;; ++round) {
-      // (the copy clears the counter of the list the next round appends to)
-      HIP_TRY(launch_publish(c->stream, r.hdr.p, r.hdr_host_d, ++r.hdr_seq, false, words[(round + 1) & 1]));
-      if (int st = wait_hdr(c)) return st;
-      const uint32_t nl = h[words[round & 1]];
-      if (nl == 0) break;
-      if (round > 100000) return fail(MCG_E_LIMIT, "surface moves did not settle");
-      HIP_TRY(surf_round(c->stream, P, lists[round & 1], r.hdr.p + words[round & 1], nl, lists[(round + 1) & 1],
-                         r.hdr.p + words[(round + 1) & 1]));
+    HIP_TRY(launch_clear_words(c->stream, r.hdr.p, kHdrSurfChanged, pass ? kHdrSurfChanged : kHdrSurfMovers,
+                               cwords[pass & 1]));
+    if (r.surf_code <= kSurfMaxRounds) {
+      for (unsigned long long* p : claims) HIP_TRY(launch_fill_claims(c->stream, p, n_all));
+      r.surf_code = kSurfFirstCode + 1;
     }
-    n_in = h[cwords[pass & 1]];
-    if (n_in == 0) return MCG_OK;
-    in_list = conts[pass & 1];
-    in_count = r.hdr.p + cwords[pass & 1];
+    for (uint32_t round = 0;;) {
+      // a batch of rounds, and the moves if its last changed nothing: three
+      // at first (2,000 molecules on 46,080 tiles: the second round changes
+      // some end in four passes of five, the third in few), then two
+      const uint32_t last = round + (round ? 1 : 2);
+      for (; round <= last; ++round) {
+        P.round = round;
+        P.check = round == last;
+        P.code_prev = round ? r.surf_code : 0u;
+        P.code = --r.surf_code;
+        P.claim = claims[round & 1];
+        P.claim_prev = claims[(round + 1) & 1];
+        P.dest = dests[round & 1];
+        P.dest_prev = dests[(round + 1) & 1];
+        HIP_TRY(surf_round(c->stream, P, pass == 0 && round == 0 ? n_all : 0u, movers));
+      }
+      HIP_TRY(surf_commit(c->stream, P, movers));
+      // (the copy clears the count of changes)
+      HIP_TRY(launch_publish(c->stream, r.hdr.p, r.hdr_host_d, ++r.hdr_seq, false, kHdrWords));
+      if (int st = wait_hdr(c)) return st;
+      if (h[kHdrSurfChanged] == 0) break;
+      if (round >= kSurfMaxRounds) return fail(MCG_E_LIMIT, "surface moves did not settle");
+    }
+    if (pass == 0) r.surf_movers = h[kHdrSurfMovers];
+    movers = h[cwords[pass & 1]];
+    if (movers == 0) return MCG_OK;
+    P.list = conts[pass & 1];
+    P.count = r.hdr.p + cwords[pass & 1];
   }
   return MCG_OK;  // a molecule listed past the last pass raised ERR_PASSES
 }

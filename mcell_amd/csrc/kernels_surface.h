@@ -23,14 +23,20 @@ struct SurfPhase {
   double* tv;
   double* ttoff;                             // diffusion-time offsets from the iteration's start
   double* birth;                             // birthdays (absolute)
-  unsigned long long* claim;                 // per slot: smallest order key proposing to move there
-  uint32_t* prop;                            // per mover slot: the slot it proposes
-  double* pu;                                // the proposed position
+  // Per slot, of this round and of the one before it: the smallest order key
+  // of the movers whose step ends on the slot's tile, under the round's code
+  // (kernels_surface.hip), ...
+  unsigned long long *claim, *claim_prev;
+  uint32_t *dest, *dest_prev;                // ... and the slot a mover's step ends on (kSurfNotDue: none this iteration)
+  double* pu;                                // the position it ends at
   double* pv;
-  uint32_t* plist;                           // proposing slots of the round
-  // per slot: the iteration's stamp once its molecule's step of a pass is
-  // over, stamp_base | kDoneFinal when it has no further step in the
-  // iteration, stamp_base | (pass + 1) when it steps again in the next pass
+  uint32_t* flags;                           // per mover slot: what its step met; while moving, the tile word
+  uint32_t* moved_id;                        // per mover slot: the one tile it was turned away from; while moving, the id
+  uint32_t* list;                            // the pass's movers
+  const uint32_t* count;
+  // per slot: the iteration's stamp, stamp_base | kDoneFinal when its
+  // molecule has no further step in the iteration, stamp_base | (pass + 1)
+  // when it steps again in the next pass
   uint32_t* done;
   uint32_t* clist;                           // slots of the molecules that step again (next pass)
   uint32_t* ccount;
@@ -42,18 +48,27 @@ struct SurfPhase {
   uint32_t pass;                             // the pass (a molecule's n-th step in the iteration)
   uint32_t stamp_base;                       // ((iteration + 1) mod 2^28) << 4
   double barrier;                            // time up to the next barrier from the iteration's start
+  uint32_t round;                            // the round of the pass
+  uint32_t check;                            // whether the round counts the movers whose end it changed
+  uint32_t code, code_prev;                  // the claims' codes of this round and the one before (0: none)
 };
 
 constexpr uint32_t kDoneFinal = 15u;
 constexpr uint32_t kSurfPasses = 8;          // steps per iteration (time steps of at least 1/8)
+constexpr uint32_t kSurfNotDue = 0xFFFFFFFFu;
+// Codes of a claim word's high 31 bits: newer rounds have smaller ones, down
+// to 1; a pass starts with enough of them left for its rounds.
+constexpr uint32_t kSurfFirstCode = 0x7FFFFFFEu;
+constexpr uint32_t kSurfMaxRounds = 100000;
 
-// One round of a pass over `list` (every slot when null: the first pass's
-// first round; else the molecules stepping again in this pass, or the
-// movers of the previous round that lost a tile or waited), then the
-// claims' settlement: winners move, losers are listed for the next round.
-// The counters of the proposals and of lose_list are zero on entry.
-hipError_t surf_round(hipStream_t s, const SurfPhase& P, const uint32_t* list, const uint32_t* count,
-                      uint32_t max_movers, uint32_t* lose_list, uint32_t* lose_count);
+// One round of a pass: every mover's step, given the ends of the movers ahead
+// of it that the round before worked out.  The first pass's first round
+// (n_all > 0) looks at every slot and lists the movers; max_movers bounds or
+// estimates them.  A round with P.check set (never the first) counts the
+// movers whose end it changed in hdr[kHdrSurfChanged], which is zero on entry.
+hipError_t surf_round(hipStream_t s, const SurfPhase& P, uint32_t n_all, uint32_t max_movers);
+// The movers move, if the last round, a checked one, changed nothing.
+hipError_t surf_commit(hipStream_t s, const SurfPhase& P, uint32_t max_movers);
 hipError_t launch_fill_done(hipStream_t s, uint32_t* done, uint32_t n);
 // Zeroes three words of the header.
 hipError_t launch_clear_words(hipStream_t s, uint32_t* hdr, uint32_t a, uint32_t b, uint32_t c);

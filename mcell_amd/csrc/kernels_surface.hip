@@ -1,22 +1,41 @@
 // The surface phase of an iteration: every surface molecule of a species
 // that diffuses takes its step (diffuse_surf_molecule,
-// diffuse_react_event.cpp:1071-1246) after the iteration's volume phases,
-// one thread per tile slot.  A molecule whose end point lies on its own tile
-// moves there at once; one whose end point lies on another tile that is
-// free proposes the move and claims the tile (smallest id wins); a tile
-// that is taken makes it draw again (move_sm_on_same_triangle /
-// move_sm_to_new_triangle, diffusion_utils.inl:453-548).  Winners move,
-// losers repeat their step from the start of their stream in the next
-// round, seeing the tiles the winners took (and left).  The reference moves
-// molecules one at a time in id order, so a tile whose occupant has a
-// smaller id and has not yet taken its step may still be vacated: a mover
-// that meets one waits for the next round instead of drawing again.
+// diffuse_react_event.cpp:1071-1246) after the iteration's volume phases.  A
+// molecule whose end point lies on its own tile moves within it; one whose
+// end point lies on another tile moves there if that tile is free, else it
+// draws again (move_sm_on_same_triangle / move_sm_to_new_triangle,
+// diffusion_utils.inl:453-548).
+//
+// The reference moves one molecule at a time: those whose diffusion time
+// falls on the iteration's start by id, then the delayed ones by id
+// (diffuse_molecules, diffuse_react_event.cpp:66-113).  So a tile is taken at
+// a molecule's turn if
+//   * its occupant at the start of the pass does not step in it, or is behind
+//     in the order, or is ahead and its step ends on that same tile, or
+//   * the step of some molecule ahead in the order ends on it.
+// A step therefore depends on where the steps of molecules ahead of it end,
+// and on nothing else that moves.  Rounds of all steps at once solve for the
+// ends: every round works each step out from the ends of the round before
+// (before the first, every molecule ends where it is); the first molecule's
+// is right after one round, and each round makes right every step whose
+// molecules ahead were, so a round that changes no end has found the
+// sequential order's.  Only then do the movers move (two launches: all
+// leave their tiles, then all arrive), so that within a round nothing is
+// written that another molecule's step reads.  Most steps meet no molecule
+// ahead and are worked out once, unless the tile they end on gets a claim
+// from ahead; a step that was turned away by one occupant ahead is worked out
+// again when that occupant's end leaves the tile free, and any other step
+// that met molecules ahead in every round (kSurfOneAhead, kSurfAhead).
+//
+// Claims: per slot the smallest order key among the movers that end there in
+// a round, by atomicMin of code << 33 | key.  The code falls from round to
+// round, so the claims of older rounds never stand in the way and need no
+// clearing; two arrays take turns.
+//
 // Species with time steps below one iteration step again in further passes
-// of the phase (the reference's later diffuse actions of the iteration),
-// each pass reading the next pass of the molecule's stream.  The order the
-// waits and claims follow is the reference's: molecules whose diffusion
-// time falls on the iteration's start first, then the delayed ones
-// (diffuse_molecules, diffuse_react_event.cpp:66-113), each group by id.
+// of the phase (the reference's later diffuse actions of the iteration), in
+// the first pass's order, each pass reading the next pass of the molecule's
+// stream.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -58,12 +77,12 @@ struct SurfTiming {
 };
 
 __device__ __forceinline__ SurfTiming surf_timing(const SurfPhase& P, const SpeciesRec& sp, uint32_t tw, double toff,
-                                                  uint32_t s) {
+                                                  double birth) {
   SurfTiming r;
   double max_time = P.barrier - toff;
   r.mature = false;
   if (!(tw & kTileMature) && sp.time_step > 1.0) {
-    const double age_dependent_max_time = 1.0 + 0.2 * (((double)P.iteration + toff) - P.birth[s]);
+    const double age_dependent_max_time = 1.0 + 0.2 * (((double)P.iteration + toff) - birth);
     if (max_time > age_dependent_max_time) max_time = age_dependent_max_time;
     r.mature = age_dependent_max_time > sp.time_step;
   }
@@ -106,41 +125,63 @@ __device__ __forceinline__ void surf_step_over(const SurfPhase& P, uint32_t s, u
   }
 }
 
-// One surface molecule's step, for the slots of `list` (every slot when
-// list is null: the first round of the first pass, which also books
-// molecules due in later iterations).
-__global__ __launch_bounds__(256) void k_surf_move(SurfPhase P, const uint32_t* __restrict__ list,
-                                                   const uint32_t* __restrict__ count, uint32_t n_all,
-                                                   uint32_t* __restrict__ lose_list,
-                                                   uint32_t* __restrict__ lose_count) {
-  const uint32_t n = list ? *count : n_all;
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t s = list ? list[i] : i;
-  const uint32_t tw = P.tiles[s];
-  if (tw == kTileEmpty) return;
+// what a step met of the molecules ahead in the order (error bits follow):
+// the occupant of moved_id[s]'s tile alone, which stays there, or more
+constexpr uint32_t kSurfAhead = 1u, kSurfOneAhead = 2u, kSurfErrShift = 2u;
+constexpr unsigned long long kClaimKey = (1ull << 33) - 1;
+
+__device__ __forceinline__ bool surf_moves(const SpeciesRec& sp) {
+  return (sp.flags & SPF_SURFACE) && sp.space_step > 0;
+}
+__device__ __forceinline__ const SpeciesRec& surf_species(const SurfPhase& P, uint32_t rep, uint32_t tw) {
+  return P.species.rec[rep * P.species.stride + tile_species(tw)];
+}
+
+// Whether a step of the round before ends on slot ts, of a molecule ahead of
+// `key` in the order.
+__device__ __forceinline__ bool claimed_ahead(const SurfPhase& P, uint32_t ts, unsigned long long key) {
+  const unsigned long long c = P.claim_prev[ts];
+  return (uint32_t)(c >> 33) == P.code_prev && (c & kClaimKey) < key;
+}
+
+// Whether the tile of slot ts, whose occupant steps ahead of `key`, is taken.
+__device__ __forceinline__ bool still_taken(const SurfPhase& P, uint32_t ts, unsigned long long key) {
+  return P.round == 0 || P.dest_prev[ts] == ts || claimed_ahead(P, ts, key);
+}
+
+// Whether the tile of slot ts is taken at the turn of the molecule in slot s
+// with order key `key`, as far as the round before knows.
+__device__ __forceinline__ bool tile_taken(const SurfPhase& P, uint32_t s, uint32_t rep, uint32_t ts,
+                                           unsigned long long key, uint32_t& flags) {
+  const uint32_t occ = P.tiles[ts];
+  if (occ != kTileEmpty) {
+    if (!surf_moves(surf_species(P, rep, occ))) return true;
+    const double toff = P.ttoff[ts];
+    const bool steps = P.pass == 0 ? ready_this_iteration(P.iteration, toff) : P.done[ts] == (P.stamp_base | P.pass);
+    if (!steps || surf_key(surf_delayed(P, occ, toff), P.tile_id[ts]) > key) return true;
+    const bool taken = still_taken(P, ts, key);
+    flags |= taken && !flags ? kSurfOneAhead : kSurfAhead;
+    if (flags == kSurfOneAhead) P.moved_id[s] = ts;
+    return taken;
+  }
+  if (!claimed_ahead(P, ts, key)) return false;
+  flags |= kSurfAhead;
+  return true;
+}
+
+// The step of the molecule in slot s: the slot it ends on, the position there
+// in pu, pv.
+__device__ __forceinline__ uint32_t surf_step(const SurfPhase& P, uint32_t s, uint32_t tw, double toff,
+                                              unsigned long long key, uint32_t& flags) {
   const uint32_t rep = s / P.total_tiles, lt = s - rep * P.total_tiles;
-  const SpeciesRec& sp = P.species.rec[rep * P.species.stride + tile_species(tw)];
-  if (!(sp.flags & SPF_SURFACE) || !(sp.space_step > 0)) {
-    P.done[s] = P.stamp_base | kDoneFinal;
-    return;
-  }
-  const double toff = P.ttoff[s];
-  if (!list && !ready_this_iteration(P.iteration, toff)) {
-    P.ttoff[s] = toff_past_iteration(P.iteration, toff);
-    P.done[s] = P.stamp_base | kDoneFinal;
-    return;
-  }
-  const SurfTiming tm = surf_timing(P, sp, tw, toff, s);
-  const uint32_t id = P.tile_id[s];
-  const bool delayed = surf_delayed(P, tw, toff);
-  const unsigned long long key = surf_key(delayed, id);
+  const SurfTiming tm = surf_timing(P, surf_species(P, rep, tw), tw, toff, P.birth[s]);
   PhiloxStream rng;
-  rng.init(P.seed, id, P.iteration, rep, P.pass);
+  rng.init(P.seed, (uint32_t)key, P.iteration, rep, P.pass);
   const uint32_t wi = P.tile_wall[lt];
   const uint32_t t0 = lt - P.grids[wi].tile_base;
   const double u = P.tu[s], v = P.tv[s];
-  uint32_t err = 0;
+  uint32_t err = 0, end = s;
+  double eu = u, ev = v;  // no position found: the molecule stays where it is for this step
   for (int attempt = 0; attempt <= kSurfRetries; ++attempt) {
     double du, dv;
     surf_displacement(rng, tm.space_factor, du, dv);
@@ -153,81 +194,107 @@ __global__ __launch_bounds__(256) void k_surf_move(SurfPhase P, const uint32_t* 
       err |= ERR_GRID;
       break;
     }
-    if (nw == wi && nt == t0) {  // the same tile: the molecule moves within it
-      P.tu[s] = nu;
-      P.tv[s] = nv;
-      surf_step_over(P, s, tw, toff, tm, delayed);
-      if (err) atomicOr(P.err, err);
-      return;
-    }
+    const bool own = nw == wi && nt == t0;  // the same tile: the molecule moves within it
     const uint32_t ts = rep * P.total_tiles + g.tile_base + nt;
-    const uint32_t occ = P.tiles[ts];
-    if (occ != kTileEmpty) {
-      // an occupant ahead in the order that still steps in this pass: wait
-      // for it (in the first pass: one not yet stamped in this iteration;
-      // later: one listed for this pass and not yet done)
-      const SpeciesRec& os = P.species.rec[rep * P.species.stride + tile_species(occ)];
-      const uint32_t d = P.done[ts];
-      const bool pending = P.pass == 0 ? (d & ~15u) != P.stamp_base : d == (P.stamp_base | P.pass);
-      if (pending && (os.flags & SPF_SURFACE) && os.space_step > 0 &&
-          surf_key(surf_delayed(P, occ, P.ttoff[ts]), P.tile_id[ts]) < key) {
-        lose_list[atomicAdd(lose_count, 1u)] = s;
-        if (err) atomicOr(P.err, err);
-        return;
-      }
-      continue;  // taken: draw again
-    }
-    P.prop[s] = ts;
-    P.pu[s] = nu;
-    P.pv[s] = nv;
-    atomicMin(P.claim + ts, key);
-    P.plist[atomicAdd(P.hdr + kHdrSurfProps, 1u)] = s;
-    if (err) atomicOr(P.err, err);
-    return;
+    if (!own && tile_taken(P, s, rep, ts, key, flags)) continue;
+    end = own ? s : ts;
+    eu = nu;
+    ev = nv;
+    break;
   }
-  // no position found: the molecule stays where it was for this step
-  surf_step_over(P, s, tw, toff, tm, delayed);
-  if (err) atomicOr(P.err, err);
+  P.pu[s] = eu;
+  P.pv[s] = ev;
+  flags |= err << kSurfErrShift;
+  return end;
 }
 
-// Claims settled: the first in the order moves to the tile it proposed (the tile
-// it leaves was taken when the round's proposals were made, so no other
-// mover enters it in this round) and ends its step there; the others are
-// listed for the next round.
-__global__ __launch_bounds__(256) void k_surf_commit(SurfPhase P, uint32_t* __restrict__ lose_list,
-                                                     uint32_t* __restrict__ lose_count, uint32_t max_props) {
-  const uint32_t n = P.hdr[kHdrSurfProps];
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n && i < max_props; i += gridDim.x * blockDim.x) {
-    const uint32_t s = P.plist[i];
-    const uint32_t ts = P.prop[s];
-    const uint32_t id = P.tile_id[s];
+// A round (n_all > 0: the first pass's first, over every slot).  Bound by the
+// latency of one step (draws, edge crossings); later rounds of a pass work
+// out a few steps only.
+__global__ __launch_bounds__(256) void k_surf_round(SurfPhase P, uint32_t n_all) {
+  const uint32_t n = n_all ? n_all : *P.count;
+  for (uint64_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t s = n_all ? (uint32_t)i : P.list[i];
+    const uint32_t tw = P.tiles[s];
+    if (n_all) {
+      if (tw == kTileEmpty || !surf_moves(surf_species(P, s / P.total_tiles, tw))) continue;
+      P.list[atomicAdd(P.hdr + kHdrSurfMovers, 1u)] = s;
+    }
+    const uint32_t before = P.round ? P.dest_prev[s] : s;
+    const double toff = P.ttoff[s];
+    if (n_all ? !ready_this_iteration(P.iteration, toff) : before == kSurfNotDue) {
+      P.dest[s] = kSurfNotDue;
+      continue;
+    }
+    const unsigned long long key = surf_key(surf_delayed(P, tw, toff), P.tile_id[s]);
+    uint32_t end = before;
+    const uint32_t met = P.round ? P.flags[s] : kSurfAhead;
+    if ((met & kSurfAhead) || ((met & kSurfOneAhead) && !still_taken(P, P.moved_id[s], key)) ||
+        (before != s && claimed_ahead(P, before, key))) {
+      uint32_t flags = 0;
+      end = surf_step(P, s, tw, toff, key, flags);
+      P.flags[s] = flags;
+      if (P.check && end != before) atomicAdd(P.hdr + kHdrSurfChanged, 1u);
+    }
+    P.dest[s] = end;
+    if (end != s) atomicMin(P.claim + end, ((unsigned long long)P.code << 33) | key);
+  }
+}
+
+// The movers leave: steps within a tile are booked where they are, the others
+// take their molecule off its tile (offset and birthday wait in the slot's
+// claim words, which this pass is done with).
+__global__ __launch_bounds__(256) void k_surf_leave(SurfPhase P) {
+  if (P.hdr[kHdrSurfChanged]) return;
+  const uint32_t n = *P.count;
+  for (uint64_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t s = P.list[i], end = P.dest[s];
     const uint32_t tw = P.tiles[s];
     const double toff = P.ttoff[s];
-    const bool delayed = surf_delayed(P, tw, toff);
-    if (P.claim[ts] == surf_key(delayed, id)) {
-      const uint32_t rep = s / P.total_tiles;
-      const SpeciesRec& sp = P.species.rec[rep * P.species.stride + tile_species(tw)];
-      // the step's timing again, from the slot it leaves
-      const SurfTiming tm = surf_timing(P, sp, tw, toff, s);
-      P.tiles[ts] = tw;
-      P.tile_id[ts] = id;
-      P.tu[ts] = P.pu[s];
-      P.tv[ts] = P.pv[s];
-      P.birth[ts] = P.birth[s];
-      P.tile_consumed[ts] = 0;  // the molecule reacts with the volume movers of later iterations
-      surf_step_over(P, ts, tw, toff, tm, delayed);
-      P.tiles[s] = kTileEmpty;
-      P.tile_id[s] = kInvalid;
-    } else {
-      lose_list[atomicAdd(lose_count, 1u)] = s;
+    if (end == kSurfNotDue) {
+      P.ttoff[s] = toff_past_iteration(P.iteration, toff);
+      P.done[s] = P.stamp_base | kDoneFinal;
+      continue;
     }
+    const uint32_t err = P.flags[s] >> kSurfErrShift;
+    if (err) atomicOr(P.err, err);
+    const double birth = P.birth[s];
+    if (end == s) {
+      P.tu[s] = P.pu[s];
+      P.tv[s] = P.pv[s];
+      surf_step_over(P, s, tw, toff, surf_timing(P, surf_species(P, s / P.total_tiles, tw), tw, toff, birth),
+                     surf_delayed(P, tw, toff));
+      continue;
+    }
+    P.flags[s] = tw;
+    P.moved_id[s] = P.tile_id[s];
+    P.claim[s] = (unsigned long long)__double_as_longlong(toff);
+    P.claim_prev[s] = (unsigned long long)__double_as_longlong(birth);
+    P.tiles[s] = kTileEmpty;
+    P.tile_id[s] = kInvalid;
   }
 }
 
-__global__ __launch_bounds__(256) void k_surf_unclaim(SurfPhase P, uint32_t max_props) {
-  const uint32_t n = P.hdr[kHdrSurfProps];
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n && i < max_props; i += gridDim.x * blockDim.x)
-    P.claim[P.prop[P.plist[i]]] = ~0ull;
+// The movers that left arrive and end their step there.
+__global__ __launch_bounds__(256) void k_surf_arrive(SurfPhase P) {
+  if (P.hdr[kHdrSurfChanged]) return;
+  const uint32_t n = *P.count;
+  for (uint64_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t s = P.list[i], ts = P.dest[s];
+    if (ts == kSurfNotDue || ts == s) continue;
+    const uint32_t tw = P.flags[s];
+    const double toff = __longlong_as_double((long long)P.claim[s]);
+    const double birth = __longlong_as_double((long long)P.claim_prev[s]);
+    P.claim[s] = P.claim_prev[s] = ~0ull;
+    P.tiles[ts] = tw;
+    P.tile_id[ts] = P.moved_id[s];
+    P.tu[ts] = P.pu[s];
+    P.tv[ts] = P.pv[s];
+    P.birth[ts] = birth;
+    P.tile_consumed[ts] = 0;  // the molecule reacts with the volume movers of later iterations
+    surf_step_over(P, ts, tw, toff, surf_timing(P, surf_species(P, s / P.total_tiles, tw), tw, toff, birth),
+                   surf_delayed(P, tw, toff));
+  }
 }
 
 __global__ void k_fill_ones(uint32_t* p, uint32_t n) {
@@ -257,15 +324,17 @@ hipError_t launch_fill_claims(hipStream_t s, unsigned long long* claim, uint32_t
   return hipGetLastError();
 }
 
-hipError_t surf_round(hipStream_t s, const SurfPhase& P, const uint32_t* list, const uint32_t* count,
-                      uint32_t max_movers, uint32_t* lose_list, uint32_t* lose_count) {
-  if (max_movers == 0) return hipSuccess;
-  const uint32_t n_all = P.total_tiles * P.num_replicas;
-  hipLaunchKernelGGL(k_surf_move, blocks_for(max_movers), dim3(256), 0, s, P, list, count, n_all, lose_list,
-                     lose_count);
-  const dim3 grid = dim3(std::min<uint32_t>(blocks_for(max_movers).x, 2048u));
-  hipLaunchKernelGGL(k_surf_commit, grid, dim3(256), 0, s, P, lose_list, lose_count, max_movers);
-  hipLaunchKernelGGL(k_surf_unclaim, grid, dim3(256), 0, s, P, max_movers);
+// (grid-stride: any grid is right)
+static inline dim3 movers_grid(uint32_t n) { return dim3(std::min<uint32_t>(blocks_for(n).x, 2048u)); }
+
+hipError_t surf_round(hipStream_t s, const SurfPhase& P, uint32_t n_all, uint32_t max_movers) {
+  hipLaunchKernelGGL(k_surf_round, n_all ? blocks_for(n_all) : movers_grid(max_movers), dim3(256), 0, s, P, n_all);
+  return hipGetLastError();
+}
+
+hipError_t surf_commit(hipStream_t s, const SurfPhase& P, uint32_t max_movers) {
+  hipLaunchKernelGGL(k_surf_leave, movers_grid(max_movers), dim3(256), 0, s, P);
+  hipLaunchKernelGGL(k_surf_arrive, movers_grid(max_movers), dim3(256), 0, s, P);
   return hipGetLastError();
 }
 

@@ -177,6 +177,55 @@ def test_dense_tiles_stay_consistent(gpu_available, oracle_lib):
     eng.close()
 
 
+@pytest.mark.parametrize("n,subdivisions,steps", [(16000, 4, None), (24000, 4, [0.5]), (30000, 4, [1.0 / 3.0]),
+                                                  (300, 1, [0.5])])
+def test_contended_tiles_match_oracle(gpu_available, oracle_lib, n, subdivisions, steps):
+    """Half and nearly all of the sphere's tiles occupied, so that molecules
+    wait for tiles others leave or take in the same pass: walls, tiles and
+    positions equal the oracle's, which moves one molecule at a time."""
+    from oracle import pyoracle as po
+    wl = W.surface_diffusion(n_s=n, iterations=12, d_surf=5e-7, sphere_subdivisions=subdivisions)
+    if steps:
+        wl = W.with_time_steps(wl, steps)
+    eng = DiffuseReactEngine.from_workload(wl, seed=37)
+    w = po.world_from_workload(wl, draw_mode=po.DRAW_PHILOX, seed=37)
+    w.set_barrier_interval(wl.barrier_interval)
+    for chunk in range(0, wl.iterations, 4):
+        eng.step(chunk, 4)
+        w.run(4)
+        _compare_surface(eng, w, "iteration %d" % (chunk + 4))
+        print("iteration %d: %s" % (chunk + 4, w.surface_stats()), flush=True)
+    assert w.surface_stats()["retries"] > 0
+    w.close()
+    eng.close()
+
+
+def test_contended_receptors_that_bind_match_oracle(gpu_available, oracle_lib):
+    """20,000 diffusing receptors in half steps (a third of the sphere's tiles)
+    and ligands that bind them: the whole run equals the oracle's, and so does
+    a second one."""
+    from oracle import pyoracle as po
+    seed = 59
+    wl = W.receptor_sphere(n_l=20000, n_r=20000, iterations=20, rate=1e8, down_fraction=0.0)
+    wl = W.with_time_steps(W.with_diffusing_surface(wl, {1: 1e-8, 2: 1e-8}), [1, 0.5, 0.5])
+    w = po.world_from_workload(wl, draw_mode=po.DRAW_PHILOX, seed=seed)
+    w.set_barrier_interval(wl.barrier_interval)
+    w.run(wl.iterations)
+    om = w.molecules()
+    live = np.nonzero(((om["flags"] & 1) == 0) & ((om["flags"] & 8) == 0))[0]
+    for _ in range(2):
+        eng = DiffuseReactEngine.from_workload(wl, seed=seed)
+        eng.step(0, wl.iterations)
+        _compare_surface(eng, w, "the end")
+        g = eng.molecules()
+        o = np.argsort(g["id"], kind="stable")
+        assert np.array_equal(g["id"][o], live)
+        assert np.abs(g["pos"][o] - om["pos"][live]).max(initial=0) <= 1e-10
+        eng.close()
+    assert w.surface_stats()["retries"] > 10000
+    w.close()
+
+
 def test_surface_round_trip_continues_exactly(gpu_available):
     wl = W.surface_diffusion(n_s=1500, iterations=30, sheet=True, n_sheet=300, d_surf=2e-7, barrier_interval=7)
     first, second = 11, 19
