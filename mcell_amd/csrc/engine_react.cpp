@@ -8,8 +8,10 @@
 #include <map>
 #include <cmath>
 #include <cstring>
+#include <thread>
 
 #include "engine.h"
+#include "poll.h"
 
 using namespace mcg;
 
@@ -139,24 +141,19 @@ ReactPipeline<PosT> make_pipeline(mcg_ctx* c, PosT* x, PosT* y, PosT* z, PosT* s
 }
 
 // Waits for the header's copy number c->rx.hdr_seq: the kernel that ends the
-// round writes it to host memory.  Polls (the wait is tens of microseconds,
-// which a stream synchronisation would add half again to), with a look at the
-// stream now and then: a copy that does not come although the stream is idle
-// or in error is an error.
+// round writes it to host memory.  Polls (a stream synchronisation would add
+// half again to the wait); a copy that does not come although the stream is
+// idle or in error is an error.
 int wait_hdr(mcg_ctx* c) {
   const uint32_t want = c->rx.hdr_seq;
   const uint32_t* const seq = c->rx.hdr_host + kHdrSeq;
-  for (;;) {
-    for (int k = 0; k < 20000; ++k) {
-      if (__atomic_load_n(seq, __ATOMIC_ACQUIRE) == want) return MCG_OK;
-      __builtin_ia32_pause();
-    }
-    const hipError_t e = hipStreamQuery(c->stream);
-    if (e == hipErrorNotReady) continue;
-    if (e != hipSuccess) return fail(MCG_E_HIP, std::string("waiting for a round: ") + hipGetErrorString(e));
-    if (__atomic_load_n(seq, __ATOMIC_ACQUIRE) == want) return MCG_OK;
-    return fail(MCG_E_HIP, "a round ended without its counters");
-  }
+  hipError_t e = hipErrorNotReady;
+  const bool there = poll_until([&] { return __atomic_load_n(seq, __ATOMIC_ACQUIRE) == want; },
+                                [] { __builtin_ia32_pause(); }, [] { std::this_thread::yield(); },
+                                [&] { return (e = hipStreamQuery(c->stream)) == hipErrorNotReady; });
+  if (there) return MCG_OK;
+  if (e != hipSuccess) return fail(MCG_E_HIP, std::string("waiting for a round: ") + hipGetErrorString(e));
+  return fail(MCG_E_HIP, "a round ended without its counters");
 }
 
 // The drain's form for the next iteration: the flag's, the decided one, or
