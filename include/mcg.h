@@ -26,6 +26,10 @@
 extern "C" {
 #endif
 
+/* Raised when a caller built for an older header would no longer work with
+ * the library (a struct, an argument or a meaning changed).  Functions added
+ * later leave it as it is: mcg_barriers_matter came within version 9, so a
+ * program that uses it checks for the symbol. */
 #define MCG_ABI_VERSION 9
 
 typedef struct mcg_ctx mcg_ctx;

@@ -169,6 +169,10 @@ def load():
         raise ImportError("libmcg.so not built: run `python -c 'import __graft_entry__ as g; g.build()'` "
                           "or `make -C mcell_amd/csrc` (%s missing)" % LIB_PATH)
     lib = ctypes.CDLL(LIB_PATH)
+    missing = [name for name in EXPORTED if not hasattr(lib, name)]
+    if missing:
+        raise ImportError("libmcg.so is older than this package (%s lacks %s): build it again"
+                          % (LIB_PATH, ", ".join(missing)))
     P = ctypes.c_void_p
     lib.mcg_last_error.restype = ctypes.c_char_p
     lib.mcg_abi_version.restype = ctypes.c_int

@@ -27,6 +27,24 @@ def test_python_binding_covers_header():
     assert sorted(_lib.EXPORTED) == declared_functions()
 
 
+def test_a_library_without_an_entry_point_is_refused(tmp_path, monkeypatch):
+    import shutil
+    import subprocess
+
+    import pytest
+    if shutil.which("gcc") is None:
+        pytest.skip("no host compiler")
+    src = tmp_path / "old.c"
+    src.write_text("".join("int %s(void) { return 0; }\n" % n for n in _lib.EXPORTED if n != "mcg_barriers_matter"))
+    old = tmp_path / "libmcg.so"
+    subprocess.check_call(["gcc", "-shared", "-fPIC", str(src), "-o", str(old)])
+    monkeypatch.setattr(_lib, "LIB_PATH", str(old))
+    monkeypatch.setattr(_lib, "_lib", None)
+    with pytest.raises(ImportError, match="lacks mcg_barriers_matter"):
+        _lib.load()
+    assert _lib._lib is None
+
+
 def test_abi_version_and_struct_sizes(tmp_path):
     import shutil
     import subprocess
