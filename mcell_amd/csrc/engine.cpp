@@ -419,8 +419,9 @@ int free_step(mcg_ctx* c, uint32_t first_iteration, uint32_t num_iterations, mcg
   const uint64_t most = std::min<uint64_t>(4096, (1ull << 28) / std::max(n, 1u));
   const uint32_t per_launch = run ? (uint32_t)std::max<uint64_t>(1, most) : 1u;
   uint32_t launches = 0;
-  for (uint32_t k = 0; k < num_iterations; k += per_launch, launches += run ? 1 : 3) {
-    const uint32_t first = first_iteration + k, num = std::min(per_launch, num_iterations - k);
+  for (uint64_t k = 0; n && k < num_iterations; k += per_launch, launches += run ? 1 : 3) {
+    const uint32_t first = first_iteration + (uint32_t)k;
+    const uint32_t num = (uint32_t)std::min<uint64_t>(per_launch, num_iterations - k);
     if (run) {
       if (k) HIP_TRY(launch_fill_u64(c->stream, c->counters.p + CTR_LAST_TRACED, 0ull, 1));
       if (c->fp32())

@@ -5,6 +5,7 @@ of the rule that chooses between the two."""
 import numpy as np
 import pytest
 
+from mcell_amd import _lib
 from mcell_amd import workloads as W
 from mcell_amd.engine import DiffuseReactEngine
 
@@ -45,3 +46,15 @@ def test_run_with_surface_classes(gpu_available, action):
         assert np.array_equal(got[0][0][k], got[1][0][k]), k
     assert got[0][1:] == got[1][1:]
     assert got[0][2] > 0 if action == 1 else got[0][3] < wl.num_molecules
+
+
+def test_no_molecules_and_the_longest_call(gpu_available):
+    """Nothing to move: a call of 2^32 - 1 iterations launches nothing, ends
+    and moves the clock on; the next call is refused as for any other clock."""
+    wl = W.free_diffusion_box(scale=0.01)
+    eng = DiffuseReactEngine.from_workload(wl, add_molecules=False)
+    st = eng.step_raw(0, 2 ** 32 - 1, 2.0 ** 32)
+    assert st.molecule_steps == 0 and st.kernel_launches == 0 and eng.num_molecules() == 0
+    with pytest.raises(_lib.McgError, match="clock"):
+        eng.step_raw(0, 1, 1.0)
+    eng.close()
