@@ -404,7 +404,9 @@ int react_step(mcg_ctx* c, uint32_t first_iteration, uint32_t num_iterations, do
     r.rc_volumes = std::max<uint32_t>(r.num_volumes, 1);
     const size_t n = (size_t)c->cfg.num_replicas * r.rc_volumes * r.rc_slots;
     if (r.rxn_counts.alloc(std::max<size_t>(n, 1))) return fail(MCG_E_NOMEM, "reaction counts");
-    HIP_TRY(hipMemset(r.rxn_counts.p, 0, std::max<size_t>(n, 1) * 8));
+    for (size_t k = 0; k < r.rxn_counts.n; k += 1u << 30)
+      HIP_TRY(launch_fill_u64(c->stream, r.rxn_counts.p + k, 0ull,
+                              (uint32_t)std::min<size_t>(r.rxn_counts.n - k, 1u << 30)));
   }
   r.volume_products = false;
   for (const RxnRec& x : r.rxns)
@@ -883,8 +885,10 @@ int sync_tiles_to_device(mcg_ctx* c, bool allow_alloc) {
   }
   HIP_TRY(hipMemcpy(r.tiles.p, r.tiles_host.data(), nt * 4, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(r.tile_id.p, r.tile_id_host.data(), nt * 4, hipMemcpyHostToDevice));
-  HIP_TRY(hipMemset(r.tile_owner.p, 0xFF, nt * 4));
-  HIP_TRY(hipMemset(r.tile_consumed.p, 0, nt * 4));
+  // (on the engine's stream: the null stream's fills return before they are
+  // done, and nothing orders them with the step's kernels)
+  HIP_TRY(launch_fill_u32(c->stream, r.tile_owner.p, kInvalid, (uint32_t)nt));
+  HIP_TRY(launch_fill_u32(c->stream, r.tile_consumed.p, 0u, (uint32_t)nt));
   if (r.surf_on) {
     if (r.tu.n != nt) {
       if (!allow_alloc) return fail(MCG_E_STATE, "surface molecules on new walls need tile buffers");

@@ -1337,7 +1337,7 @@ __global__ __launch_bounds__(256) void k_count_tiles(const uint32_t* __restrict_
 }
 
 // --------------------------------------------------------------- launchers --
-static inline dim3 blocks_for(uint32_t n) { return dim3((n + 255) / 256 > 0 ? (n + 255) / 256 : 1); }
+static inline dim3 blocks_for(uint32_t n) { return dim3(std::max(1u, n / 256 + (n % 256 != 0))); }
 // The full-step kernels walk their list grid-stride: at most two workgroups
 // per CU fit (their LDS), and every workgroup launched beyond the list's
 // actual length (a device count under a host bound) still costs a workgroup

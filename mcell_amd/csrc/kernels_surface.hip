@@ -49,7 +49,7 @@ namespace mcg {
 
 namespace {
 
-inline dim3 blocks_for(uint32_t n) { return dim3((n + 255) / 256 > 0 ? (n + 255) / 256 : 1); }
+inline dim3 blocks_for(uint32_t n) { return dim3(std::max(1u, n / 256 + (n % 256 != 0))); }
 
 __global__ void k_fill_claims(unsigned long long* claim, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
