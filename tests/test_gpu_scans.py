@@ -63,9 +63,10 @@ def test_many_species(gpu_available, precision):
         assert np.array_equal(got[0][1][k], got[1][1][k]), k
 
 
-@pytest.mark.parametrize("n_a,n_b", [(1, 0), (1, 1), (1024, 1024), (1025, 1024), (65536, 65536), (65537, 65536)])
+@pytest.mark.parametrize("n_a,n_b", [(1, 0), (1, 1), (1024, 1024), (1025, 1024), (65536, 65536), (65537, 65536),
+                                     (64512, 64512), (64513, 64512)])
 def test_waves_shares_of_the_light_pass(gpu_available, oracle_lib, n_a, n_b):
-    """One molecule a wave up to 2,048, a full wave from 131,009 on: the
+    """One molecule a wave up to 2,048, a full wave from 129,025 on: the
     positions after two snapshot iterations equal the oracle's."""
     from oracle import pyoracle as po
     wl = W.bimol_box(n_a=n_a, n_b=n_b, iterations=2, seed=4)

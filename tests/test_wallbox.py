@@ -30,9 +30,9 @@ def shim(tmp_path_factory):
     subprocess.check_call([hipcc, "-O2", "-std=c++17", "-fPIC", "-shared", "--offload-arch=gfx950",
                            "-ffp-contract=off", os.path.join(HERE, "wallbox_shim.cpp"), "-o", str(out)])
     lib = ctypes.CDLL(str(out))
-    for f in (lib.box_triangles, lib.box_segments, lib.box_overlap):
+    for f in (lib.box_triangles, lib.box_segments, lib.box_overlap, lib.union_boxes):
         f.restype = None
-    for f in (lib.overlap_walk, lib.overlap_walk_light):
+    for f in (lib.overlap_walk, lib.overlap_walk_light, lib.overlap_walk_grouped):
         f.restype = ctypes.c_uint64
     return lib
 
@@ -72,6 +72,49 @@ def test_grouped_walk_visits_the_overlapping_entries_in_order(shim):
             out = np.zeros(max(n, 1), np.uint32)
             cnt = walk(_p(box), ctypes.c_uint32(k0), ctypes.c_uint32(n), ctypes.c_uint32(int(sb)), _p(out))
             assert list(out[:cnt]) == keep, (trial, n, k0, walk)
+
+
+def _random_boxes(rng, n, width):
+    lo = rng.integers(0, 16, size=(n, 3))
+    hi = np.minimum(lo + rng.integers(0, width, size=(n, 3)), 15)
+    return lo, hi, sum((lo[:, a] | (hi[:, a] << 4)) << (8 * a) for a in range(3)).astype(np.uint32)
+
+
+def test_union_of_boxes(shim):
+    rng = np.random.default_rng(21)
+    n = 100000
+    (la, ha, a), (lb, hb, b) = _random_boxes(rng, n, 16), _random_boxes(rng, n, 16)
+    lo, hi = np.minimum(la, lb), np.maximum(ha, hb)
+    expect = sum((lo[:, x] | (hi[:, x] << 4)) << (8 * x) for x in range(3)).astype(np.uint32)
+    out = np.zeros(n, np.uint32)
+    shim.union_boxes(ctypes.c_uint64(n), _p(a), _p(b), _p(out))
+    assert np.array_equal(out, expect)
+
+
+def test_walk_through_groups_of_eight(shim):
+    """Lists that start and end anywhere between two groups' edges (groups that
+    lie only partly in the list are read entry by entry), with boxes small
+    enough for whole groups to be passed over: the entries of a plain scan, in
+    order."""
+    rng = np.random.default_rng(22)
+    n = 96
+    out = np.zeros(n, np.uint32)
+    visited = 0
+    for k0 in range(0, 25):
+        for length in list(range(0, 42)) + [n - k0]:
+            k1 = min(k0 + length, n)
+            lo, hi, box = _random_boxes(rng, n, 3)
+            # neighbours in the list lie next to each other, as a mesh's walls do
+            at = np.sort(rng.integers(0, 16, n))
+            box = ((box & np.uint32(0xFFFF00)) | at.astype(np.uint32) | (at.astype(np.uint32) << 4)).astype(np.uint32)
+            lo[:, 0] = hi[:, 0] = at
+            slo, shi, sb = _random_boxes(rng, 1, 6)
+            keep = [k for k in range(k0, k1) if np.all((lo[k] <= shi[0]) & (slo[0] <= hi[k]))]
+            m = shim.overlap_walk_grouped(_p(box), ctypes.c_uint32(n), ctypes.c_uint32(k0), ctypes.c_uint32(k1),
+                                          ctypes.c_uint32(int(sb[0])), _p(out))
+            assert out[:m].tolist() == keep, (k0, k1)
+            visited += m
+    assert visited > 0
 
 
 def _segment_triangle_distance(p, m, t):

@@ -1,5 +1,7 @@
 // Host build of the sub-cell box helpers (mcell_amd/csrc/device/wallbox.h)
 // for tests/test_wallbox.py.
+#include <vector>
+
 #include "../mcell_amd/csrc/device/wallbox.h"
 
 using namespace mcg;
@@ -32,6 +34,25 @@ uint64_t overlap_walk_light(const uint32_t* box, uint32_t k0, uint32_t k1, uint3
        k = next_overlap<kLightOverlapGroup>(box, k + 1, k1, sb))
     out[n++] = k;
   return n;
+}
+
+// The walk through the boxes of groups of eight entries, made for a list
+// [0, n) as the host makes them.
+uint64_t overlap_walk_grouped(const uint32_t* box, uint32_t n, uint32_t k0, uint32_t k1, uint32_t sb, uint32_t* out) {
+  std::vector<uint32_t> group(n / kBoxGroup + 1, 0u);
+  for (uint32_t g = 0; (g + 1) * kBoxGroup <= n; ++g) {
+    group[g] = box[g * kBoxGroup];
+    for (uint32_t u = 1; u < kBoxGroup; ++u) group[g] = box_union(group[g], box[g * kBoxGroup + u]);
+  }
+  uint64_t m = 0;
+  for (uint32_t k = next_overlap_grouped(box, group.data(), k0, k1, sb); k < k1;
+       k = next_overlap_grouped(box, group.data(), k + 1, k1, sb))
+    out[m++] = k;
+  return m;
+}
+
+void union_boxes(uint64_t n, const uint32_t* a, const uint32_t* b, uint32_t* out) {
+  for (uint64_t i = 0; i < n; ++i) out[i] = box_union(a[i], b[i]);
 }
 
 // out[i] = region_box of the triangle tri[9i..9i+8] in subpartition s[i]
