@@ -20,7 +20,6 @@ enum : uint32_t {
   kHdrErr = 9,            // error bits (ERR_*) of the call's kernels
   kHdrExd = 10,           // movers the full step deferred to its exact_disk pass
   kHdrContinue = 11,      // movers of the phase that diffuse again in this iteration
-  kHdrSurfChanged = 12,   // surface phase: movers whose end the round changed
   kHdrSurfMovers = 13,    // surface phase: the first pass's movers
   kHdrSurfCont0 = 15,     // surface phase: molecules that step again in this iteration (two lists)
   kHdrSurfCont1 = 16,
@@ -30,11 +29,13 @@ enum : uint32_t {
   kHdrMoveStart = 22,     // (64 bits) device clock at the start of the iteration's first move
   kHdrMoveTicks = 24,     // (64 bits) device clock ticks the call's first moves took
   kHdrLogBase = 26,       // (64 bits) products: reactions of the call before the phase
-  kHdrWords = 28,
+  kHdrSurfChanged = 28,   // surface phase: ends changed by each round of a batch (kSurfBatch words)
+  kHdrWords = 36,
 };
+constexpr uint32_t kSurfBatch = 8;
 // The host's copy of the counters, written by the kernels that end a round:
 // the words, then the number of the copy.
-constexpr uint32_t kHdrSeq = 32;
+constexpr uint32_t kHdrSeq = 40;
 constexpr uint32_t kHdrHostWords = 64;
 
 // A 64-bit counter of the header (its word is even, the header 8-byte aligned).

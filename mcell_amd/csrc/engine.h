@@ -140,11 +140,16 @@ struct ReactState {
   // while surface species diffuse), and the surface phase's buffers
   std::vector<double> tu_host, tv_host, ttoff_host, tbirth_host;
   bool surf_on = false;  // some surface species diffuses: grids on every wall, the surface phase runs
-  DevBuf<double> tu, tv, ttoff, tbirth, spu, spv;
+  DevBuf<double> tu, tv, ttoff, tbirth, spu, spv, stries_uv;
   DevBuf<unsigned long long> sclaim0, sclaim1;
-  DevBuf<uint32_t> sdest0, sdest1, sflags, smoved, smovers, sdone, scont0, scont1;
+  DevBuf<uint32_t> sdest0, sdest1, stries, sflags, smoved, smovers, sdone, scont0, scont1;
   uint32_t surf_code = 0;                   // the claims' code of the last round; 0: the claims are to be cleared
-  uint32_t surf_movers = RoundSizes::kUnknown;  // the last iteration's (launch sizes only)
+  // occupied tiles when they were last uploaded (no reaction adds one: a
+  // surface product takes its reactant's tile): room for the movers' attempts
+  size_t surf_mols = 0;
+  // launch sizes only: the last iteration's movers and, per pass, rounds
+  uint32_t surf_movers = RoundSizes::kUnknown;
+  uint32_t surf_rounds[kSurfPasses] = {};
   DevBuf<WallEdgeRec> edges_d;
   // reaction log of the last mcg_step call
   DevBuf<RxnEvent> log;

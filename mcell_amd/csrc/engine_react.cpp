@@ -396,6 +396,9 @@ int react_step(mcg_ctx* c, uint32_t first_iteration, uint32_t num_iterations, do
   }
   if (int st = ensure_surface_diffusion(c)) return st;
   if (int st = sync_tiles_to_device(c)) return st;
+  if (r.surf_on && r.stries.n < kSurfTries * r.surf_mols)
+    if (r.stries.alloc(kSurfTries * r.surf_mols) || r.stries_uv.alloc(2 * kSurfTries * r.surf_mols))
+      return fail(MCG_E_NOMEM, "surface phase buffers");
   if (!r.rxn_counts.p) {
     // the classes are fixed from the first step on
     r.rc_unimol = (uint32_t)r.rxns.size() * 4;
@@ -899,6 +902,7 @@ int sync_tiles_to_device(mcg_ctx* c, bool allow_alloc) {
         return fail(MCG_E_NOMEM, "surface phase buffers");
       r.surf_code = 0;
     }
+    r.surf_mols = nt - std::count(r.tiles_host.begin(), r.tiles_host.end(), kTileEmpty);
     if (r.sdone.n == nt) {
       // molecules keep their slots' stamps only within an iteration
       HIP_TRY(launch_fill_done(c->stream, r.sdone.p, (uint32_t)nt));
@@ -1051,6 +1055,9 @@ int surface_phase(mcg_ctx* c, uint32_t iteration, double barrier, uint32_t* err)
   P.birth = r.tbirth.p;
   P.pu = r.spu.p;
   P.pv = r.spv.p;
+  P.tries = r.stries.p;
+  P.tries_uv = r.stries_uv.p;
+  P.max_tries = (uint32_t)(r.stries.n / kSurfTries);
   P.flags = r.sflags.p;
   P.moved_id = r.smoved.p;
   P.done = r.sdone.p;
@@ -1078,20 +1085,20 @@ int surface_phase(mcg_ctx* c, uint32_t iteration, double barrier, uint32_t* err)
     P.pass = pass;
     P.clist = conts[pass & 1];
     P.ccount = r.hdr.p + cwords[pass & 1];
-    HIP_TRY(launch_clear_words(c->stream, r.hdr.p, kHdrSurfChanged, pass ? kHdrSurfChanged : kHdrSurfMovers,
-                               cwords[pass & 1]));
+    HIP_TRY(launch_clear_words(c->stream, r.hdr.p, pass ? cwords[pass & 1] : kHdrSurfMovers, cwords[pass & 1]));
     if (r.surf_code <= kSurfMaxRounds) {
       for (unsigned long long* p : claims) HIP_TRY(launch_fill_claims(c->stream, p, n_all));
       r.surf_code = kSurfFirstCode + 1;
     }
     for (uint32_t round = 0;;) {
-      // a batch of rounds, and the moves if its last changed nothing: three
-      // at first (2,000 molecules on 46,080 tiles: the second round changes
-      // some end in four passes of five, the third in few), then two
-      const uint32_t last = round + (round ? 1 : 2);
-      for (; round <= last; ++round) {
+      // a batch of rounds, and the moves if its last changed nothing: as many
+      // as the pass took in the last iteration (2,000 molecules on 46,080
+      // tiles take about three, 20,000 four), then two at a time
+      const uint32_t first = round;
+      const uint32_t batch = first ? 2u : std::min(std::max(r.surf_rounds[pass], 2u), kSurfBatch);
+      for (uint32_t k = 0; k < batch; ++k, ++round) {
         P.round = round;
-        P.check = round == last;
+        P.slot = k;
         P.code_prev = round ? r.surf_code : 0u;
         P.code = --r.surf_code;
         P.claim = claims[round & 1];
@@ -1101,10 +1108,15 @@ int surface_phase(mcg_ctx* c, uint32_t iteration, double barrier, uint32_t* err)
         HIP_TRY(surf_round(c->stream, P, pass == 0 && round == 0 ? n_all : 0u, movers));
       }
       HIP_TRY(surf_commit(c->stream, P, movers));
-      // (the copy clears the count of changes)
+      // (the copy clears the counts of changes)
       HIP_TRY(launch_publish(c->stream, r.hdr.p, r.hdr_host_d, ++r.hdr_seq, false, kHdrWords));
       if (int st = wait_hdr(c)) return st;
-      if (h[kHdrSurfChanged] == 0) break;
+      if (h[kHdrSurfChanged + batch - 1] == 0) {
+        uint32_t k = 0;
+        while (k + 1 < batch && (h[kHdrSurfChanged + k] != 0 || first + k == 0)) ++k;
+        r.surf_rounds[pass] = first + k + 1;
+        break;
+      }
       if (round >= kSurfMaxRounds) return fail(MCG_E_LIMIT, "surface moves did not settle");
     }
     if (pass == 0) r.surf_movers = h[kHdrSurfMovers];

@@ -177,7 +177,7 @@ __device__ __forceinline__ void publish_header(uint32_t* hdr, uint32_t* host, ui
     // the round's counters, for the next move
     hdr[kHdrProposals] = 0;
     hdr[kHdrExd] = 0;
-    hdr[kHdrSurfChanged] = 0;
+    for (uint32_t k = 0; k < kSurfBatch; ++k) hdr[kHdrSurfChanged + k] = 0;
     if (clear < kHdrWords) hdr[clear] = 0;
   }
 }

@@ -21,11 +21,10 @@
 // molecules ahead were, so a round that changes no end has found the
 // sequential order's.  Only then do the movers move (two launches: all
 // leave their tiles, then all arrive), so that within a round nothing is
-// written that another molecule's step reads.  Most steps meet no molecule
-// ahead and are worked out once, unless the tile they end on gets a claim
-// from ahead; a step that was turned away by one occupant ahead is worked out
-// again when that occupant's end leaves the tile free, and any other step
-// that met molecules ahead in every round (kSurfOneAhead, kSurfAhead).
+// written that another molecule's step reads.  The tiles a step's attempts
+// fall on do not depend on the others: they are kept, so that a later round
+// only asks which of them is the first that is free, and works attempts out
+// only where it needs one more than the rounds before.
 //
 // Claims: per slot the smallest order key among the movers that end there in
 // a round, by atomicMin of code << 33 | key.  The code falls from round to
@@ -125,9 +124,6 @@ __device__ __forceinline__ void surf_step_over(const SurfPhase& P, uint32_t s, u
   }
 }
 
-// what a step met of the molecules ahead in the order (error bits follow):
-// the occupant of moved_id[s]'s tile alone, which stays there, or more
-constexpr uint32_t kSurfAhead = 1u, kSurfOneAhead = 2u, kSurfErrShift = 2u;
 constexpr unsigned long long kClaimKey = (1ull << 33) - 1;
 
 __device__ __forceinline__ bool surf_moves(const SpeciesRec& sp) {
@@ -144,35 +140,37 @@ __device__ __forceinline__ bool claimed_ahead(const SurfPhase& P, uint32_t ts, u
   return (uint32_t)(c >> 33) == P.code_prev && (c & kClaimKey) < key;
 }
 
-// Whether the tile of slot ts, whose occupant steps ahead of `key`, is taken.
-__device__ __forceinline__ bool still_taken(const SurfPhase& P, uint32_t ts, unsigned long long key) {
-  return P.round == 0 || P.dest_prev[ts] == ts || claimed_ahead(P, ts, key);
-}
-
-// Whether the tile of slot ts is taken at the turn of the molecule in slot s
-// with order key `key`, as far as the round before knows.
-__device__ __forceinline__ bool tile_taken(const SurfPhase& P, uint32_t s, uint32_t rep, uint32_t ts,
-                                           unsigned long long key, uint32_t& flags) {
+// Whether the tile of slot ts is taken at the turn of the molecule with order
+// key `key`, as far as the round before knows.
+__device__ __forceinline__ bool tile_taken(const SurfPhase& P, uint32_t rep, uint32_t ts, unsigned long long key) {
   const uint32_t occ = P.tiles[ts];
   if (occ != kTileEmpty) {
     if (!surf_moves(surf_species(P, rep, occ))) return true;
     const double toff = P.ttoff[ts];
     const bool steps = P.pass == 0 ? ready_this_iteration(P.iteration, toff) : P.done[ts] == (P.stamp_base | P.pass);
     if (!steps || surf_key(surf_delayed(P, occ, toff), P.tile_id[ts]) > key) return true;
-    const bool taken = still_taken(P, ts, key);
-    flags |= taken && !flags ? kSurfOneAhead : kSurfAhead;
-    if (flags == kSurfOneAhead) P.moved_id[s] = ts;
-    return taken;
+    if (P.round == 0 || P.dest_prev[ts] == ts) return true;
   }
-  if (!claimed_ahead(P, ts, key)) return false;
-  flags |= kSurfAhead;
-  return true;
+  return claimed_ahead(P, ts, key);
+}
+
+// The slot the molecule in slot s, the list's entry `at`, ends on, from the
+// attempts kept: kSurfUnknown if they do not say.
+__device__ __forceinline__ uint32_t kept_end(const SurfPhase& P, uint32_t at, uint32_t s, unsigned long long key) {
+  if (at >= P.max_tries) return kSurfUnknown;
+  for (uint32_t k = 0; k < kSurfTries; ++k) {
+    const uint32_t ts = P.tries[(size_t)kSurfTries * at + k];
+    if (ts == kSurfUnknown || ts == s) return ts;
+    if (ts == kSurfSpent) return s;
+    if (!tile_taken(P, s / P.total_tiles, ts, key)) return ts;
+  }
+  return s;
 }
 
 // The step of the molecule in slot s: the slot it ends on, the position there
-// in pu, pv.
-__device__ __forceinline__ uint32_t surf_step(const SurfPhase& P, uint32_t s, uint32_t tw, double toff,
-                                              unsigned long long key, uint32_t& flags) {
+// in pu, pv, and its attempts.
+__device__ __forceinline__ uint32_t surf_step(const SurfPhase& P, uint32_t at, uint32_t s, uint32_t tw, double toff,
+                                              unsigned long long key) {
   const uint32_t rep = s / P.total_tiles, lt = s - rep * P.total_tiles;
   const SurfTiming tm = surf_timing(P, surf_species(P, rep, tw), tw, toff, P.birth[s]);
   PhiloxStream rng;
@@ -180,12 +178,16 @@ __device__ __forceinline__ uint32_t surf_step(const SurfPhase& P, uint32_t s, ui
   const uint32_t wi = P.tile_wall[lt];
   const uint32_t t0 = lt - P.grids[wi].tile_base;
   const double u = P.tu[s], v = P.tv[s];
-  uint32_t err = 0, end = s;
+  const bool keep = at < P.max_tries;
+  uint32_t* const tries = P.tries + (size_t)kSurfTries * at;
+  double* const tries_uv = P.tries_uv + 2 * (size_t)kSurfTries * at;
+  uint32_t err = 0, err_from = 0, end = s, tried = 0, next = kSurfSpent;
   double eu = u, ev = v;  // no position found: the molecule stays where it is for this step
   for (int attempt = 0; attempt <= kSurfRetries; ++attempt) {
     double du, dv;
     surf_displacement(rng, tm.space_factor, du, dv);
     double nu = 0, nv = 0;
+    if (!err) err_from = tried;
     const uint32_t nw = ray_trace_surf(P.walls, P.edges, wi, u, v, du, dv, nu, nv, err);
     if (nw == kInvalid) continue;  // an ambiguous edge crossing: draw again
     const WallGrid& g = P.grids[nw];
@@ -194,31 +196,42 @@ __device__ __forceinline__ uint32_t surf_step(const SurfPhase& P, uint32_t s, ui
       err |= ERR_GRID;
       break;
     }
-    const bool own = nw == wi && nt == t0;  // the same tile: the molecule moves within it
-    const uint32_t ts = rep * P.total_tiles + g.tile_base + nt;
-    if (!own && tile_taken(P, s, rep, ts, key, flags)) continue;
-    end = own ? s : ts;
+    // the same tile: the molecule moves within it
+    const uint32_t ts = nw == wi && nt == t0 ? s : rep * P.total_tiles + g.tile_base + nt;
+    if (keep) {
+      tries[tried] = ts;
+      tries_uv[2 * tried] = nu;
+      tries_uv[2 * tried + 1] = nv;
+    }
+    ++tried;
+    if (ts != s && tile_taken(P, rep, ts, key)) continue;
+    end = ts;
     eu = nu;
     ev = nv;
+    next = kSurfUnknown;
     break;
   }
+  if (keep && tried < kSurfTries) tries[tried] = next;
   P.pu[s] = eu;
   P.pv[s] = ev;
-  flags |= err << kSurfErrShift;
+  P.flags[s] = err ? err | err_from << 16 : 0u;
   return end;
 }
 
-// A round (n_all > 0: the first pass's first, over every slot).  Bound by the
-// latency of one step (draws, edge crossings); later rounds of a pass work
-// out a few steps only.
+// A round (n_all > 0: the first pass's first, over every slot).  The first of
+// a pass is bound by the latency of a step (draws, edge crossings), the later
+// ones by that of the few steps that need another attempt, or of the loads
+// that say which tile is free.
 __global__ __launch_bounds__(256) void k_surf_round(SurfPhase P, uint32_t n_all) {
   const uint32_t n = n_all ? n_all : *P.count;
   for (uint64_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t s = n_all ? (uint32_t)i : P.list[i];
     const uint32_t tw = P.tiles[s];
+    uint32_t at = (uint32_t)i;
     if (n_all) {
       if (tw == kTileEmpty || !surf_moves(surf_species(P, s / P.total_tiles, tw))) continue;
-      P.list[atomicAdd(P.hdr + kHdrSurfMovers, 1u)] = s;
+      at = atomicAdd(P.hdr + kHdrSurfMovers, 1u);
+      P.list[at] = s;
     }
     const uint32_t before = P.round ? P.dest_prev[s] : s;
     const double toff = P.ttoff[s];
@@ -227,15 +240,9 @@ __global__ __launch_bounds__(256) void k_surf_round(SurfPhase P, uint32_t n_all)
       continue;
     }
     const unsigned long long key = surf_key(surf_delayed(P, tw, toff), P.tile_id[s]);
-    uint32_t end = before;
-    const uint32_t met = P.round ? P.flags[s] : kSurfAhead;
-    if ((met & kSurfAhead) || ((met & kSurfOneAhead) && !still_taken(P, P.moved_id[s], key)) ||
-        (before != s && claimed_ahead(P, before, key))) {
-      uint32_t flags = 0;
-      end = surf_step(P, s, tw, toff, key, flags);
-      P.flags[s] = flags;
-      if (P.check && end != before) atomicAdd(P.hdr + kHdrSurfChanged, 1u);
-    }
+    uint32_t end = P.round ? kept_end(P, at, s, key) : kSurfUnknown;
+    if (end == kSurfUnknown) end = surf_step(P, at, s, tw, toff, key);
+    if (end != before) atomicAdd(P.hdr + kHdrSurfChanged + P.slot, 1u);
     P.dest[s] = end;
     if (end != s) atomicMin(P.claim + end, ((unsigned long long)P.code << 33) | key);
   }
@@ -245,7 +252,7 @@ __global__ __launch_bounds__(256) void k_surf_round(SurfPhase P, uint32_t n_all)
 // take their molecule off its tile (offset and birthday wait in the slot's
 // claim words, which this pass is done with).
 __global__ __launch_bounds__(256) void k_surf_leave(SurfPhase P) {
-  if (P.hdr[kHdrSurfChanged]) return;
+  if (P.hdr[kHdrSurfChanged + P.slot]) return;
   const uint32_t n = *P.count;
   for (uint64_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t s = P.list[i], end = P.dest[s];
@@ -256,8 +263,21 @@ __global__ __launch_bounds__(256) void k_surf_leave(SurfPhase P) {
       P.done[s] = P.stamp_base | kDoneFinal;
       continue;
     }
-    const uint32_t err = P.flags[s] >> kSurfErrShift;
-    if (err) atomicOr(P.err, err);
+    // the position of the attempt it takes (none: where it is), and the
+    // errors of the attempts up to it
+    uint32_t k = kSurfTries;
+    if (i < P.max_tries) {
+      const size_t t = (size_t)kSurfTries * i;
+      for (k = 0; k < kSurfTries; ++k) {
+        const uint32_t ts = P.tries[t + k];
+        if (ts == end || ts == kSurfSpent) break;
+      }
+      const bool found = k < kSurfTries && P.tries[t + k] == end;
+      P.pu[s] = found ? P.tries_uv[2 * (t + k)] : P.tu[s];
+      P.pv[s] = found ? P.tries_uv[2 * (t + k) + 1] : P.tv[s];
+    }
+    const uint32_t f = P.flags[s];
+    if (f && k >= f >> 16) atomicOr(P.err, f & 0xFFFFu);
     const double birth = P.birth[s];
     if (end == s) {
       P.tu[s] = P.pu[s];
@@ -277,7 +297,7 @@ __global__ __launch_bounds__(256) void k_surf_leave(SurfPhase P) {
 
 // The movers that left arrive and end their step there.
 __global__ __launch_bounds__(256) void k_surf_arrive(SurfPhase P) {
-  if (P.hdr[kHdrSurfChanged]) return;
+  if (P.hdr[kHdrSurfChanged + P.slot]) return;
   const uint32_t n = *P.count;
   for (uint64_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t s = P.list[i], ts = P.dest[s];
@@ -302,8 +322,8 @@ __global__ void k_fill_ones(uint32_t* p, uint32_t n) {
   if (i < n) p[i] = ~0u;
 }
 
-__global__ void k_clear_words(uint32_t* hdr, uint32_t a, uint32_t b, uint32_t c) {
-  if (threadIdx.x == 0) hdr[a] = hdr[b] = hdr[c] = 0;
+__global__ void k_clear_words(uint32_t* hdr, uint32_t a, uint32_t b) {
+  if (threadIdx.x == 0) hdr[a] = hdr[b] = 0;
 }
 
 }  // namespace
@@ -314,8 +334,8 @@ hipError_t launch_fill_done(hipStream_t s, uint32_t* done, uint32_t n) {
   return hipGetLastError();
 }
 
-hipError_t launch_clear_words(hipStream_t s, uint32_t* hdr, uint32_t a, uint32_t b, uint32_t c) {
-  hipLaunchKernelGGL(k_clear_words, dim3(1), dim3(64), 0, s, hdr, a, b, c);
+hipError_t launch_clear_words(hipStream_t s, uint32_t* hdr, uint32_t a, uint32_t b) {
+  hipLaunchKernelGGL(k_clear_words, dim3(1), dim3(64), 0, s, hdr, a, b);
   return hipGetLastError();
 }
 
