@@ -179,12 +179,15 @@ struct mcg_ctx {
   mcg::DevBuf<uint32_t> ent_group; // boxes of groups of eight entries (long lists only)
   mcg::DevBuf<uint32_t> near_walls;  // bit per subpartition: a wall is listed in it or next to it
   bool have_geometry = false;
-  // full steps run by teams of lanes (device/team.h): worth the exchanges
-  // only where a mover's wall lists are long.  The line is a mean list of 64
-  // entries, eight lanes with eight boxes each: 1.25M molecules among spheres
-  // of 20,480 triangles (mean list 233) take 2.4 ms an iteration with teams
-  // and 3.5 without; with the 12 walls of a box teams are 10-20 % slower, and
-  // at a mean of 19 (a sphere of 5,120 triangles) the two are equal.
+  // full steps run by teams of lanes (device/team.h) and group boxes in the
+  // light pass: both cost where lists are short and pay where they are long.
+  // The line, a mean list of 64 entries, is the side on which both pay
+  // everywhere tried (200,000 molecules, single lanes and entry boxes against
+  // teams and group boxes, FP64): 706 and 433 us an iteration at a mean list
+  // of 108, 1,339 and 717 at 233, 1,058 and 556 for one fine sphere alone in
+  // a large cube.  Below it teams gain less (366 and 343 at 15, 558 and 468
+  // at 41, 586 and 434 at 58; nothing with the 12 walls of a box at 100,000
+  // molecules) and group boxes lose at 19 (170 and 191 alone).
   bool long_wall_lists = false;
   // surface classes
   std::vector<uint32_t> wall_class_host;

@@ -360,7 +360,7 @@ __global__ __launch_bounds__(256) void k_hard32(MolView32 m, SpeciesTable specie
 // unfinished lanes wait for one, and are then taken together: a full step's
 // chain costs the wave many light steps however many lanes take it, and
 // about one step in ten needs one.  Few molecules are spread over all the
-// waves the chip holds (kRunWaves; 223 registers, two waves per SIMD): a
+// waves the chip holds (kRunWaves; 224 registers, two waves per SIMD): a
 // wave's chains are then shorter and fewer.  Same steps, same order per
 // molecule: the results equal those of single iterations bit for bit.
 // Bound by the chains' latency; 10,000 molecules in a box take 11 us an
@@ -533,10 +533,13 @@ static inline uint32_t run_per_wave(uint32_t n) {
   return std::max<uint32_t>(1u, std::min<uint32_t>(64u, (n + kRunWaves - 1) / kRunWaves));
 }
 
-// Two turns of the waves the chip holds.  Above, the three passes' full
-// waves win: at 10^6 molecules 141 us an iteration against 132 in calls of
-// 64 iterations and 422 against 218 in single ones, at 3 * 10^5 53 against
-// 101 and 179 against 192.
+// Two turns of the waves the chip holds: the line up to which no call loses.
+// In a box single calls of 262,144 molecules take 155 us by k_run and 170 by
+// the passes, of 300,000 173 and 170 (FP32 177 and 169), of 500,000 240 and
+// 180.  Longer calls would still gain above it (calls of 64, us an iteration:
+// 40 and 92 at 262,144, 72 and 108 at 500,000, 135 and 134 at 1,000,000), and
+// so would fine meshes, where k_run's full steps gain most (163,852 walls, a
+// mean list of 233: 35 and 317 at 1,000 molecules, 254 and 1,520 at 262,144).
 bool run_pays(uint32_t n) { return n <= 2u * 64u * kRunWaves; }
 
 hipError_t launch_run64(hipStream_t s, const MolView64& m, uint32_t n, SpeciesTable species, const SurfaceClasses& SC,

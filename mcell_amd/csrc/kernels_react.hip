@@ -36,8 +36,9 @@
 // iteration's counters are cleared by kernels that run anyway, and the host
 // waits twice (after the first moves, after the products' moves).  40
 // launches, three copies with a synchronisation and two timing events became
-// 18 launches: A + B -> C with 4,000 molecules 268 -> 177 us an iteration,
-// 50,000 E <-> A + B 500 -> 350 us.
+// 18 launches; with full steps spread over the waves A + B -> C with 4,000
+// molecules takes 158 us an iteration (318 before both), 50,000 E <-> A + B
+// 330 us (670).
 //
 // The smallest mover id among open proposals always wins its claims, so every
 // round settles at least one proposal.  Molecules leave the snapshot order in
@@ -478,8 +479,8 @@ __global__ __launch_bounds__(256, 2) void k_move_drain(ReactParams R, Snapshot<P
 // collects, are processed here in the reference's order when no wall is near
 // the collision point: exact_disk is then exactly 1, and a failed
 // test_bimolecular draw leaves the move as it was.  Bound by instruction
-// issue: half of the vector issue slots at three or four waves per SIMD,
-// which run alike (three spill nothing in either form).  With one bit for
+// issue: 58 % of the vector issue slots (FP32, four waves per SIMD; FP64 runs
+// at three, nothing spills in either form).  With one bit for
 // moves away from all walls, the partner rows read as one list, the class
 // table in LDS and collisions kept as time, class and slot the replica batch
 // (1.1e7 molecules, FP32) takes 1.36 ms for 1.53 before.
