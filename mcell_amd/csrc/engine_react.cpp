@@ -1086,7 +1086,7 @@ int surface_phase(mcg_ctx* c, uint32_t iteration, double barrier, uint32_t* err)
     P.clist = conts[pass & 1];
     P.ccount = r.hdr.p + cwords[pass & 1];
     HIP_TRY(launch_clear_words(c->stream, r.hdr.p, pass ? cwords[pass & 1] : kHdrSurfMovers, cwords[pass & 1]));
-    if (r.surf_code <= kSurfMaxRounds) {
+    if (r.surf_code <= kSurfMaxRounds + kSurfBatch) {
       for (unsigned long long* p : claims) HIP_TRY(launch_fill_claims(c->stream, p, n_all));
       r.surf_code = kSurfFirstCode + 1;
     }
