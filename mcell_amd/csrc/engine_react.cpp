@@ -340,7 +340,9 @@ int ensure_react_buffers(mcg_ctx* c) {
                     : (r.sx.alloc(cap) || r.sy.alloc(cap) || r.sz.alloc(cap));
   if (bad) return fail(MCG_E_NOMEM, "reaction buffers");
   if (!r.hdr_host) {
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r.hdr_host), kHdrHostWords * 4, hipHostMallocDefault));
+    // coherent: the host reads what a running kernel has written
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&r.hdr_host), kHdrHostWords * 4,
+                          hipHostMallocMapped | hipHostMallocCoherent));
     std::memset(r.hdr_host, 0, kHdrHostWords * 4);
     HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void**>(&r.hdr_host_d), r.hdr_host, 0));
   }

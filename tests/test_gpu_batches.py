@@ -3,6 +3,9 @@ one workgroup and rounds of up to 2,048 proposals settled by one, larger ones
 by the sort, the scans and a grid.  Whatever the size, the reactions of an
 iteration come in (replica, mover id) order, their products take consecutive
 ids per replica, and no reactant reacts twice."""
+import os
+import threading
+
 import numpy as np
 import pytest
 
@@ -60,3 +63,36 @@ def test_statistics_of_short_and_long_calls(gpu_available):
     assert runs[0][0]["reactions"] > 0 and runs[0][0]["wall_hits"] > 0
     for k in runs[0][2]:
         assert np.array_equal(runs[0][2][k], runs[1][2][k]), k
+
+
+def test_contexts_in_threads_on_one_core(gpu_available):
+    """Six contexts, each driven by a thread of its own, all on one core: each
+    gives the run it gives alone."""
+    wl = W.bimol_box(n_a=3000, n_b=3000, seed=9, rate=1e9)
+
+    def run(seed):
+        eng = DiffuseReactEngine.from_workload(wl, seed=seed)
+        st = eng.step_raw(0, 100, 100.0)
+        m = eng.molecules()
+        eng.close()
+        o = np.argsort(m["id"])
+        return st.reactions, m["id"][o], m["pos"][o]
+
+    alone = [run(k) for k in range(6)]
+    got = [None] * 6
+    cores = os.sched_getaffinity(0)
+
+    def drive(k):
+        got[k] = run(k)
+
+    try:
+        os.sched_setaffinity(0, {min(cores)})
+        threads = [threading.Thread(target=drive, args=(k,)) for k in range(6)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        os.sched_setaffinity(0, cores)
+    for a, b in zip(alone, got):
+        assert a[0] == b[0] and np.array_equal(a[1], b[1]) and np.array_equal(a[2], b[2])
