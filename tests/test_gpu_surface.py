@@ -5,14 +5,16 @@ Surface molecules take their steps after the iteration's volume moves
 displacement traced across the walls that share edges and reflected at an
 open mesh's border (ray_trace_surf, :1578-1725), then the tile under the end
 point if it is free (else a new draw, up to eleven).  The oracle moves them
-one at a time in id order; where no two molecules contend for a tile in one
-iteration the runs are equal.
+one at a time in id order; the engine solves for the same ends, so the runs
+are equal however many molecules want one tile.
 
 * Whole runs equal the oracle's: sparse molecules on the closed icosphere
   and on the open sheet (walls and tiles exactly, uv positions to 1e-9: the
   polar method's log is the device's); ligands binding diffusing receptors
   (L + R' -> LR' on the sphere with R and LR diffusing), where the oracle's
   id order also moves every ligand before the receptors.
+* The same with tiles contended in every iteration, up to nearly all of them
+  taken.
 * At size: the sheet's 2-D mean squared displacement is 4 D t; at high
   density on the sphere every molecule keeps a tile of its own, the one
   under its position, and none is lost.
